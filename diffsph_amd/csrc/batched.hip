@@ -28,6 +28,7 @@
 
 #include "common.h"
 #include "deltasph_impl.h"
+#include "row_search.h"
 
 namespace dsph {
 
@@ -116,11 +117,6 @@ template <class T>
 inline T* at(void* ws, size_t off) {
   return reinterpret_cast<T*>(static_cast<char*>(ws) + off);
 }
-
-#ifndef DSPH_BFILL_STAGE
-#define DSPH_BFILL_STAGE 48
-#endif
-constexpr int kBFillStage = DSPH_BFILL_STAGE;
 
 __device__ __forceinline__ int bcell(float x, const Dom& d, int k, const BGrid& g) {
   // clamped in float before the conversion (NaN and out-of-range
@@ -212,124 +208,148 @@ __global__ void __launch_bounds__(kBlock) k_bgather2(int n, const int32_t* __res
   dst[p] = src[si[p]];
 }
 
-// A candidate: sorted wrapped position and the state index it maps to.
-struct BCand {
-  float2 x;
-  int idx;
-};
-
-// Row i (state order) of the fixed-width sliced ELL: entry k at
+// kTurns times kRows rows (state order) of the fixed-width sliced ELL per
+// workgroup (one set of status atomics for all of them): entry k at
 // (i/64)*64*width + 64k + i%64, candidates in the single-domain search's
-// order (cell rows dy = -1, 0, 1; cells dx = -1, 0, 1, a non-wrapping row as
-// one contiguous slice), entries mapped through si to state indices (si ==
-// NULL: the sorted order is the state order).  Rows longer than `width`
-// keep their first `width` entries and are counted in status[0]; status[1]
-// is the longest row, status[2..3] (uint64) the number of pairs found.
+// order (cell rows dy = -1, 0, 1; cells dx = -1, 0, 1), entries mapped through si to state indices (si == NULL: the sorted order
+// is the state order).  Rows longer than `width` keep their first `width`
+// entries and are counted in status[0]; status[1] is the longest row,
+// status[2..3] (uint64) the number of pairs found (count_pairs only: one
+// atomic per workgroup on one address takes ~20 ns, 0.67 ms of a launch over
+// 7.8M particles, and only dsph_batch_probe reads it).  A wave takes the rows
+// of one cell together (row_search.h); the first `depth` entries are staged in LDS and written
+// column by column, whole lines at a time, as in the single-domain fill.
+template <int kRows, int kTurns>
 __global__ void __launch_bounds__(kBlock) k_bfill(int n, const int32_t* __restrict__ dom_of,
                                                   const Dom* __restrict__ doms, const BGrid* __restrict__ grids,
                                                   const float2* __restrict__ q, const float2* __restrict__ spos,
                                                   const int32_t* __restrict__ cs, const int32_t* __restrict__ si,
-                                                  float h, int width, int32_t* __restrict__ nbr,
-                                                  int32_t* __restrict__ cnt, int32_t* __restrict__ status) {
-  __shared__ int sh_max[kBlock / 64];
-  __shared__ int sh_over[kBlock / 64];
-  __shared__ int sh_sum[kBlock / 64];
-  // the first kBFillStage entries of a row are staged in LDS as 16-bit
-  // offsets idx - i (a per-thread column) and written column by column after
-  // the scan: one contiguous line per store of the wave instead of scattered
-  // words; an offset beyond 16 bits is written at once (slot marked)
-  __shared__ int16_t stage[kBFillStage + 1][kBlock];  // + the sink row of the unconditional writes
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  int total = 0;
-  if (i < n) {
-    const int b = dom_of[i];
-    const Dom d = doms[b];
-    const BGrid g = grids[b];
-    const float2 qi = q[i];
-    const int64_t base = (int64_t)(i >> 6) * 64 * width + (i & 63);
-    const int ncx = g.nc[0], ncy = g.nc[1];
-    const int cx = bcell(qi.x, d, 0, g), cy = bcell(qi.y, d, 1, g);
-    // every candidate writes the staging slot of the next entry (the sink
-    // row past the staged ones); a kept candidate advances `total`, so its
-    // value stays
-    auto take = [&](bool kp, int idx) {
-      const int di = idx - i;
-      const bool fits = di > -32768 && di <= 32767;
-      const bool st = total < kBFillStage && total < width;
-      stage[st ? total : kBFillStage][threadIdx.x] = fits ? (int16_t)di : (int16_t)-32768;
-      if (kp && !(st && fits) && total < width) nbr[base + (int64_t)total * 64] = idx;
-      total += kp ? 1 : 0;
-    };
-    auto load = [&](int j) { return BCand{spos[j], si ? si[j] : j}; };
-    // off a periodic seam (a periodic axis of 7+ cells, no wrapped row or
-    // column) the plain difference is the min-image offset
-    const bool small = (d.periodic[0] && g.nc[0] < 7) || (d.periodic[1] && g.nc[1] < 7);
-    auto visit = [&](int jb, int je, bool seam) {
-      if (seam)
-        scan_range<4>(jb, je, load, [&](int, const BCand& c) {
-          const float dx = mod_offset(qi.x - c.x.x, d, 0);
-          const float dy = mod_offset(qi.y - c.x.y, d, 1);
-          take(within_support(dist2_exact(dx, dy), h), c.idx);
-        });
-      else
-        scan_range<4>(jb, je, load, [&](int, const BCand& c) {
-          take(within_support(dist2_exact(qi.x - c.x.x, qi.y - c.x.y), h), c.idx);
-        });
-    };
-    for (int oy = -1; oy <= 1; ++oy) {
-      int yy = cy + oy;
-      if (d.periodic[1]) {
-        yy = yy < 0 ? yy + ncy : (yy >= ncy ? yy - ncy : yy);
-      } else if (yy < 0 || yy >= ncy) {
-        continue;
+                                                  float h, int width, int depth, int32_t* __restrict__ nbr,
+                                                  int32_t* __restrict__ cnt, int32_t* __restrict__ status,
+                                                  bool count_pairs) {
+  extern __shared__ int32_t stage[];  // depth x (kRows + 1)
+  __shared__ CellRow rows[3][kRows];
+  __shared__ float2 qs[kRows];
+  __shared__ int ds[kRows], cells[kRows], found[kRows];
+  const int lane = threadIdx.x & 63;
+  const NearTest within(h);
+  int longest = 0, over_rows = 0, sum = 0;  // of this thread's rows
+  for (int turn = 0; turn < kTurns; ++turn) {
+    const int i0 = (blockIdx.x * kTurns + turn) * kRows;
+    if (i0 >= n) break;
+    if (turn > 0) __syncthreads();
+    {
+      const int r = threadIdx.x % kRows, part = threadIdx.x / kRows, i = i0 + r;
+      if (part < 3) {
+        CellRow cr{0, 0, 0, 0};
+        if (i < n) {
+          const int b = dom_of[i];
+          const Dom d = doms[b];
+          const BGrid g = grids[b];
+          const float2 qi = q[i];
+          const int ncx = g.nc[0], ncy = g.nc[1];
+          const int cx = bcell(qi.x, d, 0, g), cy = bcell(qi.y, d, 1, g);
+          if (part == 0) {
+            qs[r] = qi;
+            ds[r] = b;
+            cells[r] = g.cell_off + cy * ncx + cx;
+          }
+          int yy = cy + part - 1;
+          bool in = true;
+          if (d.periodic[1])
+            yy = yy < 0 ? yy + ncy : (yy >= ncy ? yy - ncy : yy);
+          else
+            in = yy >= 0 && yy < ncy;
+          if (in) {
+            // off a periodic seam (a periodic axis of 7+ cells, no wrapped row
+            // or column) the plain difference is the min-image offset
+            const bool small = (d.periodic[0] && ncx < 7) || (d.periodic[1] && ncy < 7);
+            const bool wraps = d.periodic[0] && (cx == 0 || cx == ncx - 1);
+            bool over = false;
+            cr = cell_row(cs + g.cell_off + (int64_t)yy * ncx, ncx, cx, d.periodic[0],
+                          small || wraps || yy != cy + part - 1, INT32_MAX >> 2, over);
+          }
+        } else if (part == 0) {
+          qs[r] = make_float2(0.f, 0.f);
+          ds[r] = 0;
+          cells[r] = -1;
+        }
+        rows[part][r] = cr;
       }
-      const int row = g.cell_off + yy * ncx;
-      const bool wraps = d.periodic[0] && (cx == 0 || cx == ncx - 1);
-      const bool seam = small || wraps || yy != cy + oy;
-      if (!wraps) {
-        const int x0 = cx - 1 < 0 ? 0 : cx - 1;
-        const int x1 = cx + 1 > ncx - 1 ? ncx - 1 : cx + 1;
-        visit(cs[row + x0], cs[row + x1 + 1], seam);
-      } else {
-        for (int ox = -1; ox <= 1; ++ox) {
-          int xx = cx + ox;
-          xx = xx < 0 ? xx + ncx : (xx >= ncx ? xx - ncx : xx);
-          visit(cs[row + xx], cs[row + xx + 1], seam);
+    }
+    __syncthreads();
+    constexpr int kMine = kRows / 4;
+    const int r0 = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * kMine;
+    const int own = r0 + (lane < kMine ? lane : 0);
+    const float2 mine = qs[own];
+    const int cell = lane < kMine ? cells[own] : -1;
+    auto d2 = [&](const float2& x, int k, bool seam) {
+      float dx = lane_value(mine.x, k) - x.x, dy = lane_value(mine.y, k) - x.y;
+      if (seam) {
+        const Dom d = doms[ds[r0 + k]];
+        dx = mod_offset(dx, d, 0);
+        dy = mod_offset(dy, d, 1);
+      }
+      return dist2_exact(dx, dy);
+    };
+    const int mine_found = scan_rows_by_cell(
+        (uint32_t)__builtin_amdgcn_ballot_w64(cell >= 0), cell, depth,
+        [&](int p, int k) { return rows[p][r0 + k]; }, [&](int j) { return spos[j]; },
+        [](int, int, bool, int j) { return j; },
+        [&](const float2& x, int k, bool seam) { return within(d2(x, k, seam)); },
+        [&](const float2& x, int k, bool seam) { return within.exact(d2(x, k, seam)); },
+        [&](int k, int pos, int j) { stage[__umul24(pos, kRows + 1) + r0 + k] = j; },
+        [&](int k, int pos, int j) {
+          const int i = i0 + r0 + k;
+          if (pos < width) nbr[(int64_t)(i >> 6) * 64 * width + (int64_t)pos * 64 + (i & 63)] = si ? si[j] : j;
+        });
+    if (cell >= 0) found[own] = mine_found;
+    __syncthreads();
+    {
+      const int r = threadIdx.x % kRows, i = i0 + r;
+      if (i < n) {
+        const int staged = found[r] < depth ? found[r] : depth;
+        const int64_t base = (int64_t)(i >> 6) * 64 * width + (i & 63);
+        constexpr int kStep = kBlock / kRows;
+        int c = threadIdx.x / kRows;
+        for (; c + 3 * kStep < staged; c += 4 * kStep) {
+          int j[4];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) j[u] = stage[(c + u * kStep) * (kRows + 1) + r];
+          if (si) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) j[u] = si[j[u]];
+          }
+#pragma unroll
+          for (int u = 0; u < 4; ++u) nbr[base + (int64_t)(c + u * kStep) * 64] = j[u];
+        }
+        for (; c < staged; c += kStep) {
+          const int j = stage[c * (kRows + 1) + r];
+          nbr[base + (int64_t)c * 64] = si ? si[j] : j;
+        }
+        if (threadIdx.x < kRows) {
+          const int m = found[r];
+          cnt[i] = m < width ? m : width;
+          longest = m > longest ? m : longest;
+          over_rows += m > width ? 1 : 0;
+          sum += m;
         }
       }
     }
-    const int staged = total < kBFillStage ? total : kBFillStage;
-    for (int t = 0; t < staged && t < width; ++t) {
-      const int16_t v = stage[t][threadIdx.x];
-      if (v != (int16_t)-32768) nbr[base + (int64_t)t * 64] = i + v;
-    }
-    cnt[i] = total < width ? total : width;
   }
-  int m = total, over = total > width ? 1 : 0, sum = total;
+  if (threadIdx.x < 64) {
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    const int t = __shfl_xor(m, o, 64);
-    m = t > m ? t : m;
-    over += __shfl_xor(over, o, 64);
-    sum += __shfl_xor(sum, o, 64);
-  }
-  if ((threadIdx.x & 63) == 0) {
-    sh_max[threadIdx.x >> 6] = m;
-    sh_over[threadIdx.x >> 6] = over;
-    sh_sum[threadIdx.x >> 6] = sum;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int bm = 0, bo = 0;
-    unsigned long long bs = 0;
-    for (int w = 0; w < (int)(blockDim.x >> 6); ++w) {
-      bm = sh_max[w] > bm ? sh_max[w] : bm;
-      bo += sh_over[w];
-      bs += (unsigned long long)sh_sum[w];
+    for (int o = 32; o > 0; o >>= 1) {
+      const int t = __shfl_xor(longest, o, 64);
+      longest = t > longest ? t : longest;
+      over_rows += __shfl_xor(over_rows, o, 64);
+      sum += __shfl_xor(sum, o, 64);
     }
-    if (bo) atomicAdd(&status[0], bo);
-    atomicMax(&status[1], bm);
-    atomicAdd(reinterpret_cast<unsigned long long*>(status + 2), bs);
+    if (lane == 0) {
+      if (over_rows) atomicAdd(&status[0], over_rows);
+      if (longest > status[1]) atomicMax(&status[1], longest);  // rarely grows
+      if (count_pairs) atomicAdd(reinterpret_cast<unsigned long long*>(status + 2), (unsigned long long)sum);
+    }
   }
 }
 
@@ -481,11 +501,19 @@ int build_grid(const Ctx& c, const float2* x, float2* wq) {
   return launch_status();
 }
 
-int fill_rows(const Ctx& c, const float2* q, const float2* spos, const int32_t* si) {
+int fill_rows(const Ctx& c, const float2* q, const float2* spos, const int32_t* si, bool count_pairs = false) {
   const Layout& L = c.L;
-  k_bfill<<<c.grid(c.n), c.block, 0, c.st>>>(c.n, c.p<int32_t>(L.dom_of), c.p<Dom>(L.doms), c.p<BGrid>(L.grids), q,
-                                             spos, c.p<int32_t>(L.cell_start), si, c.b->support, c.b->width,
-                                             c.p<int32_t>(L.nbr), c.p<int32_t>(L.cnt), c.p<int32_t>(L.status));
+  const int depth = c.b->width < kRowStage ? c.b->width : kRowStage;
+  auto launch = [&](auto kernel, int rows, int turns) {
+    kernel<<<grid_for(c.n, rows * turns), kBlock, (size_t)depth * (rows + 1) * sizeof(int32_t), c.st>>>(
+        c.n, c.p<int32_t>(L.dom_of), c.p<Dom>(L.doms), c.p<BGrid>(L.grids), q, spos, c.p<int32_t>(L.cell_start), si,
+        c.b->support, c.b->width, depth, c.p<int32_t>(L.nbr), c.p<int32_t>(L.cnt), c.p<int32_t>(L.status),
+        count_pairs);
+  };
+  if (c.n < kRowSmall)
+    launch(k_bfill<16, 1>, 16, 1);
+  else
+    launch(k_bfill<64, 4>, 64, 4);
   return launch_status();
 }
 
@@ -828,7 +856,7 @@ extern "C" int dsph_batch_probe(const dsph_batch* batch, const float* pos, int32
   s = build_grid(c, reinterpret_cast<const float2*>(pos), wq);
   if (s != DSPH_OK) return s;
   k_bgather2<<<c.grid(c.n), c.block, 0, st>>>(c.n, c.p<int32_t>(c.L.si), wq, c.p<float2>(c.L.spos));
-  s = fill_rows(c, wq, c.p<float2>(c.L.spos), c.p<int32_t>(c.L.si));
+  s = fill_rows(c, wq, c.p<float2>(c.L.spos), c.p<int32_t>(c.L.si), true);
   if (s != DSPH_OK) return s;
   int32_t h[4] = {0, 0, 0, 0};
   DSPH_CHECK_HIP(hipMemcpyAsync(h, status, sizeof(h), hipMemcpyDeviceToHost, st));

@@ -4,10 +4,11 @@
 // give a provisional slot) -> exclusive scan -> scatter -> per-cell sort by
 // original index (makes the order deterministic) -> gather positions and
 // supports into cell order.
-// Query: one thread per query particle walks the 3x3 cell block; the three
-// cells of a row are one contiguous slice of the sorted arrays unless the
-// row wraps around a periodic x boundary.
+// Query: a wave takes the queries of one cell together (row_search.h); the
+// three cells of a row are one contiguous slice of the sorted arrays unless
+// the row wraps around a periodic x boundary.
 #include "common.h"
+#include "row_search.h"
 
 namespace dsph {
 
@@ -162,85 +163,133 @@ __device__ __forceinline__ bool small_periodic_grid(const SearchArgs& a) {
   return (a.d.periodic[0] && a.g.nc[0] < 7) || (a.d.periodic[1] && a.g.nc[1] < 7);
 }
 
-// Visit the candidate slices of query i in offset order (dy=-1,0,1;
-// dx=-1,0,1): f(b, e, seam), seam true when the slice's pairs may cross a
-// periodic seam (a wrapped row or column of cells, or a small periodic grid).
-// A slice longer than three cells of DSPH_CELL_MAX is skipped and sets
-// `over`, as does a query cell of more than DSPH_CELL_MAX particles (a
-// diverged state: the work stays bounded, the caller reports it).
 constexpr int kRangeMax = 3 * DSPH_CELL_MAX;
-template <class F>
-__device__ __forceinline__ void for_candidates(const SearchArgs& a, float2 qi, bool& over, F&& f) {
+
+// The rows of cells dy = -1, 0, 1 around the query at qi, one per `part`
+// 0..2 (threads of one workgroup share a query's three rows), and the
+// query's cell.  A slice longer than three cells of DSPH_CELL_MAX is left out
+// and sets `over`, as does a query cell of more than DSPH_CELL_MAX particles
+// (a diverged state: the work stays bounded, the caller reports it).
+__device__ __forceinline__ CellRow query_cell_row(const SearchArgs& a, float2 qi, int part, int& cell, bool& over) {
   const int ncx = a.g.nc[0], ncy = a.g.nc[1];
-  int cx = cell_coord(qi.x, a.d, 0, a.g), cy = cell_coord(qi.y, a.d, 1, a.g);
-  const bool small = small_periodic_grid(a);
-  {
-    const int c = cy * ncx + cx;
-    if (a.cs[c + 1] - a.cs[c] > DSPH_CELL_MAX) over = true;  // the query's own cell
+  const int cx = cell_coord(qi.x, a.d, 0, a.g), cy = cell_coord(qi.y, a.d, 1, a.g);
+  cell = cy * ncx + cx;
+  if (part == 1) {
+    if (a.cs[cell + 1] - a.cs[cell] > DSPH_CELL_MAX) over = true;  // the query's own cell
   }
-  for (int oy = -1; oy <= 1; ++oy) {
-    int yy = cy + oy;
-    if (a.d.periodic[1]) {
-      yy = yy < 0 ? yy + ncy : (yy >= ncy ? yy - ncy : yy);
-    } else if (yy < 0 || yy >= ncy) {
-      continue;
-    }
-    const int row = yy * ncx;
-    bool wraps = a.d.periodic[0] && (cx == 0 || cx == ncx - 1);
-    const bool seam = small || wraps || yy != cy + oy;
-    auto visit = [&](int b, int e) {
-      if (e - b > kRangeMax)
-        over = true;
-      else
-        f(b, e, seam);
+  int yy = cy + part - 1;
+  if (a.d.periodic[1])
+    yy = yy < 0 ? yy + ncy : (yy >= ncy ? yy - ncy : yy);
+  else if (yy < 0 || yy >= ncy)
+    return CellRow{0, 0, 0, 0};
+  const bool wraps = a.d.periodic[0] && (cx == 0 || cx == ncx - 1);
+  const bool seam = small_periodic_grid(a) || wraps || yy != cy + part - 1;
+  return cell_row(a.cs + (int64_t)yy * ncx, ncx, cx, a.d.periodic[0], seam, kRangeMax, over);
+}
+
+__device__ __forceinline__ float2 query_pos(const SearchArgs& a, int i) {
+  const float2 p = a.qpos[i];
+  return a.wrapped ? p : make_float2(wrap_coord(p.x, a.d, 0), wrap_coord(p.y, a.d, 1));
+}
+
+// A workgroup's kRows queries and their cell rows in LDS.
+template <int kRows>
+struct Queries {
+  CellRow rows[3][kRows];
+  float x[kRows], y[kRows], h[kRows];
+  int cell[kRows];  // -1: past the last query
+};
+
+// put(part, r, row) sees every cell row stored.
+template <int kRows, class Put>
+__device__ __forceinline__ void load_queries(const SearchArgs& a, int i0, Queries<kRows>& Q, bool& over,
+                                             const Put& put) {
+  const int r = threadIdx.x % kRows, part = threadIdx.x / kRows;
+  if (part >= 3) return;
+  const int i = i0 + r;
+  CellRow cr{0, 0, 0, 0};
+  float2 qi = make_float2(0.f, 0.f);
+  float hi = 0.f;
+  int cell = -1;
+  if (i < a.nq) {
+    qi = query_pos(a, i);
+    hi = h_of(a.qh, i, a.h0);
+    cr = query_cell_row(a, qi, part, cell, over);
+  }
+  Q.rows[part][r] = cr;
+  if (part == 0) {
+    Q.x[r] = qi.x;
+    Q.y[r] = qi.y;
+    Q.h[r] = hi;
+    Q.cell[r] = cell;
+  }
+  put(part, r, cr);
+}
+
+// The rows of this wave's quarter of the workgroup's queries: value / put /
+// spill as scan_rows_by_cell takes them, with the row's number in the
+// workgroup; done(r, n): row r has n entries (one lane per row).  The
+// min-image is evaluated only for cell rows at a periodic seam (elsewhere the
+// plain difference is the offset).  kH: supports per particle (else the
+// uniform a.h0).
+template <int kRows, bool kH, class Value, class Put, class Spill, class Done>
+__device__ __forceinline__ void scan_queries(const SearchArgs& a, const Queries<kRows>& Q, int depth,
+                                             const Value& value, const Put& put, const Spill& spill,
+                                             const Done& done) {
+  constexpr int kMine = kRows / 4;
+  const int lane = threadIdx.x & 63;
+  const int r0 = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * kMine;
+  const int own = r0 + (lane < kMine ? lane : 0);
+  const float qx = Q.x[own], qy = Q.y[own], qh = Q.h[own];
+  const int cell = lane < kMine ? Q.cell[own] : -1;
+  const uint32_t todo = (uint32_t)__builtin_amdgcn_ballot_w64(cell >= 0);
+  auto rows = [&](int p, int k) { return Q.rows[p][r0 + k]; };
+  auto val = [&](int p, int k, bool first, int j) { return value(p, r0 + k, first, j); };
+  auto in = [&](int k, int pos, int v) { put(r0 + k, pos, v); };
+  auto out = [&](int k, int pos, int v) { spill(r0 + k, pos, v); };
+  int n;
+  if (kH) {
+    auto keep = [&](const Cand& c, int k, bool seam) {
+      const float2 qi = make_float2(lane_value(qx, k), lane_value(qy, k));
+      const float hi = lane_value(qh, k);
+      return seam ? keep_pair(qi, hi, c.x, c.h, a) : keep_pair_near(qi, hi, c.x, c.h, a);
     };
-    if (!wraps) {
-      int x0 = cx - 1 < 0 ? 0 : cx - 1;
-      int x1 = cx + 1 > ncx - 1 ? ncx - 1 : cx + 1;
-      visit(a.cs[row + x0], a.cs[row + x1 + 1]);
-    } else {
-      for (int ox = -1; ox <= 1; ++ox) {
-        int xx = cx + ox;
-        xx = xx < 0 ? xx + ncx : (xx >= ncx ? xx - ncx : xx);
-        visit(a.cs[row + xx], a.cs[row + xx + 1]);
+    n = scan_rows_by_cell(
+        todo, cell, depth, rows, [&](int j) { return Cand{a.rpos[j], h_of(a.rh, j, a.h0)}; }, val,
+        [&](const Cand& c, int k, bool seam) { return LaneTest{__builtin_amdgcn_ballot_w64(keep(c, k, seam)), 0}; },
+        [](const Cand&, int, bool) { return false; }, in, out);
+  } else {
+    const NearTest within(a.h0);
+    auto d2 = [&](const float2& x, int k, bool seam) {
+      float dx = lane_value(qx, k) - x.x, dy = lane_value(qy, k) - x.y;
+      if (seam) {
+        dx = mod_offset(dx, a.d, 0);
+        dy = mod_offset(dy, a.d, 1);
       }
-    }
+      return dist2_exact(dx, dy);
+    };
+    n = scan_rows_by_cell(
+        todo, cell, depth, rows, [&](int j) { return a.rpos[j]; }, val,
+        [&](const float2& x, int k, bool seam) { return within(d2(x, k, seam)); },
+        [&](const float2& x, int k, bool seam) { return within.exact(d2(x, k, seam)); }, in, out);
   }
+  if (cell >= 0) done(own, n);
 }
 
+// Supports that differ between particles.
+static bool varied_support(const SearchArgs& a) { return a.rh || a.qh; }
+
+template <int kRows, bool kH>
 __global__ void __launch_bounds__(kBlock) k_neighbor_count(SearchArgs a, int32_t* __restrict__ counts) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= a.nq) return;
-  float2 qi = a.qpos[i];
-  if (!a.wrapped) qi = make_float2(wrap_coord(qi.x, a.d, 0), wrap_coord(qi.y, a.d, 1));
-  float hi = h_of(a.qh, i, a.h0);
-  int c = 0;
+  __shared__ Queries<kRows> Q;
+  const int i0 = blockIdx.x * kRows;
   bool over = false;  // counted without the skipped ranges; the host checks the cells
-  auto load = [&](int j) { return Cand{a.rpos[j], h_of(a.rh, j, a.h0)}; };
-  for_candidates(a, qi, over, [&](int b, int e, bool seam) {
-    if (seam)
-      scan_range<4>(b, e, load, [&](int, const Cand& r) { c += keep_pair(qi, hi, r.x, r.h, a) ? 1 : 0; });
-    else
-      scan_range<4>(b, e, load, [&](int, const Cand& r) { c += keep_pair_near(qi, hi, r.x, r.h, a) ? 1 : 0; });
-  });
-  counts[i] = c;
+  load_queries<kRows>(a, i0, Q, over, [](int, int, const CellRow&) {});
+  __syncthreads();
+  scan_queries<kRows, kH>(
+      a, Q, INT32_MAX, [](int, int, bool, int) { return 0; }, [](int, int, int) {}, [](int, int, int) {},
+      [&](int r, int n) { counts[i0 + r] = n; });
 }
-
-// Fill row i.  CSR (slice == NULL): entries at off[i] + n.  Sliced ELL:
-// entries at slice[i/64] + 64 n + i%64, the rest of the slice's columns
-// padded with -1.  Writes stay below `cap` and inside the row's own range.
-// In the sliced layout the first kFillStage entries of every row are staged
-// in LDS as 16-bit offsets j - i (a per-thread column: the staging costs 2
-// bytes per entry, so a whole typical row fits) while the candidates are
-// scanned, then written column by column, so each store of the wave is one
-// contiguous line instead of 64 scattered words.  An entry whose offset does
-// not fit in 16 bits, and every entry past kFillStage, is written as it is
-// found.
-#ifndef DSPH_FILL_STAGE
-#define DSPH_FILL_STAGE 48
-#endif
-constexpr int kFillStage = DSPH_FILL_STAGE;
-constexpr int16_t kStagedOut = -32768;  // slot already written to global memory
 
 // With `d16` the 16-bit modular delta (j - i) mod nref of every entry is
 // written beside it (rows = reference slots); a delta beyond int16 sets *ovf.
@@ -265,9 +314,9 @@ __device__ __forceinline__ void put_entry(int32_t* __restrict__ nbr, int16_t* __
 }
 
 // Tile slots written by the fill (fixed-width layout, rows = reference
-// slots): workgroup b of the fill is tile b of the list; each entry also
-// gets its neighbor's slot, j + run_d[u] for the run u holding j.  The tile
-// runs come first (they depend on the cells only).
+// slots): 256 consecutive rows are a tile of the list; each entry also gets
+// its neighbor's slot, j + run_d[u] for the run u holding j.  The tile runs
+// come first (they depend on the cells only).
 struct FillTiles {
   int32_t* runs;        // run tables, kTileRunStride ints per tile
   int32_t* n;           // particles per tile (set to -1 here when unusable)
@@ -275,146 +324,178 @@ struct FillTiles {
   int cap;
 };
 
-// Largest tile whose staged (run << 12 | slot) values stay below the
-// sentinel 0xffff.
+// Largest tile whose staged (run << 12 | slot) values stay 16 bits.
 constexpr int kFillTileMax = 4095;
-constexpr int16_t kStagedNoRun = -1;  // slot mode: entry already written to global memory
+constexpr int kNoRun = INT32_MIN;
 
-// Row i of the fill.  kSlot: staged values are (u << 12) | slot, u the run
-// of the candidate range in the tile's run table (rt_*), and the slots are
-// written beside the entries; otherwise they are j - i.
-template <bool kSlot>
-__device__ __forceinline__ int64_t fill_row(const SearchArgs& a, int i, float2 qi, float hi, int64_t base,
-                                            int64_t step, int64_t len, int64_t staged, int fixed_w,
-                                            int16_t (*stage)[kBlock], int32_t* __restrict__ nbr, int64_t cap,
-                                            int16_t* __restrict__ d16, const int32_t* __restrict__ map,
-                                            const FillTiles& T, const int* rt_s, const int* rt_e, const int* rt_d,
-                                            int R, bool& bad, bool& tbad, bool& over) {
-  constexpr int16_t kOut = kSlot ? kStagedNoRun : kStagedOut;
-  int64_t n = 0;
-  // Every candidate writes the staging slot of the next entry (row
-  // kFillStage, a sink, once the row is past the staged entries); a kept
-  // candidate then advances n, so its value stays and the next candidates
-  // write the following slot.  Only an entry past the staged ones, or whose
-  // value does not fit the staging (a delta beyond 16 bits; a range in no
-  // run), takes the branch to global memory.
-  auto take = [&](bool kp, int j, int sb, bool range_ok) {
-    const int v = j + sb;
-    const bool fits = kSlot ? range_ok : (v > -32768 && v <= 32767);
-    const bool st = n < staged;
-    stage[st ? n : kFillStage][threadIdx.x] = fits ? (int16_t)v : kOut;
-    if (kp && !(st && fits)) {
-      const int64_t o = base + n * step;
-      if (n < len && o < cap) {
-        put_entry(nbr, d16, map, o, j, i, a.nref, bad);
-        if (kSlot && fits) T.slot[o] = (uint16_t)(v & 0xfff);
-      }
-    }
-    n += kp ? 1 : 0;
-  };
-  auto load = [&](int j) { return Cand{a.rpos[j], h_of(a.rh, j, a.h0)}; };
-  for_candidates(a, qi, over, [&](int b, int e, bool seam) {
-    // staged value of candidate j: j + sb
-    int sb = -i;
-    bool ok = true;
-    if (kSlot && e > b) {
-      int u = -1;
-      for (int r = 0; r < R; ++r) u = (b >= rt_s[r] && e <= rt_e[r]) ? r : u;
-      ok = u >= 0;
-      tbad = tbad || !ok;
-      sb = ok ? (u << 12) + rt_d[u] : 0;
-    }
-    if (seam)
-      scan_range<4>(b, e, load, [&](int j, const Cand& r) { take(keep_pair(qi, hi, r.x, r.h, a), j, sb, ok); });
-    else
-      scan_range<4>(b, e, load, [&](int j, const Cand& r) { take(keep_pair_near(qi, hi, r.x, r.h, a), j, sb, ok); });
-  });
-  for (int64_t t = 0; t < staged; ++t) {
-    const int64_t o = base + t * step;
-    if (o >= cap) continue;
-    if (t < n) {
-      const int16_t v = stage[t][threadIdx.x];
-      if (v == kOut) continue;
-      if (kSlot) {
-        const int w = (uint16_t)v, s = w & 0xfff;
-        put_entry(nbr, d16, map, o, s - rt_d[w >> 12], i, a.nref, bad);
-        T.slot[o] = (uint16_t)s;
-      } else {
-        put_entry(nbr, d16, map, o, i + v, i, a.nref, bad);
-      }
-    } else if (fixed_w == 0) {
-      nbr[o] = -1;
-    }
-  }
-  return n;
-}
+// Where the rows go.  Fixed width w > 0 (slice s at s * 64 * w, no count
+// pass): counts[i] = min(entries, w), *row_ovf set when a row has more
+// entries than w (the list is then incomplete).  Else sliced ELL (slice !=
+// NULL): the rest of the slice's columns padded with -1.  Else CSR: entries
+// at off[i] + n.  Writes stay below `cap` and inside the row's own range.
+struct FillOut {
+  const int32_t* off;
+  const int32_t* slice;
+  int32_t* nbr;
+  int64_t cap;
+  int16_t* d16;
+  int32_t* ovf;
+  int width;
+  int32_t* counts;
+  int32_t* row_ovf;
+  const int32_t* map;
+  int depth;  // staged entries per row (0: CSR)
+};
 
-// fixed_w > 0: the one-pass fixed-width layout (slice s at s * 64 * fixed_w,
-// no count pass): counts[i] = min(entries, fixed_w), *row_ovf set when a row
-// has more entries than fixed_w (the list is then incomplete).  kTiles: the
-// fixed-width layout with tile slots (T); a tile that does not fit T.cap
-// (or kFillTileMax) is filled without them, and one whose rows name a
-// candidate range outside its runs gets tile_n = -1.
-template <bool kTiles>
-__global__ void __launch_bounds__(kBlock) k_neighbor_fill(SearchArgs a, const int32_t* __restrict__ off,
-                                                          const int32_t* __restrict__ slice,
-                                                          int32_t* __restrict__ nbr, int64_t cap,
-                                                          int16_t* __restrict__ d16, int32_t* __restrict__ ovf,
-                                                          int fixed_w, int32_t* __restrict__ counts,
-                                                          int32_t* __restrict__ row_ovf,
-                                                          const int32_t* __restrict__ map, FillTiles T) {
-  // one extra row: the sink of the unconditional staging writes
-  __shared__ int16_t stage[kFillStage + 1][kBlock];
+// Neighbor rows [blockIdx * kRows, + kRows).  In the sliced layouts the first
+// `depth` entries of every row are staged in LDS (rows side by side, one
+// padding column: a wave writes one row at consecutive entries, so the odd
+// stride of kRows + 1 spreads them over the banks) and written column
+// by column after the scan, so each store covers whole lines; an entry past
+// them is written as it is found.  A CSR row is contiguous and takes no
+// staging.  kTiles: with tile slots (T), staged as (u << 12) | slot with u
+// the run of the candidate range, as ~j for a range outside the tile's runs
+// (tile_n = -1 then); a tile that does not fit T.cap (or kFillTileMax) is
+// filled without slots.
+template <int kRows, bool kTiles, bool kH>
+__global__ void __launch_bounds__(kBlock) k_neighbor_fill(SearchArgs a, FillOut F, FillTiles T) {
+  extern __shared__ int32_t stage[];
+  __shared__ Queries<kRows> Q;
+  __shared__ int2 run_add[kTiles ? 3 : 1][kTiles ? kRows : 1];
+  __shared__ int found[kRows];
   __shared__ int rt_s[kTileMaxRuns], rt_e[kTileMaxRuns], rt_d[kTileMaxRuns];
+  const int i0 = blockIdx.x * kRows;
+  const int tile = i0 / kBlock;
   bool fit = false;
   int R = 0;
   if (kTiles) {
-    // every thread reads tile_n before any may set it to -1 (barrier)
-    const int S = T.n[blockIdx.x];
-    fit = S >= 0 && S <= T.cap && S <= kFillTileMax;
-    if (fit) R = load_run_table(T.runs, blockIdx.x, rt_s, rt_e, rt_d);
+    // a workgroup of the same tile may set tile_n to -1 meanwhile: whoever
+    // reads that fills without slots, which no one then reads
+    const int S = T.n[tile];
+    fit = __syncthreads_and(S >= 0 && S <= T.cap && S <= kFillTileMax);
+    if (fit) R = load_run_table(T.runs, tile, rt_s, rt_e, rt_d);
     __syncthreads();
-    if (S > kFillTileMax && S <= T.cap && threadIdx.x == 0) T.n[blockIdx.x] = -1;
+    if (S > kFillTileMax && S <= T.cap && threadIdx.x == 0) T.n[tile] = -1;
   }
   bool bad = false, tbad = false, over = false;
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= a.nq) return;
-  float2 qi = a.qpos[i];
-  if (!a.wrapped) qi = make_float2(wrap_coord(qi.x, a.d, 0), wrap_coord(qi.y, a.d, 1));
-  float hi = h_of(a.qh, i, a.h0);
-  int64_t base, step, len;
-  if (fixed_w > 0) {
-    base = (int64_t)(i >> 6) * 64 * fixed_w + (i & 63);
-    step = 64;
-    len = fixed_w;
-  } else if (slice) {
-    const int s = i >> 6;
-    base = (int64_t)slice[s] + (i & 63);
-    step = 64;
-    len = ((int64_t)slice[s + 1] - slice[s]) >> 6;
-  } else {
-    base = off[i];
-    step = 1;
-    len = (int64_t)off[i + 1] - off[i];
-  }
-  const int64_t staged = (slice || fixed_w > 0) ? (kFillStage < len ? kFillStage : len) : 0;
-  const int64_t n = (kTiles && fit) ? fill_row<true>(a, i, qi, hi, base, step, len, staged, fixed_w, stage, nbr,
-                                                     cap, d16, map, T, rt_s, rt_e, rt_d, R, bad, tbad, over)
-                                    : fill_row<false>(a, i, qi, hi, base, step, len, staged, fixed_w, stage, nbr,
-                                                      cap, d16, map, T, rt_s, rt_e, rt_d, R, bad, tbad, over);
-  if (kTiles && tbad) T.n[blockIdx.x] = -1;
-  if (fixed_w > 0) {
-    // entries past the row's count are never read: no padding
-    counts[i] = n < len ? (int32_t)n : (int32_t)len;
-    if (n > len) atomicMax(row_ovf, 1);
-    if (over) atomicMax(row_ovf, 2);
-  } else {
-    for (int64_t t = n > staged ? n : staged; t < len; ++t) {
-      const int64_t o = base + t * step;
-      if (o < cap) nbr[o] = -1;
+  load_queries<kRows>(a, i0, Q, over, [&](int part, int r, const CellRow& cr) {
+    if (kTiles && fit) {
+      // what a candidate of each range adds to j for its staged value
+      auto run_of = [&](int b, int len) {
+        int u = -1;
+        for (int k = 0; k < R; ++k) u = (b >= rt_s[k] && b + len <= rt_e[k]) ? k : u;
+        if (u < 0 && len > 0) tbad = true;
+        return u < 0 ? kNoRun : (u << 12) + rt_d[u];
+      };
+      run_add[part][r] = make_int2(run_of(cr.b0, cr.len0), run_of(cr.b1, cr.len1 & (kSeamBit - 1)));
+    }
+  });
+  __syncthreads();
+  const bool slots = kTiles && fit;
+  auto row_of = [&](int i, int64_t& base, int64_t& step, int64_t& len) {
+    if (F.width > 0) {
+      base = (int64_t)(i >> 6) * 64 * F.width + (i & 63);
+      step = 64;
+      len = F.width;
+    } else if (F.slice) {
+      const int s = i >> 6;
+      base = (int64_t)F.slice[s] + (i & 63);
+      step = 64;
+      len = ((int64_t)F.slice[s + 1] - F.slice[s]) >> 6;
+    } else {
+      base = F.off[i];
+      step = 1;
+      len = (int64_t)F.off[i + 1] - F.off[i];
+    }
+  };
+  // slot of the reference particle a staged value stands for
+  auto ref_of = [&](int v) { return !slots ? v : (v >= 0 ? (v & 0xfff) - rt_d[v >> 12] : ~v); };
+  scan_queries<kRows, kH>(
+      a, Q, F.depth,
+      [&](int p, int r, bool first, int j) {
+        if (!slots) return j;
+        const int2 add = run_add[kTiles ? p : 0][kTiles ? r : 0];
+        const int ad = first ? add.x : add.y;
+        return ad == kNoRun ? ~j : j + ad;
+      },
+      [&](int r, int pos, int v) { stage[__umul24(pos, kRows + 1) + r] = v; },
+      [&](int r, int pos, int v) {
+        const int i = i0 + r;
+        int64_t base, step, len;
+        row_of(i, base, step, len);
+        const int64_t o = base + pos * step;
+        if (pos < len && o < F.cap) {
+          put_entry(F.nbr, F.d16, F.map, o, ref_of(v), i, a.nref, bad);
+          if (slots && v >= 0) T.slot[o] = (uint16_t)(v & 0xfff);
+        }
+      },
+      [&](int r, int n) { found[r] = n; });
+  if (kTiles && tbad) T.n[tile] = -1;
+  if (F.width > 0 && over) atomicMax(F.row_ovf, 2);
+  __syncthreads();
+  const int r = threadIdx.x % kRows, i = i0 + r;
+  if (i < a.nq) {
+    const int n = found[r];
+    int64_t base, step, len;
+    row_of(i, base, step, len);
+    if (F.width > 0 && threadIdx.x < kRows) {
+      // entries past the row's count are never read: no padding
+      F.counts[i] = n < len ? n : (int32_t)len;
+      if (n > len) atomicMax(F.row_ovf, 1);
+    }
+    if (F.depth > 0) {
+      const int staged = (int)(n < F.depth ? (n < len ? n : len) : (F.depth < len ? F.depth : len));
+      constexpr int kStep = kBlock / kRows;
+      int c = threadIdx.x / kRows;
+      if (!slots && !F.d16 && base + (int64_t)staged * 64 <= F.cap) {
+        // plain entries: four gathers through the map in flight
+        for (; c + 3 * kStep < staged; c += 4 * kStep) {
+          int j[4];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) j[u] = stage[(c + u * kStep) * (kRows + 1) + r];
+          if (F.map) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) j[u] = F.map[j[u]];
+          }
+#pragma unroll
+          for (int u = 0; u < 4; ++u) F.nbr[base + (int64_t)(c + u * kStep) * 64] = j[u];
+        }
+      }
+      for (; c < staged; c += kStep) {
+        const int64_t o = base + (int64_t)c * 64;
+        if (o >= F.cap) break;
+        const int v = stage[c * (kRows + 1) + r];
+        put_entry(F.nbr, F.d16, F.map, o, ref_of(v), i, a.nref, bad);
+        if (slots && v >= 0) T.slot[o] = (uint16_t)(v & 0xfff);
+      }
+      if (F.width == 0) {
+        for (; c < len; c += kBlock / kRows) {
+          const int64_t o = base + (int64_t)c * 64;
+          if (c >= n && o < F.cap) F.nbr[o] = -1;
+        }
+      }
     }
   }
-  if (bad) *ovf = 1;
+  if (bad) *F.ovf = 1;
+}
+
+template <int kRows, bool kH>
+static void launch_fill_rows(const SearchArgs& a, const FillOut& F, const FillTiles* tiles, hipStream_t st) {
+  const size_t lds = (size_t)F.depth * (kRows + 1) * sizeof(int32_t);
+  if (tiles)
+    k_neighbor_fill<kRows, true, kH><<<grid_for(a.nq, kRows), kBlock, lds, st>>>(a, F, *tiles);
+  else
+    k_neighbor_fill<kRows, false, kH><<<grid_for(a.nq, kRows), kBlock, lds, st>>>(a, F, FillTiles{});
+}
+
+static int launch_fill(const SearchArgs& a, FillOut F, const FillTiles* tiles, hipStream_t st) {
+  F.depth = F.width > 0 ? (F.width < kRowStage ? F.width : kRowStage) : (F.slice ? kRowStage : 0);
+  const bool vary = varied_support(a);
+  if (a.nq < kRowSmall)
+    vary ? launch_fill_rows<16, true>(a, F, tiles, st) : launch_fill_rows<16, false>(a, F, tiles, st);
+  else
+    vary ? launch_fill_rows<64, true>(a, F, tiles, st) : launch_fill_rows<64, false>(a, F, tiles, st);
+  return launch_status();
 }
 
 __global__ void __launch_bounds__(kBlock) k_fixed_slices(int nslices, int width, int32_t* __restrict__ slice_off,
@@ -602,7 +683,13 @@ extern "C" int dsph_neighbor_count(const dsph_domain* domain, const dsph_grid* g
   if (s != DSPH_OK) return s;
   if (nq > 0 && !counts) return DSPH_ERR_ARG;
   if (nq == 0) return DSPH_OK;
-  k_neighbor_count<<<grid_for(nq), kBlock, 0, as_stream(stream)>>>(a, counts);
+  hipStream_t st = as_stream(stream);
+  const bool vary = varied_support(a);
+  auto launch = [&](auto kernel, int rows) { kernel<<<grid_for(nq, rows), kBlock, 0, st>>>(a, counts); };
+  if (nq < kRowSmall)
+    vary ? launch(k_neighbor_count<16, true>, 16) : launch(k_neighbor_count<16, false>, 16);
+  else
+    vary ? launch(k_neighbor_count<64, true>, 64) : launch(k_neighbor_count<64, false>, 64);
   return launch_status();
 }
 
@@ -618,9 +705,7 @@ extern "C" int dsph_neighbor_fill(const dsph_domain* domain, const dsph_grid* gr
   if (nq == 0) return DSPH_OK;
   if ((!offsets && !slice_off) || (capacity > 0 && !nbr) || capacity < 0 || layout_total < 0) return DSPH_ERR_ARG;
   if (layout_total > capacity) return DSPH_ERR_CAPACITY;
-  k_neighbor_fill<false><<<grid_for(nq), kBlock, 0, as_stream(stream)>>>(
-      a, offsets, slice_off, nbr, capacity, nullptr, nullptr, 0, nullptr, nullptr, nullptr, FillTiles{});
-  return launch_status();
+  return launch_fill(a, FillOut{offsets, slice_off, nbr, capacity}, nullptr, as_stream(stream));
 }
 
 extern "C" int dsph_neighbor_fill16(const dsph_domain* domain, const dsph_grid* grid, const int32_t* cell_start,
@@ -642,9 +727,7 @@ extern "C" int dsph_neighbor_fill16(const dsph_domain* domain, const dsph_grid* 
   if (nq == 0) return DSPH_OK;
   if ((!offsets && !slice_off) || (capacity > 0 && !nbr) || capacity < 0 || layout_total < 0) return DSPH_ERR_ARG;
   if (layout_total > capacity) return DSPH_ERR_CAPACITY;
-  k_neighbor_fill<false><<<grid_for(nq), kBlock, 0, st>>>(a, offsets, slice_off, nbr, capacity, nbr16, overflow, 0,
-                                                           nullptr, nullptr, nullptr, FillTiles{});
-  return launch_status();
+  return launch_fill(a, FillOut{offsets, slice_off, nbr, capacity, nbr16, overflow}, nullptr, st);
 }
 
 namespace dsph {
@@ -672,13 +755,10 @@ static int fill_fixed(const dsph_domain* domain, const dsph_grid* grid, const in
   if (tiles) {
     int s2 = launch_tile_runs(nq, grid, domain, cell_start, tiles->runs, tiles->n, st);
     if (s2 != DSPH_OK) return s2;
-    k_neighbor_fill<true><<<grid_for(nq), kBlock, 0, st>>>(a, nullptr, nullptr, nbr, capacity, nbr16, delta_overflow,
-                                                          width, counts, row_overflow, map, *tiles);
-  } else {
-    k_neighbor_fill<false><<<grid_for(nq), kBlock, 0, st>>>(a, nullptr, nullptr, nbr, capacity, nbr16, delta_overflow,
-                                                           width, counts, row_overflow, map, FillTiles{});
   }
-  return launch_status();
+  return launch_fill(a,
+                     FillOut{nullptr, nullptr, nbr, capacity, nbr16, delta_overflow, width, counts, row_overflow, map},
+                     tiles, st);
 }
 }  // namespace dsph
 

@@ -397,6 +397,36 @@ def test_grid_cell_order_matches_oracle(orc, nside, hscale):
     np.testing.assert_array_equal(g.sort_index.cpu().numpy(), g_o.sort_index)
 
 
+# 33^2: a last workgroup of one row; 364^2 = 132496: the 64-row
+# workgroups.
+# Cells of 1.6 h and 2.4 h: cell rows beyond 64 and 128 candidates; 2.4 h of
+# 33^2 is a periodic grid under 7 cells (every row at the seam).
+@pytest.mark.parametrize("nside,hscale,per,vary", [
+    (33, 1.0, (True, True), False), (33, 2.4, (True, True), True), (33, 1.6, (False, True), False),
+    (364, 1.0, (True, False), True), (364, 1.6, (True, True), False), (364, 2.4, (False, False), False)])
+def test_search_rows_by_cell_match_oracle(orc, nside, hscale, per, vary):
+    """Rows of the search (a wave takes the queries of a cell together) equal
+    the oracle's in every layout, also past the staged depth."""
+    print(f"case {nside} {hscale} {per} {vary}", flush=True)
+    d, _ = _case(nside, 21, 0.4)
+    dev = torch.device("cuda:0")
+    h = np.float32(d["h"])
+    dom_o, dom = orc.make_domain((-1, -1), (1, 1), per), _lib.make_domain((-1, -1), (1, 1), per)
+    hs = float(h) * hscale
+    g_o = orc.grid_build(dom_o, d["pos"], hs)
+    hp = (h * (0.8 + 0.2 * np.random.default_rng(4).random(nside * nside))).astype(np.float32) if vary else None
+    g = CellGrid.build(torch.from_numpy(d["pos"]).to(dev), torch.from_numpy(hp).to(dev) if vary else None, dom, hs,
+                       h_uniform=0.0 if vary else float(h))
+    sh = hp[g_o.sort_index] if vary else None
+    c_o, off_o, nbr_o = orc.neighbors_cell(dom_o, g_o, g_o.sorted_pos, sh, h0=float(h), sorted_h=sh)
+    qh = g.sorted_h if vary else None
+    longest = int(c_o.max())
+    for layout, width in [("csr", 0), ("sell", 0), ("fixed", longest), ("fixed", longest + 70), ("fixed", longest - 1)]:
+        nl = search(g, g.sorted_pos, qh, "scatter", qpos_wrapped=True, layout=layout, width=width)
+        np.testing.assert_array_equal(nl.counts.cpu().numpy(), c_o)
+        np.testing.assert_array_equal(nl.csr_nbr().cpu().numpy()[: nbr_o.size], nbr_o)
+
+
 def test_gather_set_permutes_every_array():
     """dsph_gather_set: arrays of 1, 2 and 4 words per element (float32,
     float32 pairs, int64, float32 quads) permuted by one index in one pass
