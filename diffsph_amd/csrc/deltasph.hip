@@ -22,9 +22,11 @@
 #include "common.h"
 #include "deltasph_impl.h"
 #include "mdbc_op.h"
+#include "near_math.h"
 #include "pmath.h"
 
 namespace dsph {
+
 
 // The wall particles seen by the fluid rows: pair list with rows = fluid
 // particles (same order as the fluid list) and entries = boundary indices,
@@ -178,7 +180,208 @@ __global__ void __launch_bounds__(kBlock) k_dsph_normalization(PairsDev P, Bound
 }
 
 
+// The same pass for a uniform support (near_support), with the square root,
+// the reciprocals and the pair arithmetic of near_math.h and kLanes lanes per
+// row (sum_row: the sums run in row order, so the bits are those of the
+// kernel above).  A group of entries out of near_math.h's range is evaluated
+// with pair_geom.
+template <class DF, bool kVol, int kLanes>
+__global__ void __launch_bounds__(kBlock) k_dsph_normalization_near(PairsDev P, BoundaryDev B, DF domain,
+                                                                    const float* __restrict__ mass,
+                                                                    const float* __restrict__ rho,
+                                                                    const float* __restrict__ vol,
+                                                                    float4* __restrict__ L_out,
+                                                                    float2* __restrict__ ev_out,
+                                                                    float2* __restrict__ grad_rho) {
+  const int row = (int)((blockIdx.x * (unsigned)blockDim.x + threadIdx.x) / kLanes);
+  const bool valid = row < P.nq;
+  const int i = valid ? row : P.nq - 1;
+  const Dom dm = domain(i);
+  const float2 xi = P.qpos[i];
+  const float h = P.h0;
+  const KConst kc = kconst(h);
+  RowRef rr = row_ref(P, i);
+  if (!valid) rr.cnt = 0;
+  const float rho_i = rho[i];
+  auto ld = [&](int j) {
+    NbrXMR d;
+    d.x = P.rpos[j];
+    d.m = kVol ? vol[j] : mass[j];
+    d.r = rho[j];
+    return d;
+  };
+  auto put = [&](const Geom& g, float Vj, float rho_j, float(&t)[6]) {
+    const float s = -(g.q * g.h);  // -(distances * supports)
+    const float qx = s * g.ex, qy = s * g.ey;
+    const float kx = Vj * g.gx, ky = Vj * g.gy;
+    t[0] = qx * kx;
+    t[1] = qx * ky;
+    t[2] = qy * kx;
+    t[3] = qy * ky;
+    const float dr = rho_i - rho_j;
+    t[4] = dr * kx;
+    t[5] = dr * ky;
+  };
+  constexpr int U = 4;
+  float acc[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  sum_row<kLanes, U>(P.nbr, rr, i, acc, ld, [&](const NbrXMR(&d)[U], float(&t)[U][6]) {
+    float dx[U], dy[U], V[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      dx[u] = xi.x - d[u].x.x;
+      dy[u] = xi.y - d[u].x.y;
+      V[u] = kVol ? d[u].m : d[u].m / d[u].r;
+    }
+    wrap_offsets(dx, dy, dm);
+    NearRange range;
+#pragma unroll
+    for (int u = 0; u < U; ++u) put(pair_geom_near(dx[u], dy[u], h, kc, range), V[u], d[u].r, t[u]);
+    if (range.odd()) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) put(pair_geom(xi, d[u].x, h, kc, dm), V[u], d[u].r, t[u]);
+    }
+  });
+  float bx = 0.f, by = 0.f;
+  if (B.on) {
+    RowRef br = row_ref(B.P, i);
+    if (!valid) br.cnt = 0;
+    float b[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    // lanes past the row's end repeat its first entry (a row without entries takes no turn)
+    const int pad = br.cnt > 0 ? B.P.nbr[br.base] : 0;
+    sum_row<kLanes, 1>(
+        B.P.nbr, br, pad, b, [&](int j) { return j; }, [&](const int(&j)[1], float(&t)[1][6]) {
+          if (br.cnt > 0) {
+            const Geom g = pair_geom(xi, B.P.rpos[j[0]], pick_h(B.P.mode, h, h_of(B.P.rh, j[0], B.P.h0)), B.P.dom);
+            put(g, B.mass[j[0]] / B.rho[j[0]], B.rho[j[0]], t[0]);
+          } else {
+            for (int k = 0; k < 6; ++k) t[0][k] = 0.f;
+          }
+        });
+    for (int k = 0; k < 4; ++k) acc[k] = acc[k] + b[k];
+    bx = b[4];
+    by = b[5];
+  }
+  if (rr.cnt < 4) {
+    acc[0] = 1.f;
+    acc[1] = 0.f;
+    acc[2] = 0.f;
+    acc[3] = 1.f;
+  }
+  auto finish = [&](int k, const float(&m)[6], float wx, float wy) {
+    const dsph_pm::Pinv2 Lm = dsph_pm::pinv2x2(m[0], m[1], m[2], m[3]);
+    if (L_out) L_out[k] = make_float4(Lm.l00, Lm.l01, Lm.l10, Lm.l11);
+    if (ev_out) ev_out[k] = make_float2(Lm.ev0, Lm.ev1);
+    float ax = Lm.l00 * m[4] + Lm.l01 * m[5];
+    float ay = Lm.l10 * m[4] + Lm.l11 * m[5];
+    if (B.on) {
+      ax = ax + wx;
+      ay = ay + wy;
+    }
+    grad_rho[k] = make_float2(ax, ay);
+  };
+  if (kLanes == 1) {
+    if (valid) finish(i, acc, bx, by);
+    return;
+  }
+  // The pseudo-inverse is ~500 float64 instructions: one thread per row, the
+  // workgroup's rows side by side, instead of all lanes of a group (16k rows
+  // of 16 lanes: 22 -> 16 us).
+  __shared__ float sums[8][kBlock / kLanes];
+  const int r = threadIdx.x / kLanes;
+  if ((threadIdx.x & (kLanes - 1)) == 0) {
+    for (int k = 0; k < 6; ++k) sums[k][r] = acc[k];
+    sums[6][r] = bx;
+    sums[7][r] = by;
+  }
+  __syncthreads();
+  const int rows = blockDim.x / kLanes, t = threadIdx.x;
+  const int k = blockIdx.x * rows + t;
+  if (t >= rows || k >= P.nq) return;
+  const float m[6] = {sums[0][t], sums[1][t], sums[2][t], sums[3][t], sums[4][t], sums[5][t]};
+  finish(k, m, sums[6][t], sums[7][t]);
+}
+
 __device__ __forceinline__ float eos_p(float rho, float rho0, float c) { return c * (rho - rho0); }
+
+// Sums over the wall entries of a row: viscosity, continuity, pressure.
+struct WallSums {
+  float vx = 0.f, vy = 0.f, c = 0.f, px = 0.f, py = 0.f;
+};
+
+// The wall terms of one pair (zero where the wall has no viscosity).
+__device__ __forceinline__ void wall_terms(const BoundaryDev& B, const RhsArgs& A, float2 xi, float2 ui, float hi,
+                                           float rho_i, float p_i, int j, float (&t)[5]) {
+  const float h = pick_h(B.P.mode, hi, h_of(B.P.rh, j, B.P.h0));
+  const Geom g = pair_geom(xi, B.P.rpos[j], h, B.P.dom);
+  const float2 uj = B.vel[j];
+  const float rho_j = B.rho[j];
+  const float m_j = B.mass[j];
+  const float rij = g.q * g.h;
+  t[0] = t[1] = 0.f;
+  if (B.viscosity >= 0) {
+    const float vx = ui.x - uj.x, vy = ui.y - uj.y;
+    const float vr = vx * g.ex + vy * g.ey;
+    float pi = vr / (rij + B.visc_eps * (g.h * g.h));
+    if (B.pi_switch) pi = vr < 0.0f ? pi : 0.0f;
+    const float Vb = B.viscosity == 0 ? m_j / (rho_i + rho_j) : m_j / rho_j;
+    const float vs = Vb * pi;
+    t[0] = vs * g.gx;
+    t[1] = vs * g.gy;
+  }
+  const float qx = (uj.x - ui.x) * m_j, qy = (uj.y - ui.y) * m_j;
+  const float kq = qx * g.gx + qy * g.gy;
+  t[2] = (kq * rho_i) / rho_j;
+  const float Vj = m_j / rho_j;
+  const float ps = p_i + eos_p(rho_j, A.rho0, A.eos_c);
+  t[3] = ps * (Vj * g.gx);
+  t[4] = ps * (Vj * g.gy);
+}
+
+// dudt, drhodt (and the terms) of row i from its sums: acc = diffusion,
+// viscosity x / y, continuity, pressure x / y.
+__device__ __forceinline__ void finish_rhs(const RhsArgs& A, const BoundaryDev& B, int i, float hi, float rho_i,
+                                           float p_i, const float (&acc)[6], const WallSums& w) {
+  float apx = (-acc[4]) / rho_i, apy = (-acc[5]) / rho_i;
+  float vsx = 0.f, vsy = 0.f;
+  if (A.visc_scheme == 1) {
+    const float s = A.visc_c / rho_i;
+    vsx = s * acc[1];
+    vsy = s * acc[2];
+  } else if (A.visc_scheme == 0) {
+    const float s = (((A.visc_c * hi) * A.cs) * A.rho0) / rho_i;
+    vsx = s * acc[1];
+    vsy = s * acc[2];
+  }
+  float cont = -acc[3];
+  if (B.on) {
+    apx = apx + (-w.px) / rho_i;
+    apy = apy + (-w.py) / rho_i;
+    cont = cont + (-w.c);
+    if (B.viscosity == 1) {
+      const float s = B.visc_c_viscid / rho_i;
+      vsx = vsx + s * w.vx;
+      vsy = vsy + s * w.vy;
+    } else if (B.viscosity == 0) {
+      const float s = (((B.visc_coeff * hi) * A.cs) * A.rho0) / rho_i;
+      vsx = vsx + s * w.vx;
+      vsy = vsy + s * w.vy;
+    }
+  }
+  const float D = A.diffusion ? (((A.delta * hi) / A.kscale) * A.cs) * acc[0] : 0.0f;
+  A.dudt[i] = make_float2((apx + A.gx) + vsx, (apy + A.gy) + vsy);
+  A.drhodt[i] = cont + D;
+  if (A.terms) {
+    float* t = A.terms + (int64_t)i * 8;
+    t[0] = apx;
+    t[1] = apy;
+    t[2] = vsx;
+    t[3] = vsy;
+    t[4] = cont;
+    t[5] = D;
+    t[6] = p_i;
+    t[7] = 0.0f;
+  }
+}
 
 // With a boundary (deltaPlus.py:281-329, direction 'all' / 'boundaryToFluid'
 // for the fluid rows): continuity and pressure add the wall pairs as a
@@ -245,79 +448,131 @@ __global__ void __launch_bounds__(kBlock) k_dsph_rhs(PairsDev P, BoundaryDev B, 
       accPy += ps * ky;
     }
   });
-  float apx = (-accPx) / rho_i, apy = (-accPy) / rho_i;
-  float vsx = 0.f, vsy = 0.f;
-  if (A.visc_scheme == 1) {
-    const float s = A.visc_c / rho_i;
-    vsx = s * accVx;
-    vsy = s * accVy;
-  } else if (A.visc_scheme == 0) {
-    const float s = (((A.visc_c * hi) * A.cs) * A.rho0) / rho_i;
-    vsx = s * accVx;
-    vsy = s * accVy;
-  }
-  float cont = -accC;
+  WallSums w;
   if (B.on) {
-    float bVx = 0.f, bVy = 0.f, bC = 0.f, bPx = 0.f, bPy = 0.f;
     const RowRef br = row_ref(B.P, i);
     for (int n = 0, k = br.base; n < br.cnt; ++n, k += br.step) {
-      const int j = B.P.nbr[k];
-      const float h = pick_h(B.P.mode, hi, h_of(B.P.rh, j, B.P.h0));
-      const Geom g = pair_geom(xi, B.P.rpos[j], h, B.P.dom);
-      const float2 uj = B.vel[j];
-      const float rho_j = B.rho[j];
-      const float m_j = B.mass[j];
-      const float rij = g.q * g.h;
-      if (B.viscosity >= 0) {
-        const float vx = ui.x - uj.x, vy = ui.y - uj.y;
-        const float vr = vx * g.ex + vy * g.ey;
-        float pi = vr / (rij + B.visc_eps * (g.h * g.h));
-        if (B.pi_switch) pi = vr < 0.0f ? pi : 0.0f;
-        const float Vb = B.viscosity == 0 ? m_j / (rho_i + rho_j) : m_j / rho_j;
-        const float vs = Vb * pi;
-        bVx += vs * g.gx;
-        bVy += vs * g.gy;
-      }
-      {
-        const float qx = (uj.x - ui.x) * m_j, qy = (uj.y - ui.y) * m_j;
-        float kq = qx * g.gx + qy * g.gy;
-        kq = (kq * rho_i) / rho_j;
-        bC += kq;
-      }
-      {
-        const float Vj = m_j / rho_j;
-        const float ps = p_i + eos_p(rho_j, A.rho0, A.eos_c);
-        bPx += ps * (Vj * g.gx);
-        bPy += ps * (Vj * g.gy);
-      }
-    }
-    apx = apx + (-bPx) / rho_i;
-    apy = apy + (-bPy) / rho_i;
-    cont = cont + (-bC);
-    if (B.viscosity == 1) {
-      const float s = B.visc_c_viscid / rho_i;
-      vsx = vsx + s * bVx;
-      vsy = vsy + s * bVy;
-    } else if (B.viscosity == 0) {
-      const float s = (((B.visc_coeff * hi) * A.cs) * A.rho0) / rho_i;
-      vsx = vsx + s * bVx;
-      vsy = vsy + s * bVy;
+      float t[5];
+      wall_terms(B, A, xi, ui, hi, rho_i, p_i, B.P.nbr[k], t);
+      w.vx += t[0];
+      w.vy += t[1];
+      w.c += t[2];
+      w.px += t[3];
+      w.py += t[4];
     }
   }
-  const float D = A.diffusion ? (((A.delta * hi) / A.kscale) * A.cs) * accD : 0.0f;
-  A.dudt[i] = make_float2((apx + A.gx) + vsx, (apy + A.gy) + vsy);
-  A.drhodt[i] = cont + D;
-  if (A.terms) {
-    float* t = A.terms + (int64_t)i * 8;
-    t[0] = apx;
-    t[1] = apy;
-    t[2] = vsx;
-    t[3] = vsy;
-    t[4] = cont;
-    t[5] = D;
-    t[6] = p_i;
-    t[7] = 0.0f;
+  const float acc[6] = {accD, accVx, accVy, accC, accPx, accPy};
+  finish_rhs(A, B, i, hi, rho_i, p_i, acc, w);
+}
+
+// The right-hand side for a uniform support (near_support) with density
+// diffusion and a viscosity (the scheme as the solvers run it), as the
+// normalization above: near_math.h, kLanes lanes per row, the bits of
+// k_dsph_rhs.  The reciprocal of rho_j serves V_j and the continuity term.
+template <class DF, int kLanes, bool kSwitch>
+__global__ void __launch_bounds__(kBlock) k_dsph_rhs_near(PairsDev P, BoundaryDev B, RhsArgs A, DF domain) {
+  const int row = (int)((blockIdx.x * (unsigned)blockDim.x + threadIdx.x) / kLanes);
+  const bool valid = row < P.nq;
+  const int i = valid ? row : P.nq - 1;
+  const Dom dm = domain(i);
+  const float2 xi = P.qpos[i];
+  const float h = P.h0;
+  const float2 ui = A.vel[i];
+  const float rho_i = A.rho[i];
+  const float2 gri = A.grad_rho[i];
+  const float p_i = eos_p(rho_i, A.rho0, A.eos_c);
+  const KConst kc = kconst(h);
+  const float eps_d = 1e-6f * h, eps_v = A.eps * (h * h);
+  RowRef rr = row_ref(P, i);
+  if (!valid) rr.cnt = 0;
+  auto ld = [&](int j) {
+    NbrRhs d;
+    d.x = P.rpos[j];
+    d.u = A.vel[j];
+    d.r = A.rho[j];
+    d.m = A.mass[j];
+    d.g = A.grad_rho[j];
+    return d;
+  };
+  // the pair's terms from its quotients: V_j, the diffusion's r_ij, the
+  // viscosity's pi and the continuity's last factor
+  auto put = [&](const Geom& g, const NbrRhs& e, float Vj, float r_ij, float pi, float cont, float(&t)[6]) {
+    const float kx = Vj * g.gx, ky = Vj * g.gy;
+    const float psx = (-r_ij) * g.ex + (gri.x + e.g.x);
+    const float psy = (-r_ij) * g.ey + (gri.y + e.g.y);
+    t[0] = psx * kx + psy * ky;
+    const float vs = Vj * pi;
+    t[1] = vs * g.gx;
+    t[2] = vs * g.gy;
+    t[3] = cont;
+    const float ps = p_i + eos_p(e.r, A.rho0, A.eos_c);
+    t[4] = ps * kx;
+    t[5] = ps * ky;
+  };
+  auto vr_of = [&](const Geom& g, const NbrRhs& e) {
+    const float vx = ui.x - e.u.x, vy = ui.y - e.u.y;
+    return vx * g.ex + vy * g.ey;
+  };
+  auto kq_of = [&](const Geom& g, const NbrRhs& e) {
+    const float qx = (e.u.x - ui.x) * e.m, qy = (e.u.y - ui.y) * e.m;
+    const float kq = qx * g.gx + qy * g.gy;
+    return kq * rho_i;
+  };
+  constexpr int U = 4;
+  float acc[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  sum_row<kLanes, U>(P.nbr, rr, i, acc, ld, [&](const NbrRhs(&d)[U], float(&t)[U][6]) {
+    float dx[U], dy[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      dx[u] = xi.x - d[u].x.x;
+      dy[u] = xi.y - d[u].x.y;
+    }
+    wrap_offsets(dx, dy, dm);
+    NearRange range;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const NbrRhs& e = d[u];
+      const Geom g = pair_geom_near(dx[u], dy[u], h, kc, range);
+      const float ir = range.divisor(e.r);
+      const float rij = g.q * g.h;  // distances * supports
+      const float dr = 2.0f * (e.r - rho_i), bd = rij + eps_d;
+      const float vr = vr_of(g, e), bv = rij + eps_v;
+      const float kq = kq_of(g, e);
+      range.operand(e.m);
+      range.operand(vr);
+      range.operand(kq);
+      float pi = div_near(vr, bv, rcp_near(bv));
+      if (kSwitch) pi = vr < 0.0f ? pi : 0.0f;
+      put(g, e, div_near(e.m, e.r, ir), div_near(dr, bd, rcp_near(bd)), pi, div_near(kq, e.r, ir), t[u]);
+    }
+    if (range.odd()) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const NbrRhs& e = d[u];
+        const Geom g = pair_geom(xi, e.x, h, kc, dm);
+        const float rij = g.q * g.h;
+        const float vr = vr_of(g, e);
+        float pi = vr / (rij + eps_v);
+        if (kSwitch) pi = vr < 0.0f ? pi : 0.0f;
+        put(g, e, e.m / e.r, (2.0f * (e.r - rho_i)) / (rij + eps_d), pi, kq_of(g, e) / e.r, t[u]);
+      }
+    }
+  });
+  WallSums w;
+  if (B.on) {
+    RowRef br = row_ref(B.P, i);
+    if (!valid) br.cnt = 0;
+    float b[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
+    const int pad = br.cnt > 0 ? B.P.nbr[br.base] : 0;
+    sum_row<kLanes, 1>(
+        B.P.nbr, br, pad, b, [&](int j) { return j; }, [&](const int(&j)[1], float(&t)[1][5]) {
+          for (int k = 0; k < 5; ++k) t[0][k] = 0.f;
+          if (br.cnt > 0) wall_terms(B, A, xi, ui, h, rho_i, p_i, j[0], t[0]);
+        });
+    w = WallSums{b[0], b[1], b[2], b[3], b[4]};
   }
+  if (!valid || (threadIdx.x & (kLanes - 1)) != 0) return;
+  finish_rhs(A, B, i, h, rho_i, p_i, acc, w);
 }
 
 // out = base + k * c for the three state fields (any may be absent).
@@ -673,6 +928,58 @@ extern "C" int dsph_volume(int64_t n, const float* mass, const float* rho, float
   return launch_volume((int)n, mass, rho, vol, as_stream(stream));
 }
 
+// Lanes per row of the *_near kernels.  More lanes shorten a row's chain and
+// fill the chip with fewer rows, but each of them adds all terms, so the
+// fewest that keep ~4 waves on every SIMD win.  Normalization / right-hand
+// side, us, with 16, 4 and 1 lanes: 4k rows 10 / 6.2, 13.7 / 10.6 and 32.6 /
+// 36.9; 16k 16.0 / 9.9, 12.5 / 10.7; 27k 21.2 / 15.6, 15.3 / 13.8; 131k - ,
+// 33 / 38, 41 / 50; 262k - , 48 / 57, 42 / 51 (one thread per row with the
+// IEEE forms and no prefetch of the entries, before: 4k 33 / 39, 131k with
+// walls 48 / 58, 262k 51 / 68, 7.8M 1099 / 1597, now 890 / 1290).
+static int row_lanes(int64_t nq, int64_t up_to_16) { return nq <= up_to_16 ? 16 : (nq <= (1 << 17) ? 4 : 1); }
+constexpr int64_t kNorm16 = 1 << 13, kRhs16 = 1 << 14;
+
+template <class DF>
+static int launch_normalization(const PairsDev& P, const BoundaryDev& B, const DF& dom, const float* mass,
+                                const float* rho, const float* vol, float4* L, float2* ev, float2* grad, int block,
+                                hipStream_t st) {
+  auto go = [&](auto kernel, int lanes) {
+    kernel<<<grid_for(P.nq, block / lanes), block, 0, st>>>(P, B, dom, mass, rho, vol, L, ev, grad);
+    return launch_status();
+  };
+  if (!near_support(P))
+    return vol ? go(k_dsph_normalization<DF, true>, 1) : go(k_dsph_normalization<DF, false>, 1);
+  switch (row_lanes(P.nq, kNorm16)) {
+    case 16:
+      return vol ? go(k_dsph_normalization_near<DF, true, 16>, 16) : go(k_dsph_normalization_near<DF, false, 16>, 16);
+    case 4:
+      return vol ? go(k_dsph_normalization_near<DF, true, 4>, 4) : go(k_dsph_normalization_near<DF, false, 4>, 4);
+    default:
+      return vol ? go(k_dsph_normalization_near<DF, true, 1>, 1) : go(k_dsph_normalization_near<DF, false, 1>, 1);
+  }
+}
+
+template <class DF>
+static int launch_rhs(const PairsDev& P, const BoundaryDev& B, const RhsArgs& A, const DF& dom, int block,
+                      hipStream_t st) {
+  auto go = [&](auto kernel, int lanes) {
+    kernel<<<grid_for(P.nq, block / lanes), block, 0, st>>>(P, B, A, dom);
+    return launch_status();
+  };
+  // the viscosity's denominator must stay away from zero
+  const float ev = A.eps * (P.h0 * P.h0);
+  if (!near_support(P) || !A.diffusion || A.visc_scheme < 0 || !(ev >= 0x1p-58f && ev <= 0x1p40f))
+    return go(k_dsph_rhs<DF>, 1);
+  switch (row_lanes(P.nq, kRhs16)) {
+    case 16:
+      return A.pi_switch ? go(k_dsph_rhs_near<DF, 16, true>, 16) : go(k_dsph_rhs_near<DF, 16, false>, 16);
+    case 4:
+      return A.pi_switch ? go(k_dsph_rhs_near<DF, 4, true>, 4) : go(k_dsph_rhs_near<DF, 4, false>, 4);
+    default:
+      return A.pi_switch ? go(k_dsph_rhs_near<DF, 1, true>, 1) : go(k_dsph_rhs_near<DF, 1, false>, 1);
+  }
+}
+
 extern "C" int dsph_deltasph_normalization_v(const dsph_pairs* pairs, const dsph_boundary* boundary,
                                              const float* mass, const float* rho, const float* vol, float* L,
                                              float* eigvals, float* grad_rho, void* stream) {
@@ -687,13 +994,7 @@ extern "C" int dsph_deltasph_normalization_v(const dsph_pairs* pairs, const dsph
   float4* Lo = reinterpret_cast<float4*>(L);
   float2* eo = reinterpret_cast<float2*>(eigvals);
   float2* go = reinterpret_cast<float2*>(grad_rho);
-  if (vol)
-    k_dsph_normalization<OneDomain, true><<<grid_for(P.nq), kBlock, 0, as_stream(stream)>>>(
-        P, B, OneDomain{P.dom}, mass, rho, vol, Lo, eo, go);
-  else
-    k_dsph_normalization<OneDomain, false><<<grid_for(P.nq), kBlock, 0, as_stream(stream)>>>(
-        P, B, OneDomain{P.dom}, mass, rho, nullptr, Lo, eo, go);
-  return launch_status();
+  return launch_normalization(P, B, OneDomain{P.dom}, mass, rho, vol, Lo, eo, go, kBlock, as_stream(stream));
 }
 
 extern "C" int dsph_deltasph_normalization(const dsph_pairs* pairs, const dsph_boundary* boundary, const float* mass,
@@ -738,22 +1039,15 @@ int dsph::launch_normalization_per_particle(const PairsDev& P, const Dom* doms, 
                                             int block, hipStream_t st) {
   if (block != 64 && block != 128 && block != 256) return DSPH_ERR_ARG;
   if (P.nq == 0) return DSPH_OK;
-  const DomainPerParticle dp{doms, dom_of};
-  if (vol)
-    k_dsph_normalization<DomainPerParticle, true><<<grid_for(P.nq, block), block, 0, st>>>(
-        P, make_boundary(nullptr), dp, mass, rho, vol, nullptr, nullptr, grad_rho);
-  else
-    k_dsph_normalization<DomainPerParticle, false><<<grid_for(P.nq, block), block, 0, st>>>(
-        P, make_boundary(nullptr), dp, mass, rho, nullptr, nullptr, nullptr, grad_rho);
-  return launch_status();
+  return launch_normalization(P, make_boundary(nullptr), DomainPerParticle{doms, dom_of}, mass, rho, vol, nullptr,
+                              nullptr, grad_rho, block, st);
 }
 
 int dsph::launch_rhs_per_particle(const PairsDev& P, const RhsArgs& A, const Dom* doms, const int32_t* dom_of,
                                   int block, hipStream_t st) {
   if (block != 64 && block != 128 && block != 256) return DSPH_ERR_ARG;
   if (P.nq == 0) return DSPH_OK;
-  k_dsph_rhs<<<grid_for(P.nq, block), block, 0, st>>>(P, make_boundary(nullptr), A, DomainPerParticle{doms, dom_of});
-  return launch_status();
+  return launch_rhs(P, make_boundary(nullptr), A, DomainPerParticle{doms, dom_of}, block, st);
 }
 
 extern "C" int dsph_deltasph_rhs(const dsph_pairs* pairs, const dsph_boundary* boundary,
@@ -773,8 +1067,7 @@ extern "C" int dsph_deltasph_rhs(const dsph_pairs* pairs, const dsph_boundary* b
   PairsDev P = make_pairs(*pairs);
   BoundaryDev B = make_boundary(boundary);
   if (B.on && B.viscosity == 1) B.visc_c_viscid = (float)(2.0 * 4.0 * (double)B.visc_coeff * (double)prm->rho0);
-  k_dsph_rhs<<<grid_for(P.nq), kBlock, 0, as_stream(stream)>>>(P, B, A, OneDomain{P.dom});
-  return launch_status();
+  return launch_rhs(P, B, A, OneDomain{P.dom}, kBlock, as_stream(stream));
 }
 
 extern "C" int dsph_rk_update(int64_t n, const float* x0, const float* dxdt, float* x, const float* u0,

@@ -2,13 +2,14 @@
 multi-step RK4 trajectories bit for bit, the float64 error of the float32
 path, and Taylor-Green properties at 512^2 (the differentiable-rollout
 size)."""
+import ctypes as C
 import math
 
 import numpy as np
 import pytest
 import torch
 
-from diffsph_amd import sampling
+from diffsph_amd import _lib, sampling
 from diffsph_amd.deltasph import (DeltaSPHConfig, DeltaSPHSolver, analytic_tgv_energy_ratio, compute_timestep,
                                   taylor_green_state)
 from oracle import oracle as orc
@@ -270,3 +271,51 @@ def test_dam_break_config_properties():
     under = (wp[:, 0] > 0.1) & (wp[:, 0] < 0.5) & (wp[:, 1] < 0)
     assert int(under.sum()) > 200
     assert float((wr[under] - cfg.rho0).abs().max()) < 0.01 * cfg.rho0
+
+
+# rows of 16, 4 and 1 lanes, with a last workgroup that is not full
+@pytest.mark.parametrize("nside", [33, 91, 131, 363])
+@pytest.mark.parametrize("state", ["plain", "switch", "odd"])
+def test_near_kernels_equal_general_kernels(nside, state):
+    """The uniform-support kernels give the bits of the general ones (reached
+    by passing the same support per particle), also for operands out of
+    their fast range: zero, tiny and huge densities, infinities, NaN, pairs
+    closer than 2^-48."""
+    print(f"case {nside} {state}", flush=True)
+    rng = np.random.default_rng(3)
+    pos, dx = sampling.sample_regular(nside)
+    pos = sampling.jitter(pos, dx, 0.3, 5).astype(np.float32)
+    n = pos.shape[0]
+    vel = rng.standard_normal((n, 2)).astype(np.float32)
+    rho = (1.0 + 0.01 * rng.standard_normal(n)).astype(np.float32)
+    if state == "odd":
+        pos[0] = (1e-16, 1e-17)
+        pos[1] = (1e-16, 3e-16)
+        pick = rng.permutation(n)[:12]
+        rho[pick[:6]] = [0.0, 1e-30, 1e30, np.inf, np.nan, -1.0]
+        vel[pick[6:11], 0] = [np.inf, np.nan, 1e25, 0.0, -np.inf]
+    h = sampling.volume_to_support(dx * dx, 50.0)
+    dev = torch.device("cuda:0")
+    T = lambda a: torch.from_numpy(np.ascontiguousarray(a, np.float32)).to(dev)  # noqa: E731
+    cfg = DeltaSPHConfig(support=h, dx=dx, viscosity="deltaSPH_inviscid" if state == "switch" else "deltaSPH_viscid",
+                         pi_switch=state == "switch")
+    sv = DeltaSPHSolver(T(pos), T(vel), T(np.full(n, dx * dx)), T(rho), cfg)
+    nl, pr, wpos, grid = sv.neighbors(sv.pos)
+    L, st = _lib.lib(), _lib.stream_handle(dev)
+    hs = torch.full((n,), h, dtype=torch.float32, device=dev)
+    out = []
+    for general in (False, True):
+        pr.qh = pr.rh = _lib.ptr(hs) if general else None
+        vol, g, m = torch.empty(n, device=dev), torch.empty(n, 2, device=dev), torch.empty(n, 4, device=dev)
+        g2, du, dr = torch.empty(n, 2, device=dev), torch.empty(n, 2, device=dev), torch.empty(n, device=dev)
+        P = _lib.ptr
+        _lib.check(L.dsph_volume(n, P(sv.mass), P(sv.rho), P(vol), st), "volume")
+        _lib.check(L.dsph_deltasph_normalization_v(C.byref(pr), None, P(sv.mass), P(sv.rho), P(vol), P(m), None, P(g),
+                                                   st), "normalization")
+        _lib.check(L.dsph_deltasph_normalization_v(C.byref(pr), None, P(sv.mass), P(sv.rho), None, None, None, P(g2),
+                                                   st), "normalization")
+        _lib.check(L.dsph_deltasph_rhs(C.byref(pr), None, C.byref(sv.prm), P(sv.vel), P(sv.mass), P(sv.rho), P(g),
+                                       P(du), P(dr), None, st), "rhs")
+        out.append([t.cpu().numpy() for t in (m, g, g2, du, dr)])
+    for name, a, b in zip(("L", "grad", "grad, no volumes", "dudt", "drhodt"), *out):
+        np.testing.assert_array_equal(a, b, err_msg=name)
