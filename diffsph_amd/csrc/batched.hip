@@ -11,7 +11,7 @@
 // 231-307 + v2/modules/timestep.py:8-39 as the single-domain entry points
 // run it):
 //   sort:   cell keys (global cell = domain cell offset + local cell) ->
-//           counting sort with per-cell insertion sort -> permute the state
+//           counting sort, ranked by index within a cell -> permute the state
 //           A -> B (B is in cell order; domains stay contiguous)
 //   stage s = 0..3: grid of the stage positions (stage 0 reuses the sort's)
 //           -> fixed-width sliced-ELL rows (entries mapped to state order)
@@ -56,7 +56,7 @@ constexpr int64_t kSqStride = (int64_t)kSqBlocks * kBlock;
 inline size_t a256(size_t b) { return (b + 255) / 256 * 256; }
 
 struct Layout {
-  size_t doms, grids, dom_of, slice, cnt, nbr, keys, slot, si, cell_count, cell_start, scan, wq, spos;
+  size_t doms, grids, dom_of, slice, cnt, nbr, keys, slot, order, si, cell_count, cell_start, scan, wq, spos;
   size_t Bpos, Bvel, Bmass, Brho, Buid;
   size_t Spos[3], Svel[3], Srho[3];
   size_t ku[4], kr[4];
@@ -83,6 +83,7 @@ Layout make_layout(int64_t n, int ndom, int64_t ncell, int width) {
   L.nbr = take((size_t)4 * L.npad * width);
   L.keys = take(4 * n);
   L.slot = take(4 * n);
+  L.order = take(4 * n);
   L.si = take(4 * n);
   L.cell_count = take(4 * ncell);
   L.cell_start = take(4 * (ncell + 1));
@@ -155,30 +156,28 @@ __global__ void __launch_bounds__(kBlock) k_bkeys(int n, const float2* __restric
   if (valid) slot[i] = sl;
 }
 
+// Particles of each cell side by side, in any order.
 __global__ void __launch_bounds__(kBlock) k_bscatter(int n, const int32_t* __restrict__ keys,
                                                      const int32_t* __restrict__ slot,
                                                      const int32_t* __restrict__ cell_start,
-                                                     int32_t* __restrict__ si) {
+                                                     int32_t* __restrict__ order) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  si[cell_start[keys[i]] + slot[i]] = i;
+  order[cell_start[keys[i]] + slot[i]] = i;
 }
 
-// Insertion sort of each cell by particle index (deterministic order).
-__global__ void __launch_bounds__(kBlock) k_bcellsort(int ncell, const int32_t* __restrict__ cell_start,
-                                                      int32_t* __restrict__ si) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= ncell) return;
-  const int b = cell_start[c], e = cell_start[c + 1];
-  for (int a = b + 1; a < e; ++a) {
-    const int v = si[a];
-    int k = a - 1;
-    while (k >= b && si[k] > v) {
-      si[k + 1] = si[k];
-      --k;
-    }
-    si[k + 1] = v;
-  }
+// The final order, by particle index within each cell (cell_rank); with
+// `dst`, dst[slot] = src[particle] in the same pass.
+__global__ void __launch_bounds__(kBlock) k_bcellrank(int n, const int32_t* __restrict__ keys,
+                                                      const int32_t* __restrict__ slot,
+                                                      const int32_t* __restrict__ cell_start,
+                                                      const int32_t* __restrict__ order, int32_t* __restrict__ si,
+                                                      const float2* __restrict__ src, float2* __restrict__ dst) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const int p = cell_rank(i, keys[i], slot, cell_start, order);
+  si[p] = i;
+  if (dst) dst[p] = src[i];
 }
 
 // State A -> B in cell order; wout[p] = wrapped position of B's particle p.
@@ -199,13 +198,6 @@ __global__ void __launch_bounds__(kBlock) k_bpermute(int n, const int32_t* __res
   Brho[p] = rho[i];
   Buid[p] = uid[i];
   wout[p] = win[i];
-}
-
-__global__ void __launch_bounds__(kBlock) k_bgather2(int n, const int32_t* __restrict__ si,
-                                                     const float2* __restrict__ src, float2* __restrict__ dst) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= n) return;
-  dst[p] = src[si[p]];
 }
 
 // kTurns times kRows rows (state order) of the fixed-width sliced ELL per
@@ -484,8 +476,9 @@ struct Ctx {
 };
 
 // Cell grid of positions x (state order): wrapped positions into wq, sorted
-// slots into si, cell starts; with permute, also the state A -> B.
-int build_grid(const Ctx& c, const float2* x, float2* wq) {
+// slots into si, cell starts, the sorted wrapped positions into spos (unless
+// NULL).
+int build_grid(const Ctx& c, const float2* x, float2* wq, float2* spos) {
   const Layout& L = c.L;
   int32_t* cc = c.p<int32_t>(L.cell_count);
   k_fill_i32<<<grid_for(c.ncell), kBlock, 0, c.st>>>(cc, c.ncell, 0);
@@ -496,8 +489,10 @@ int build_grid(const Ctx& c, const float2* x, float2* wq) {
   int s = scan_exclusive(cc, c.ncell, c.p<int32_t>(L.cell_start), c.p<void>(L.scan), scan_ws(c.ncell), c.st);
   if (s != DSPH_OK) return s;
   k_bscatter<<<c.grid(c.n), c.block, 0, c.st>>>(c.n, c.p<int32_t>(L.keys), c.p<int32_t>(L.slot),
-                                                c.p<int32_t>(L.cell_start), c.p<int32_t>(L.si));
-  k_bcellsort<<<c.grid(c.ncell), c.block, 0, c.st>>>(c.ncell, c.p<int32_t>(L.cell_start), c.p<int32_t>(L.si));
+                                                c.p<int32_t>(L.cell_start), c.p<int32_t>(L.order));
+  k_bcellrank<<<c.grid(c.n), c.block, 0, c.st>>>(c.n, c.p<int32_t>(L.keys), c.p<int32_t>(L.slot),
+                                                 c.p<int32_t>(L.cell_start), c.p<int32_t>(L.order),
+                                                 c.p<int32_t>(L.si), wq, spos);
   return launch_status();
 }
 
@@ -567,7 +562,7 @@ int one_step(const Ctx& c, const dsph_deltasph_params* prm, const dsph_timestep_
   float2* Bvel = c.p<float2>(L.Bvel);
   float* Brho = c.p<float>(L.Brho);
   // sort A into cell order -> B; wq = wrapped B positions
-  int s = build_grid(c, pos, spos);
+  int s = build_grid(c, pos, spos, nullptr);
   if (s != DSPH_OK) return s;
   k_bpermute<<<c.grid(c.n), c.block, 0, c.st>>>(c.n, si, pos, vel, mass, rho, uid, spos, Bpos, Bvel,
                                                 c.p<float>(L.Bmass), Brho, c.p<int32_t>(L.Buid), wq);
@@ -580,10 +575,8 @@ int one_step(const Ctx& c, const dsph_deltasph_params* prm, const dsph_timestep_
       // the sorted state's grid is the sort's own (identity order)
       s = fill_rows(c, wq, wq, nullptr);
     } else {
-      s = build_grid(c, sx[k], wq);
+      s = build_grid(c, sx[k], wq, spos);
       if (s != DSPH_OK) return s;
-      k_bgather2<<<c.grid(c.n), c.block, 0, c.st>>>(c.n, si, wq, spos);
-      DSPH_LAUNCH_CHECK();
       s = fill_rows(c, wq, spos, si);
     }
     if (s != DSPH_OK) return s;
@@ -853,9 +846,8 @@ extern "C" int dsph_batch_probe(const dsph_batch* batch, const float* pos, int32
   int32_t* status = c.p<int32_t>(c.L.status);
   k_fill_i32<<<1, kBlock, 0, st>>>(status, 4, 0);
   float2* wq = c.p<float2>(c.L.wq);
-  s = build_grid(c, reinterpret_cast<const float2*>(pos), wq);
+  s = build_grid(c, reinterpret_cast<const float2*>(pos), wq, c.p<float2>(c.L.spos));
   if (s != DSPH_OK) return s;
-  k_bgather2<<<c.grid(c.n), c.block, 0, st>>>(c.n, c.p<int32_t>(c.L.si), wq, c.p<float2>(c.L.spos));
   s = fill_rows(c, wq, c.p<float2>(c.L.spos), c.p<int32_t>(c.L.si), true);
   if (s != DSPH_OK) return s;
   int32_t h[4] = {0, 0, 0, 0};

@@ -1,9 +1,9 @@
 // Cell-list neighbor search on a dense grid (gfx950).
 //
 // Build: key = cell of the wrapped position -> per-cell histogram (atomics
-// give a provisional slot) -> exclusive scan -> scatter -> per-cell sort by
-// original index (makes the order deterministic) -> gather positions and
-// supports into cell order.
+// give a provisional slot) -> exclusive scan -> scatter -> rank by original
+// index within the cell (makes the order deterministic), with positions and
+// supports moved into cell order in the same pass.
 // Query: a wave takes the queries of one cell together (row_search.h); the
 // three cells of a row are one contiguous slice of the sorted arrays unless
 // the row wraps around a periodic x boundary.
@@ -48,66 +48,31 @@ __global__ void __launch_bounds__(kBlock) k_cell_keys(const float2* __restrict__
   if (valid) slot[i] = sl;
 }
 
+// Particles of each cell side by side, in any order (`order`, scratch).
 __global__ void __launch_bounds__(kBlock) k_cell_scatter(int n, const int32_t* __restrict__ keys,
                                                          const int32_t* __restrict__ slot,
                                                          const int32_t* __restrict__ cell_start,
-                                                         int32_t* __restrict__ sort_index) {
+                                                         int32_t* __restrict__ order) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  sort_index[cell_start[keys[i]] + slot[i]] = i;
+  order[cell_start[keys[i]] + slot[i]] = i;
 }
 
-// Each cell's slice sorted by original index (cells hold ~16 particles),
-// one thread per cell.  A slice of up to kSortLds entries is loaded into
-// the thread's LDS column with its loads in flight together, and each entry
-// goes to its rank (the count of smaller entries: the indices are
-// distinct); a longer one is insertion-sorted in place.
-constexpr int kSortLds = 32;
-__global__ void __launch_bounds__(kBlock) k_cell_sort(int ncell, const int32_t* __restrict__ cell_start,
-                                                      int32_t* __restrict__ sort_index) {
-  __shared__ int32_t col[kSortLds][kBlock];
-  int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= ncell) return;
-  int b = cell_start[c], e = cell_start[c + 1];
-  const int m = e - b;
-  const int t = threadIdx.x;
-  if (m > DSPH_CELL_MAX) return;  // a diverged state: the search reports it
-  if (m <= kSortLds) {
-    for (int a0 = 0; a0 < m; a0 += 8) {
-      int v[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) v[u] = a0 + u < m ? sort_index[b + a0 + u] : 0;
-#pragma unroll
-      for (int u = 0; u < 8; ++u)
-        if (a0 + u < m) col[a0 + u][t] = v[u];
-    }
-    for (int a = 0; a < m; ++a) {
-      const int v = col[a][t];
-      int r = 0;
-      for (int u = 0; u < m; ++u) r += col[u][t] < v ? 1 : 0;
-      sort_index[b + r] = v;
-    }
-    return;
-  }
-  for (int a = b + 1; a < e; ++a) {
-    int v = sort_index[a];
-    int k = a - 1;
-    while (k >= b && sort_index[k] > v) {
-      sort_index[k + 1] = sort_index[k];
-      --k;
-    }
-    sort_index[k + 1] = v;
-  }
-}
-
-__global__ void __launch_bounds__(kBlock) k_sorted_gather(int n, Dom d, const int32_t* __restrict__ sort_index,
-                                                          const float2* __restrict__ pos, const float* __restrict__ h,
-                                                          float2* __restrict__ spos, float* __restrict__ sh,
-                                                          int32_t* __restrict__ rank) {
-  int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= n) return;
-  int i = sort_index[p];
-  float2 x = pos[i];
+// The final order, by original index within each cell: particle i goes to its
+// rank in the cell (cell_rank, row_search.h), with its sorted position,
+// support and rank in the same pass.
+__global__ void __launch_bounds__(kBlock) k_cell_rank(int n, Dom d, const int32_t* __restrict__ keys,
+                                                      const int32_t* __restrict__ slot,
+                                                      const int32_t* __restrict__ cell_start,
+                                                      const int32_t* __restrict__ order,
+                                                      const float2* __restrict__ pos, const float* __restrict__ h,
+                                                      int32_t* __restrict__ sort_index, float2* __restrict__ spos,
+                                                      float* __restrict__ sh, int32_t* __restrict__ rank) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const int p = cell_rank(i, keys[i], slot, cell_start, order);
+  const float2 x = pos[i];
+  sort_index[p] = i;
   spos[p] = make_float2(wrap_coord(x.x, d, 0), wrap_coord(x.y, d, 1));
   if (sh) sh[p] = h[i];
   if (rank) rank[i] = p;
@@ -627,7 +592,7 @@ extern "C" int dsph_grid_dims(const dsph_domain* domain, float hsearch, dsph_gri
 extern "C" size_t dsph_grid_build_workspace(int64_t n, const dsph_grid* grid) {
   if (!grid) return 0;
   int64_t ncell = (int64_t)grid->ncell[0] * grid->ncell[1];
-  return align256((size_t)n * 4) * 2 + align256((size_t)ncell * 4) + scan_ws(ncell);
+  return align256((size_t)n * 4) * 3 + align256((size_t)ncell * 4) + scan_ws(ncell);
 }
 
 extern "C" int dsph_grid_build(const dsph_domain* domain, const dsph_grid* grid, const float* pos, const float* h,
@@ -648,6 +613,8 @@ extern "C" int dsph_grid_build(const dsph_domain* domain, const dsph_grid* grid,
   w += align256((size_t)n * 4);
   int32_t* slot = reinterpret_cast<int32_t*>(w);
   w += align256((size_t)n * 4);
+  int32_t* order = reinterpret_cast<int32_t*>(w);
+  w += align256((size_t)n * 4);
   int32_t* count = reinterpret_cast<int32_t*>(w);
   w += align256((size_t)ncell * 4);
   void* scan_w = w;
@@ -664,10 +631,10 @@ extern "C" int dsph_grid_build(const dsph_domain* domain, const dsph_grid* grid,
   int s = scan_exclusive(count, ncell, cell_start, scan_w, scan_b, st);
   if (s != DSPH_OK) return s;
   if (n > 0) {
-    k_cell_scatter<<<grid_for(n), kBlock, 0, st>>>((int)n, keys, slot, cell_start, sort_index);
-    k_cell_sort<<<grid_for(ncell), kBlock, 0, st>>>((int)ncell, cell_start, sort_index);
-    k_sorted_gather<<<grid_for(n), kBlock, 0, st>>>((int)n, d, sort_index, reinterpret_cast<const float2*>(pos), h,
-                                                    reinterpret_cast<float2*>(sorted_pos), sorted_h, rank);
+    k_cell_scatter<<<grid_for(n), kBlock, 0, st>>>((int)n, keys, slot, cell_start, order);
+    k_cell_rank<<<grid_for(n), kBlock, 0, st>>>((int)n, d, keys, slot, cell_start, order,
+                                                reinterpret_cast<const float2*>(pos), h, sort_index,
+                                                reinterpret_cast<float2*>(sorted_pos), sorted_h, rank);
     DSPH_LAUNCH_CHECK();
   }
   return DSPH_OK;
