@@ -23,6 +23,7 @@
 // owner and those where it is the neighbor, using the neighbor's
 // cotangents.  No atomics; results do not depend on scheduling.
 #include "common.h"
+#include "near_math.h"
 #include "pmath.h"
 
 namespace dsph {
@@ -38,242 +39,89 @@ struct VjpConst {
   int diffusion;
 };
 
-// Pair geometry and derivatives for d = x_i - x_j (d != 0).
-struct PGeo {
-  float dx, dy, r, e, ex, ey, q, rr, w1, w1p, gx, gy;
+__device__ __forceinline__ float dot2(float2 a, float2 b) { return __builtin_fmaf(a.y, b.y, a.x * b.x); }
+__device__ __forceinline__ float2 axpy(float c, float2 x, float2 y) {
+  return make_float2(__builtin_fmaf(c, x.x, y.x), __builtin_fmaf(c, x.y, y.y));
+}
+
+// lambda_s_i = L_i^T lambda_g_i with lambda_g_k = sum_j (cD lc_k V_j -
+// cD lc_j V_k) gradW_kj, and g_i once more where L_i is not constant:
+// lambda_M_i = -L_i^T (lambda_g_i s_i^T) L_i^T = -lambda_s_i (L_i s_i)^T =
+// -lambda_s_i g_i^T (zero when the row has < 4 entries: M_i = I).  lsg[i] =
+// (lambda_s_i, g_i or 0).  One pass forms both sums (lambda_g and M): they
+// share the pair geometry, and neither is used elsewhere.  kLanes lanes per
+// row; the pseudo-inverse on one thread per row (see k_dsph_normalization_near).
+struct NbrGrad {
+  float2 x;
+  float m, r, lc;
 };
-
-__device__ __forceinline__ PGeo pgeo(float dx, float dy, float h) {
-  PGeo g;
-  g.dx = dx;
-  g.dy = dy;
-  g.r = sqrt_rn(dist2_exact(dx, dy));
-  g.e = g.r + 1e-7f;
-  // the forward kernels' reciprocal form (pair_geom)
-  const KConst k = kconst(h);
-  const float ri = 1.0f / g.e;
-  g.ex = dx * ri;
-  g.ey = dy * ri;
-  g.q = g.r * k.ih;
-  g.rr = g.q * h;
-  const float t = clamp01(1.0f - g.q);
-  g.w1 = wendland_dw(g.q, k);
-  // d w1 / dr = C/h^4 (-20) (1-q)^2 (1-4q)
-  g.w1p = g.q < 1.0f ? (((-20.0f * (t * t)) * (1.0f - 4.0f * g.q)) * kC2) / (((h * h) * h) * h) : 0.0f;
-  g.gx = g.ex * g.w1;
-  g.gy = g.ey * g.w1;
-  return g;
-}
-
-// The geometry of the mirrored pair (d -> -d): every quantity of pgeo is
-// either even in d (r, e, q, rr, w1, w1p: the squares, sums and kernel
-// values are the same floats) or odd and formed as d times an even one
-// (dx, dy, ex, ey, gx, gy: IEEE negation commutes with the products), so
-// this equals pgeo(-dx, -dy, h) bit for bit without its sqrt and division.
-__device__ __forceinline__ PGeo mirrored(const PGeo& g) {
-  PGeo m = g;
-  m.dx = -g.dx;
-  m.dy = -g.dy;
-  m.ex = -g.ex;
-  m.ey = -g.ey;
-  m.gx = -g.gx;
-  m.gy = -g.gy;
-  return m;
-}
-
-// J_xhat^T v (J_xhat is symmetric): v/e - d (d.v) / (r e^2)
-__device__ __forceinline__ float2 jxhat(const PGeo& g, float vx, float vy) {
-  const float dv = g.dx * vx + g.dy * vy;
-  const float c = dv / (g.r * g.e * g.e);
-  return make_float2(vx / g.e - g.dx * c, vy / g.e - g.dy * c);
-}
-
-// J_gradW^T v = w1 J_xhat^T v + (w1'/r)(xhat.v) d
-__device__ __forceinline__ float2 jgradw(const PGeo& g, float vx, float vy) {
-  const float2 a = jxhat(g, vx, vy);
-  const float c = (g.w1p / g.r) * (g.ex * vx + g.ey * vy);
-  return make_float2(g.w1 * a.x + c * g.dx, g.w1 * a.y + c * g.dy);
-}
-
-struct PairCot {
-  float lax, lay, lc;        // cotangents of dudt_i, drhodt_i
-  float lsx, lsy;            // of s_i
-  float m00, m01, m10, m11;  // of M_i
-};
-
-struct PairOut {
-  float gdx, gdy;      // dl/dd
-  float gui_x, gui_y;  // dl/du_i
-  float guj_x, guj_y;  // dl/du_j
-  float gri, grj;      // dl/drho_i, dl/drho_j
-};
-
-// All pair terms of row i with neighbor j (see the header).
-__device__ __forceinline__ PairOut pair_vjp(const PGeo& g, const VjpConst& K, float rho_i, float rho_j, float2 ui,
-                                            float2 uj, float m_j, float2 gi, float2 gj, const PairCot& c) {
-  PairOut o = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  const float Vj = m_j / rho_j;
-  const float lw = c.lax * g.gx + c.lay * g.gy;
-  const float r_inv = 1.0f / g.r;
-  // pressure
-  {
-    const float P = K.eos_c * (rho_i - K.rho0) + K.eos_c * (rho_j - K.rho0);
-    const float coef = -Vj * P / rho_i;
-    const float2 jl = jgradw(g, c.lax, c.lay);
-    o.gdx += coef * jl.x;
-    o.gdy += coef * jl.y;
-    o.gri += (Vj * P / (rho_i * rho_i)) * lw - (Vj * K.eos_c / rho_i) * lw;
-    o.grj += (Vj * P / (rho_i * rho_j)) * lw - (Vj * K.eos_c / rho_i) * lw;
-  }
-  // viscosity
-  if (K.visc >= 0) {
-    const float vx = ui.x - uj.x, vy = ui.y - uj.y;
-    const float den = g.rr + K.eps * (K.h * K.h);
-    const float vr = vx * g.ex + vy * g.ey;
-    if (!(K.pi_switch && !(vr < 0.0f))) {
-      const float pi = vr / den;
-      const float Kv = K.cV * Vj / rho_i;
-      const float t = Kv * pi * lw;
-      const float f = Kv * lw / den;
-      o.gui_x += f * g.ex;
-      o.gui_y += f * g.ey;
-      o.guj_x -= f * g.ex;
-      o.guj_y -= f * g.ey;
-      o.gri -= t / rho_i;
-      o.grj -= t / rho_j;
-      const float2 jv = jxhat(g, vx, vy);
-      const float2 jl = jgradw(g, c.lax, c.lay);
-      const float dpx = jv.x / den - (pi / den) * (g.dx * r_inv);
-      const float dpy = jv.y / den - (pi / den) * (g.dy * r_inv);
-      o.gdx += Kv * (lw * dpx + pi * jl.x);
-      o.gdy += Kv * (lw * dpy + pi * jl.y);
-    }
-  }
-  // continuity
-  {
-    const float dux = uj.x - ui.x, duy = uj.y - ui.y;
-    const float f = m_j * rho_i / rho_j;
-    const float t = -c.lc * f * (dux * g.gx + duy * g.gy);
-    o.guj_x += -c.lc * f * g.gx;
-    o.guj_y += -c.lc * f * g.gy;
-    o.gui_x += c.lc * f * g.gx;
-    o.gui_y += c.lc * f * g.gy;
-    o.gri += t / rho_i;
-    o.grj += -t / rho_j;
-    const float2 jd = jgradw(g, dux, duy);
-    o.gdx += -c.lc * f * jd.x;
-    o.gdy += -c.lc * f * jd.y;
-  }
-  // density diffusion (g_i, g_j held fixed here; their cotangent is gathered separately)
-  if (K.diffusion) {
-    const float den2 = g.rr + 1e-6f * K.h;
-    const float rt = 2.0f * (rho_j - rho_i) / den2;
-    const float xx = g.ex * g.ex + g.ey * g.ey;
-    const float xw = xx * g.w1;
-    const float Gx = gi.x + gj.x, Gy = gi.y + gj.y;
-    const float psiw = -rt * xw + (Gx * g.gx + Gy * g.gy);
-    const float a = c.lc * K.cD * Vj;
-    o.gri += a * (2.0f / den2) * xw;
-    o.grj += -a * (2.0f / den2) * xw - a * psiw / rho_j;
-    const float2 jx = jxhat(g, g.ex, g.ey);
-    const float dxw_x = 2.0f * g.w1 * jx.x + xx * g.w1p * (g.dx * r_inv);
-    const float dxw_y = 2.0f * g.w1 * jx.y + xx * g.w1p * (g.dy * r_inv);
-    const float drt = -rt / den2;  // times d/r
-    const float2 jG = jgradw(g, Gx, Gy);
-    o.gdx += a * (-(drt * (g.dx * r_inv)) * xw - rt * dxw_x + jG.x);
-    o.gdy += a * (-(drt * (g.dy * r_inv)) * xw - rt * dxw_y + jG.y);
-  }
-  // s_i = sum V_j (rho_i - rho_j) gradW
-  {
-    const float ls = c.lsx * g.gx + c.lsy * g.gy;
-    const float ts = Vj * (rho_i - rho_j) * ls;
-    o.gri += Vj * ls;
-    o.grj += -Vj * ls - ts / rho_j;
-    const float2 js = jgradw(g, c.lsx, c.lsy);
-    o.gdx += Vj * (rho_i - rho_j) * js.x;
-    o.gdy += Vj * (rho_i - rho_j) * js.y;
-  }
-  // M_i = sum V_j (-rr xhat) (x) gradW = -sum V_j rr w1 xhat xhat^T
-  {
-    const float a = g.ex * (c.m00 * g.ex + c.m01 * g.ey) + g.ey * (c.m10 * g.ex + c.m11 * g.ey);
-    const float tM = -Vj * g.rr * g.w1 * a;
-    o.grj += -tM / rho_j;
-    const float sx = (c.m00 + c.m00) * g.ex + (c.m01 + c.m10) * g.ey;
-    const float sy = (c.m10 + c.m01) * g.ex + (c.m11 + c.m11) * g.ey;
-    const float2 jm = jxhat(g, sx, sy);
-    const float b = a * (g.w1 + g.rr * g.w1p);
-    o.gdx += -Vj * (b * (g.dx * r_inv) + g.rr * g.w1 * jm.x);
-    o.gdy += -Vj * (b * (g.dy * r_inv) + g.rr * g.w1 * jm.y);
-  }
-  return o;
-}
-
-// lambda_g_k = sum_j (cD lc_k V_j - cD lc_j V_k) gradW_kj
-__global__ void __launch_bounds__(kBlock) k_vjp_lg(PairsDev P, VjpConst K, const float* __restrict__ mass,
-                                                   const float* __restrict__ rho, const float* __restrict__ lc,
-                                                   float2* __restrict__ lg) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= P.nq) return;
+template <int kLanes>
+__global__ void __launch_bounds__(kBlock) k_vjp_grad(PairsDev P, VjpConst K, const float* __restrict__ mass,
+                                                     const float* __restrict__ rho, const float* __restrict__ lc,
+                                                     const float2* __restrict__ grad_rho, float4* __restrict__ lsg) {
+  const int row = (int)((blockIdx.x * (unsigned)blockDim.x + threadIdx.x) / kLanes);
+  const bool valid = row < P.nq;
+  const int k = valid ? row : P.nq - 1;
   const float2 xk = P.qpos[k];
-  const float Vk = mass[k] / rho[k];
-  const float lck = lc[k];
-  float ax = 0.f, ay = 0.f;
-  const RowRef rr = row_ref(P, k);
-  for (int n = 0, e = rr.base; n < rr.cnt; ++n, e += rr.step) {
-    const int j = P.nbr[e];
-    if (j == k) continue;
-    const float2 xj = P.rpos[j];
-    const PGeo g = pgeo(mod_offset(xk.x - xj.x, P.dom, 0), mod_offset(xk.y - xj.y, P.dom, 1), K.h);
-    const float Vj = mass[j] / rho[j];
-    const float f = K.cD * lck * Vj - K.cD * lc[j] * Vk;
-    ax += f * g.gx;
-    ay += f * g.gy;
+  const float cVk = K.cD * (mass[k] / rho[k]), cLk = K.cD * lc[k];
+  const KConst kc = kconst(K.h);
+  RowRef rr = row_ref(P, k);
+  if (!valid) rr.cnt = 0;
+  constexpr int U = 4;
+  float acc[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  sum_row<kLanes, U>(
+      P.nbr, rr, k, acc, [&](int j) { return NbrGrad{P.rpos[j], mass[j], rho[j], lc[j]}; },
+      [&](const NbrGrad(&d)[U], float(&t)[U][6]) {
+        float dx[U], dy[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          dx[u] = xk.x - d[u].x.x;
+          dy[u] = xk.y - d[u].x.y;
+        }
+        wrap_offsets(dx, dy, P.dom);
+        auto put = [&](const Geom& g, float Vj, float lcj, float(&o)[6]) {
+          const float f = cLk * Vj - cVk * lcj;
+          o[0] = f * g.gx;
+          o[1] = f * g.gy;
+          const float s = -(g.q * g.h);
+          const float qx = s * g.ex, qy = s * g.ey;
+          const float kx = Vj * g.gx, ky = Vj * g.gy;
+          o[2] = qx * kx;
+          o[3] = qx * ky;
+          o[4] = qy * kx;
+          o[5] = qy * ky;
+        };
+        NearRange range;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const float ir = range.divisor(d[u].r);
+          range.operand(d[u].m);
+          put(pair_geom_near(dx[u], dy[u], K.h, kc, range), div_near(d[u].m, d[u].r, ir), d[u].lc, t[u]);
+        }
+        if (range.odd()) {
+#pragma unroll
+          for (int u = 0; u < U; ++u)
+            put(pair_geom(xk, d[u].x, K.h, kc, P.dom), d[u].m / d[u].r, d[u].lc, t[u]);
+        }
+      });
+  __shared__ float sums[7][kBlock / kLanes];
+  const int r = threadIdx.x / kLanes;
+  if ((threadIdx.x & (kLanes - 1)) == 0) {
+    for (int q = 0; q < 6; ++q) sums[q][r] = acc[q];
+    sums[6][r] = rr.cnt < 4 ? 1.f : 0.f;
   }
-  lg[k] = make_float2(ax, ay);
-}
-
-// lambda_s_i = L_i^T lambda_g_i, lambda_M_i = -L_i^T (lambda_g_i s_i^T) L_i^T
-// (zero when the row has < 4 entries: M_i = I).
-__global__ void __launch_bounds__(kBlock) k_vjp_lsm(PairsDev P, VjpConst K, const float* __restrict__ mass,
-                                                    const float* __restrict__ rho, const float2* __restrict__ lg,
-                                                    float2* __restrict__ ls, float4* __restrict__ lM) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= P.nq) return;
-  const float2 xi = P.qpos[i];
-  const float rho_i = rho[i];
-  float m00 = 0.f, m01 = 0.f, m10 = 0.f, m11 = 0.f, sx = 0.f, sy = 0.f;
-  const RowRef rr = row_ref(P, i);
-  for (int n = 0, e = rr.base; n < rr.cnt; ++n, e += rr.step) {
-    const int j = P.nbr[e];
-    const Geom g = pair_geom(xi, P.rpos[j], K.h, P.dom);
-    const float Vj = mass[j] / rho[j];
-    const float s = -(g.q * g.h);
-    const float qx = s * g.ex, qy = s * g.ey;
-    const float kx = Vj * g.gx, ky = Vj * g.gy;
-    m00 += qx * kx;
-    m01 += qx * ky;
-    m10 += qy * kx;
-    m11 += qy * ky;
-    const float d = rho_i - rho[j];
-    sx += d * kx;
-    sy += d * ky;
-  }
-  const float2 l = lg[i];
-  if (rr.cnt < 4) {
-    ls[i] = l;  // L = I
-    lM[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+  __syncthreads();
+  constexpr int rows = kBlock / kLanes;
+  const int t = threadIdx.x, i = blockIdx.x * rows + t;
+  if (t >= rows || i >= P.nq) return;
+  const float2 l = make_float2(sums[0][t], sums[1][t]);
+  if (sums[6][t] != 0.f) {
+    lsg[i] = make_float4(l.x, l.y, 0.f, 0.f);  // L = I
     return;
   }
-  const dsph_pm::Pinv2 L = dsph_pm::pinv2x2(m00, m01, m10, m11);
-  ls[i] = make_float2(L.l00 * l.x + L.l10 * l.y, L.l01 * l.x + L.l11 * l.y);
-  // A = lambda_g s^T ; lM = -L^T A L^T
-  const float a00 = l.x * sx, a01 = l.x * sy, a10 = l.y * sx, a11 = l.y * sy;
-  // B = L^T A
-  const float b00 = L.l00 * a00 + L.l10 * a10, b01 = L.l00 * a01 + L.l10 * a11;
-  const float b10 = L.l01 * a00 + L.l11 * a10, b11 = L.l01 * a01 + L.l11 * a11;
-  // C = B L^T
-  lM[i] = make_float4(-(b00 * L.l00 + b01 * L.l01), -(b00 * L.l10 + b01 * L.l11), -(b10 * L.l00 + b11 * L.l01),
-                      -(b10 * L.l10 + b11 * L.l11));
+  const dsph_pm::Pinv2 L = dsph_pm::pinv2x2(sums[2][t], sums[3][t], sums[4][t], sums[5][t]);
+  const float2 g = grad_rho[i];
+  lsg[i] = make_float4(L.l00 * l.x + L.l10 * l.y, L.l01 * l.x + L.l11 * l.y, g.x, g.y);
 }
 
 struct VjpArgs {
@@ -283,72 +131,178 @@ struct VjpArgs {
   const float2* grad_rho;
   const float2* la;
   const float* lc;
-  const float2* ls;
-  const float4* lM;
+  const float4* lsg;
   const float2* lx_in;  // cotangent of dx/dt (= u), added to lambda_u; may be NULL
   float2* out_x;
   float2* out_u;
   float* out_rho;
 };
 
+// The cotangents and state of one particle as the pair terms take them.
+struct Cot {
+  float2 x, u, g, la;
+  float4 lsg;
+  float r, m, lc;
+  int self;  // its index
+};
+
+// The geometry of a pair for d = x_k - x_j (d != 0).
+struct PGeo {
+  float2 d, e, G;              // offset, xhat, gradW
+  float rr, w1, w1p, ri, Ei;   // q h, dW/dr, its derivative, 1/r, 1/(r + 1e-7)
+};
+
+// Everything particle k gets from its pair with j: as the owner of row k and
+// as the neighbor in row j.  The mirrored pair has -d, -xhat, -gradW, -du and
+// the same r, W', pi, so with J = d xhat / d d (symmetric, even in d) and
+//   Y = V_j/rho_k la_k - V_k/rho_j la_j,        S = cV Y.gradW
+//   F = lc_k V_j rho_k + lc_j V_k rho_j,        A = cD (lc_k V_j - lc_j V_k)
+//   W = (pi cV - P) Y + F (u_k - u_j) + A (g_k + g_j)
+//       + (rho_k - rho_j)(V_j ls_k + V_k ls_j)
+//   T = V_j (ls_k (g_k.e) + g_k (ls_k.e)) + V_k (ls_j (g_j.e) + g_j (ls_j.e))
+// both rows' terms are one J product, J (w1 W + S/den (u_k - u_j) + rr w1 T),
+// and a multiple of d (J xhat = 1e-7 d / (r + 1e-7)^3).  The terms evaluated
+// one by one for both rows, each with its own quotients, took ten times the
+// instructions (262k particles: 493 us, now 82; with two passes for lambda_g
+// and M 626 us, now 130; 16k particles 223 us, now 31).
+__device__ __forceinline__ void pair_cotangent(const PGeo& g, const VjpConst& K, const Cot& k, float ik, float Vk,
+                                               const Cot& j, float ij, float (&t)[5]) {
+  const float Vj = j.m * ij;
+  const float2 v = make_float2(k.u.x - j.u.x, k.u.y - j.u.y);
+  const float2 lsk = make_float2(k.lsg.x, k.lsg.y), gmk = make_float2(k.lsg.z, k.lsg.w);
+  const float2 lsj = make_float2(j.lsg.x, j.lsg.y), gmj = make_float2(j.lsg.z, j.lsg.w);
+  const float ak = Vj * ik, aj = Vk * ij;
+  const float2 Y = make_float2(ak * k.la.x - aj * j.la.x, ak * k.la.y - aj * j.la.y);
+  const float YG = dot2(Y, g.G);
+  const float P = K.eos_c * (k.r - K.rho0) + K.eos_c * (j.r - K.rho0);
+  float pi = 0.f, S = 0.f, Sd = 0.f, Spi = 0.f;
+  if (K.visc >= 0) {
+    const float iden = rcp_near(g.rr + K.eps * (K.h * K.h));
+    const float vr = dot2(v, g.e);
+    const bool on = !K.pi_switch || vr < 0.0f;
+    pi = on ? vr * iden : 0.f;
+    S = on ? K.cV * YG : 0.f;
+    Sd = S * iden;
+    Spi = Sd * pi;
+  }
+  const float Fk = k.lc * Vj * k.r, Fj = j.lc * Vk * j.r, F = Fk + Fj;
+  const float a1 = K.cD * k.lc * Vj, a2 = K.cD * j.lc * Vk, A = a1 - a2;
+  const float i2 = rcp_near(g.rr + 1e-6f * K.h);
+  const float dr = k.r - j.r;
+  const float rt = -2.0f * dr * i2;
+  const float xx = dot2(g.e, g.e), xw = xx * g.w1;
+  const float2 Gs = make_float2(k.g.x + j.g.x, k.g.y + j.g.y);
+  const float psiw = __builtin_fmaf(-rt, xw, dot2(Gs, g.G));
+  const float eLk = dot2(g.e, lsk), eGk = dot2(g.e, gmk), eLj = dot2(g.e, lsj), eGj = dot2(g.e, gmj);
+  const float pk = Vj * eGk, qk = Vj * eLk, pj = Vk * eGj, qj = Vk * eLj;
+  const float rw = g.rr * g.w1;
+  const float aN = __builtin_fmaf(qk, eGk, qj * eGj);  // minus e.(V_j M_k + V_k M_j) e
+  float2 W = axpy(K.cV * pi - P, Y, make_float2(F * v.x, F * v.y));
+  W = axpy(A, Gs, W);
+  W = axpy(dr * Vj, lsk, W);
+  W = axpy(dr * Vk, lsj, W);
+  float2 T = axpy(pk, lsk, make_float2(qk * gmk.x, qk * gmk.y));
+  T = axpy(pj, lsj, T);
+  T = axpy(qj, gmj, T);
+  float2 X = axpy(g.w1, W, make_float2(Sd * v.x, Sd * v.y));
+  X = axpy(rw, T, X);
+  float D = __builtin_fmaf(g.w1p, dot2(g.e, W), -Spi);
+  const float Art = A * rt;
+  D = __builtin_fmaf(Art, __builtin_fmaf(i2, xw, -xx * g.w1p), D);
+  D = __builtin_fmaf(aN, __builtin_fmaf(g.rr, g.w1p, g.w1), D);
+  const float E2 = g.Ei * g.Ei;
+  const float c = g.ri * __builtin_fmaf(-E2, dot2(g.d, X), D) - 2e-7f * (Art * g.w1) * (E2 * g.Ei);
+  t[0] = __builtin_fmaf(c, g.d.x, X.x * g.Ei);
+  t[1] = __builtin_fmaf(c, g.d.y, X.y * g.Ei);
+  t[2] = __builtin_fmaf(F, g.G.x, Sd * g.e.x);
+  t[3] = __builtin_fmaf(F, g.G.y, Sd * g.e.y);
+  // the terms with a factor 1 / rho_k first
+  float q = __builtin_fmaf(P, YG, -pi * S);
+  q = __builtin_fmaf(Fk - Fj, dot2(v, g.G), q);
+  q = __builtin_fmaf(a2, psiw, q);
+  q = __builtin_fmaf(Vk * j.r, dot2(lsj, g.G), q);
+  q = __builtin_fmaf(-rw, qj * eGj, q);
+  float l = __builtin_fmaf(q, ik, -K.eos_c * YG);
+  l = __builtin_fmaf(2.0f * A * i2, xw, l);
+  t[4] = __builtin_fmaf(Vj, dot2(lsk, g.G), l);
+}
+
+template <int kLanes>
 __global__ void __launch_bounds__(kBlock) k_vjp_main(PairsDev P, VjpConst K, VjpArgs A) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= P.nq) return;
-  const float2 xk = P.qpos[k];
-  const float2 uk = A.vel[k];
-  const float rk = A.rho[k];
-  const float mk = A.mass[k];
-  const float2 gk = K.diffusion ? A.grad_rho[k] : make_float2(0.f, 0.f);
-  PairCot ck;
-  {
-    const float2 a = A.la[k];
-    const float2 s = A.ls[k];
-    const float4 m = A.lM[k];
-    ck = {a.x, a.y, A.lc[k], s.x, s.y, m.x, m.y, m.z, m.w};
-  }
-  float lxx = 0.f, lxy = 0.f, lux = 0.f, luy = 0.f, lr = 0.f;
-  const RowRef rr = row_ref(P, k);
-  for (int n = 0, e = rr.base; n < rr.cnt; ++n, e += rr.step) {
-    const int j = P.nbr[e];
-    if (j == k) continue;
-    const float2 xj = P.rpos[j];
-    const float dx = mod_offset(xk.x - xj.x, P.dom, 0), dy = mod_offset(xk.y - xj.y, P.dom, 1);
-    const float2 uj = A.vel[j];
-    const float rj = A.rho[j];
-    const float mj = A.mass[j];
-    const float2 gj = K.diffusion ? A.grad_rho[j] : make_float2(0.f, 0.f);
-    // k as the row owner of pair (k, j)
-    const PGeo g1 = pgeo(dx, dy, K.h);
-    const PairOut o1 = pair_vjp(g1, K, rk, rj, uk, uj, mj, gk, gj, ck);
-    lxx += o1.gdx;
-    lxy += o1.gdy;
-    lux += o1.gui_x;
-    luy += o1.gui_y;
-    lr += o1.gri;
-    // k as the neighbor in pair (j, k): d_jk = -d_kj
-    PairCot cj;
-    {
-      const float2 a = A.la[j];
-      const float2 s = A.ls[j];
-      const float4 m = A.lM[j];
-      cj = {a.x, a.y, A.lc[j], s.x, s.y, m.x, m.y, m.z, m.w};
+  const int row = (int)((blockIdx.x * (unsigned)blockDim.x + threadIdx.x) / kLanes);
+  const bool valid = row < P.nq;
+  const int k = valid ? row : P.nq - 1;
+  auto load = [&](int j) {
+    Cot c;
+    c.x = P.rpos[j];
+    c.u = A.vel[j];
+    c.g = K.diffusion ? A.grad_rho[j] : make_float2(0.f, 0.f);
+    c.la = A.la[j];
+    c.lsg = A.lsg[j];
+    c.r = A.rho[j];
+    c.m = A.mass[j];
+    c.lc = A.lc[j];
+    c.self = j;
+    return c;
+  };
+  Cot ck = load(k);
+  ck.x = P.qpos[k];
+  const float ik = 1.0f / ck.r, Vk = ck.m / ck.r;
+  const KConst kc = kconst(K.h);
+  const float cp = kC2 / (((K.h * K.h) * K.h) * K.h);
+  RowRef rr = row_ref(P, k);
+  if (!valid) rr.cnt = 0;
+  constexpr int U = 2;
+  float acc[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
+  sum_row<kLanes, U>(P.nbr, rr, k, acc, load, [&](const Cot(&d)[U], float(&t)[U][5]) {
+    float dx[U], dy[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      dx[u] = ck.x.x - d[u].x.x;
+      dy[u] = ck.x.y - d[u].x.y;
     }
-    const PGeo g2 = mirrored(g1);
-    const PairOut o2 = pair_vjp(g2, K, rj, rk, uj, uk, mk, gj, gk, cj);
-    lxx -= o2.gdx;
-    lxy -= o2.gdy;
-    lux += o2.guj_x;
-    luy += o2.guj_y;
-    lr += o2.grj;
-  }
+    wrap_offsets(dx, dy, P.dom);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      NearRange range;
+      PGeo g;
+      g.d = make_float2(dx[u], dy[u]);
+      const float d2 = dist2_exact(dx[u], dy[u]);
+      range.d2(d2);
+      float r = sqrt_near(d2), ij = range.divisor(d[u].r);
+      if (range.odd()) {
+        r = sqrt_rn(d2);
+        ij = 1.0f / d[u].r;
+      }
+      g.Ei = rcp_near(r + 1e-7f);
+      g.ri = rcp_near(r);
+      g.e = make_float2(dx[u] * g.Ei, dy[u] * g.Ei);
+      const float q = r * kc.ih;
+      g.rr = q * K.h;
+      const float s = clamp01(1.0f - q);
+      g.w1 = wendland_dw(q, kc);
+      // d w1 / dr = C/h^4 (-20) (1-q)^2 (1-4q)
+      g.w1p = q < 1.0f ? ((-20.0f * (s * s)) * (1.0f - 4.0f * q)) * cp : 0.0f;
+      g.G = make_float2(g.e.x * g.w1, g.e.y * g.w1);
+      pair_cotangent(g, K, ck, ik, Vk, d[u], ij, t[u]);
+      // the particle itself (and the padding of its row) has no pair; r = 0
+      // between distinct particles stays NaN, as the gradient is
+      const bool self = d[u].self == k;
+      if (self) {
+#pragma unroll
+        for (int c = 0; c < 5; ++c) t[u][c] = 0.f;
+      }
+    }
+  });
+  if (!valid || (threadIdx.x & (kLanes - 1)) != 0) return;
   if (A.lx_in) {
     const float2 t = A.lx_in[k];
-    lux += t.x;
-    luy += t.y;
+    acc[2] += t.x;
+    acc[3] += t.y;
   }
-  A.out_x[k] = make_float2(lxx, lxy);
-  A.out_u[k] = make_float2(lux, luy);
-  A.out_rho[k] = lr;
+  A.out_x[k] = make_float2(acc[0], acc[1]);
+  A.out_u[k] = make_float2(acc[2], acc[3]);
+  A.out_rho[k] = acc[4];
 }
 
 }  // namespace dsph
@@ -356,7 +310,7 @@ __global__ void __launch_bounds__(kBlock) k_vjp_main(PairsDev P, VjpConst K, Vjp
 using namespace dsph;
 
 extern "C" size_t dsph_deltasph_vjp_workspace(int64_t n) {
-  return ((size_t)n * (2 + 2 + 4) * sizeof(float) + 255) / 256 * 256 + 256;
+  return ((size_t)n * 4 * sizeof(float) + 255) / 256 * 256 + 256;
 }
 
 extern "C" int dsph_deltasph_rhs_vjp(const dsph_pairs* pairs, const dsph_deltasph_params* prm, const float* vel,
@@ -391,15 +345,18 @@ extern "C" int dsph_deltasph_rhs_vjp(const dsph_pairs* pairs, const dsph_deltasp
   K.pi_switch = prm->pi_switch;
   K.diffusion = prm->diffusion;
   char* w = static_cast<char*>(ws);
-  float2* lg = reinterpret_cast<float2*>(w);
-  float2* ls = lg + n;
-  float4* lM = reinterpret_cast<float4*>(ls + n);
-  const int nb = grid_for(n);
+  float4* lsg = reinterpret_cast<float4*>(w);
+  // lanes per row, as the forward passes choose them
+  const int lanes = n <= (1 << 14) ? 16 : (n <= (1 << 17) ? 4 : 1);
+  const int grad_lanes = n <= (1 << 13) ? 16 : (n <= (1 << 17) ? 4 : 1);
   if (prm->diffusion) {
-    k_vjp_lg<<<nb, kBlock, 0, st>>>(P, K, mass, rho, cot_drhodt, lg);
-    k_vjp_lsm<<<nb, kBlock, 0, st>>>(P, K, mass, rho, lg, ls, lM);
+    auto go = [&](auto kernel) {
+      kernel<<<grid_for(n, kBlock / grad_lanes), kBlock, 0, st>>>(P, K, mass, rho, cot_drhodt,
+                                                                  reinterpret_cast<const float2*>(grad_rho), lsg);
+    };
+    grad_lanes == 16 ? go(k_vjp_grad<16>) : (grad_lanes == 4 ? go(k_vjp_grad<4>) : go(k_vjp_grad<1>));
   } else {
-    DSPH_CHECK_HIP(hipMemsetAsync(ls, 0, sizeof(float) * 6 * n, st));
+    DSPH_CHECK_HIP(hipMemsetAsync(lsg, 0, sizeof(float4) * n, st));
   }
   VjpArgs A;
   A.vel = reinterpret_cast<const float2*>(vel);
@@ -408,12 +365,12 @@ extern "C" int dsph_deltasph_rhs_vjp(const dsph_pairs* pairs, const dsph_deltasp
   A.grad_rho = reinterpret_cast<const float2*>(grad_rho);
   A.la = reinterpret_cast<const float2*>(cot_dudt);
   A.lc = cot_drhodt;
-  A.ls = ls;
-  A.lM = lM;
+  A.lsg = lsg;
   A.lx_in = reinterpret_cast<const float2*>(cot_dxdt);
   A.out_x = reinterpret_cast<float2*>(grad_pos);
   A.out_u = reinterpret_cast<float2*>(grad_vel);
   A.out_rho = grad_rho_out;
-  k_vjp_main<<<nb, kBlock, 0, st>>>(P, K, A);
+  auto go = [&](auto kernel) { kernel<<<grid_for(n, kBlock / lanes), kBlock, 0, st>>>(P, K, A); };
+  lanes == 16 ? go(k_vjp_main<16>) : (lanes == 4 ? go(k_vjp_main<4>) : go(k_vjp_main<1>));
   return launch_status();
 }

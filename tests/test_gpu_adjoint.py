@@ -26,12 +26,9 @@ def _oprm(cfg):
                            visc_coeff=cfg.nu if cfg.viscosity == "deltaSPH_viscid" else cfg.alpha, eps=cfg.eps)
 
 
-@pytest.mark.parametrize("what", ["x", "u", "rho", "all"])
-@pytest.mark.parametrize("visc", ["deltaSPH_viscid", "deltaSPH_inviscid"])
-def test_rhs_vjp_matches_float64_finite_differences(what, visc):
-    print(f"case {what} {visc}", flush=True)
+def _check_vjp(ns, what, visc):
+    print(f"case {ns} {what} {visc}", flush=True)
     rng = np.random.default_rng(11)
-    ns = 32
     pos, dx = sampling.sample_regular(ns)
     pos = sampling.jitter(pos, dx, 0.3, 11)
     n = pos.shape[0]
@@ -68,6 +65,19 @@ def test_rhs_vjp_matches_float64_finite_differences(what, visc):
     print(f"<lambda, J v>: finite differences {fd:.8e} adjoint {adj:.8e} rel {abs(adj - fd) / abs(fd):.2e}",
           flush=True)
     assert abs(adj - fd) <= 2e-4 * abs(fd)
+
+
+@pytest.mark.parametrize("what", ["x", "u", "rho", "all"])
+@pytest.mark.parametrize("visc", ["deltaSPH_viscid", "deltaSPH_inviscid"])
+def test_rhs_vjp_matches_float64_finite_differences(what, visc):
+    _check_vjp(32, what, visc)
+
+
+# the passes' 16, 4 and 1 lanes per row change at 8192, 16384 and 131072 rows
+# (the bound of the small case: float32 sums, measured 3e-6)
+@pytest.mark.parametrize("ns", [91, 131, 363])
+def test_rhs_vjp_lanes_match_float64_finite_differences(ns):
+    _check_vjp(ns, "all", "deltaSPH_viscid")
 
 
 def test_rollout_gradient_matches_reference_autograd():
