@@ -35,6 +35,15 @@ def test_scan_matches_numpy(n):
     assert np.array_equal(out.astype(np.int64), ref) and tot == ref[-1]
 
 
+# the one-workgroup form: per-thread counts 1 to 16 and its last size
+@pytest.mark.parametrize("n", [1023, 1025, 4097, 8191, 16384, 16385])
+def test_scan_one_workgroup_matches_numpy(n):
+    c = np.random.default_rng(n).integers(0, 200, n).astype(np.int64)
+    out, tot = _scan(c)
+    ref = np.concatenate([[0], np.cumsum(c)])
+    assert np.array_equal(out.astype(np.int64), ref) and tot == ref[-1]
+
+
 def test_scan_total_at_int32_max_is_accepted():
     c = np.array([2 ** 30, 2 ** 30 - 1], np.int64)
     out, tot = _scan(c)
