@@ -70,7 +70,7 @@ __global__ void __launch_bounds__(kBlock) k_vjp_grad(PairsDev P, VjpConst K, con
   constexpr int U = 4;
   float acc[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   sum_row<kLanes, U>(
-      P.nbr, rr, k, acc, [&](int j) { return NbrGrad{P.rpos[j], mass[j], rho[j], lc[j]}; },
+      P.nbr, rr, k, acc, [&](int j, int) { return NbrGrad{P.rpos[j], mass[j], rho[j], lc[j]}; },
       [&](const NbrGrad(&d)[U], float(&t)[U][6]) {
         float dx[U], dy[U];
 #pragma unroll
@@ -232,7 +232,7 @@ __global__ void __launch_bounds__(kBlock) k_vjp_main(PairsDev P, VjpConst K, Vjp
   const int row = (int)((blockIdx.x * (unsigned)blockDim.x + threadIdx.x) / kLanes);
   const bool valid = row < P.nq;
   const int k = valid ? row : P.nq - 1;
-  auto load = [&](int j) {
+  auto load = [&](int j, int) {
     Cot c;
     c.x = P.rpos[j];
     c.u = A.vel[j];
@@ -245,7 +245,7 @@ __global__ void __launch_bounds__(kBlock) k_vjp_main(PairsDev P, VjpConst K, Vjp
     c.self = j;
     return c;
   };
-  Cot ck = load(k);
+  Cot ck = load(k, -1);
   ck.x = P.qpos[k];
   const float ik = 1.0f / ck.r, Vk = ck.m / ck.r;
   const KConst kc = kconst(K.h);

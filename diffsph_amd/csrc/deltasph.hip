@@ -203,7 +203,7 @@ __global__ void __launch_bounds__(kBlock) k_dsph_normalization_near(PairsDev P, 
   RowRef rr = row_ref(P, i);
   if (!valid) rr.cnt = 0;
   const float rho_i = rho[i];
-  auto ld = [&](int j) {
+  auto ld = [&](int j, int) {
     NbrXMR d;
     d.x = P.rpos[j];
     d.m = kVol ? vol[j] : mass[j];
@@ -249,7 +249,7 @@ __global__ void __launch_bounds__(kBlock) k_dsph_normalization_near(PairsDev P, 
     // lanes past the row's end repeat its first entry (a row without entries takes no turn)
     const int pad = br.cnt > 0 ? B.P.nbr[br.base] : 0;
     sum_row<kLanes, 1>(
-        B.P.nbr, br, pad, b, [&](int j) { return j; }, [&](const int(&j)[1], float(&t)[1][6]) {
+        B.P.nbr, br, pad, b, [&](int j, int) { return j; }, [&](const int(&j)[1], float(&t)[1][6]) {
           if (br.cnt > 0) {
             const Geom g = pair_geom(xi, B.P.rpos[j[0]], pick_h(B.P.mode, h, h_of(B.P.rh, j[0], B.P.h0)), B.P.dom);
             put(g, B.mass[j[0]] / B.rho[j[0]], B.rho[j[0]], t[0]);
@@ -485,7 +485,7 @@ __global__ void __launch_bounds__(kBlock) k_dsph_rhs_near(PairsDev P, BoundaryDe
   const float eps_d = 1e-6f * h, eps_v = A.eps * (h * h);
   RowRef rr = row_ref(P, i);
   if (!valid) rr.cnt = 0;
-  auto ld = [&](int j) {
+  auto ld = [&](int j, int) {
     NbrRhs d;
     d.x = P.rpos[j];
     d.u = A.vel[j];
@@ -565,7 +565,7 @@ __global__ void __launch_bounds__(kBlock) k_dsph_rhs_near(PairsDev P, BoundaryDe
     float b[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
     const int pad = br.cnt > 0 ? B.P.nbr[br.base] : 0;
     sum_row<kLanes, 1>(
-        B.P.nbr, br, pad, b, [&](int j) { return j; }, [&](const int(&j)[1], float(&t)[1][5]) {
+        B.P.nbr, br, pad, b, [&](int j, int) { return j; }, [&](const int(&j)[1], float(&t)[1][5]) {
           for (int k = 0; k < 5; ++k) t[0][k] = 0.f;
           if (br.cnt > 0) wall_terms(B, A, xi, ui, h, rho_i, p_i, j[0], t[0]);
         });

@@ -24,6 +24,7 @@
 // queue several iterations ahead and synchronise only once per chunk.
 
 #include "common.h"
+#include "near_math.h"
 
 namespace dsph {
 
@@ -1056,17 +1057,116 @@ __global__ void __launch_bounds__(kBlock) k_ws_ring(PairsDev P, const float* __r
   for (int c = 8; c < 11; ++c) o[c] = c < nfeat ? (t[c - 8] - mean[c]) * istd[c] : 0.0f;
 }
 
-// Sweep launches: over neighbor tiles when the list carries them and the
-// sweep gathers records.
+// Small domains: the sweeps over records with several lanes per row (sum_row:
+// the row's order), because one thread per row is a chain of ~13 dependent
+// groups on too few waves (2304 rows: 9 workgroups, 18.5 us a sweep).
+struct NbrRec {
+  float4 r;
+  float s;
+};
+
+template <int kLanes, class Rec, class Term, int K>
+__device__ __forceinline__ void sweep_row_lanes(const PairsDev& P, const float* __restrict__ kv, const RowRef& rr,
+                                                int i, const Rec& rec, float (&acc)[K], const Term& term) {
+  const float2 xi = P.qpos[i];
+  sum_row<kLanes, 4>(
+      P.nbr, rr, i, acc, [&](int j, int at) { return NbrRec{rec[j], at >= 0 ? kv[at] : 0.f}; },
+      [&](const NbrRec(&d)[4], float(&t)[4][K]) {
+        float dx[4], dy[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          dx[u] = xi.x - d[u].r.x;
+          dy[u] = xi.y - d[u].r.y;
+        }
+        wrap_offsets(dx, dy, P.dom);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) term(d[u].r, dx[u] * d[u].s, dy[u] * d[u].s, t[u]);
+      });
+}
+
+template <int kLanes>
+__global__ void __launch_bounds__(kBlock) k_dfsph_sweep_a_lanes(PairsDev P, SweepAArgs A, const SolveCtrl* ctrl) {
+  if (ctrl && ctrl->done) return;
+  const int row = (int)((blockIdx.x * (unsigned)kBlock + threadIdx.x) / kLanes);
+  const bool valid = row < P.nq;
+  const int i = valid ? row : P.nq - 1;
+  RowRef rr = row_ref(P, i);
+  if (!valid) rr.cnt = 0;
+  const float4 own = A.xp[i];
+  const float pi = own.z, sj = A.diff ? -1.0f : 1.0f;
+  float acc[2] = {0.f, 0.f};
+  sweep_row_lanes<kLanes>(P, A.kv, rr, i, A.xp, acc, [&](const float4& r, float cx, float cy, float(&t)[2]) {
+    const float s = pi + sj * r.z;
+    t[0] = s * cx;
+    t[1] = s * cy;
+  });
+  if (!valid || (threadIdx.x & (kLanes - 1)) != 0) return;
+  const float r = A.rho[i];
+  const float2 a = make_float2(-acc[0] / r, -acc[1] / r);
+  if (A.xa)
+    A.xa[i] = make_float4(own.x, own.y, a.x, a.y);
+  else
+    A.acc[i] = a;
+}
+
+// 1024 threads keep the 256 rows, and so the partial sum's tree, of the other
+// sweeps' workgroups.
+constexpr int kSweepBLanes = 4;
+__global__ void __launch_bounds__(kBlock* kSweepBLanes) k_dfsph_sweep_b_lanes(PairsDev P, SweepBArgs B) {
+  __shared__ double errs[kBlock];
+  __shared__ double sh[kBlock / 64];
+  if (B.ctrl && B.ctrl->done) return;
+  const int row = blockIdx.x * kBlock + threadIdx.x / kSweepBLanes;
+  const bool valid = row < P.nq;
+  const int i = valid ? row : P.nq - 1;
+  RowRef rr = row_ref(P, i);
+  if (!valid) rr.cnt = 0;
+  const float4 own = B.xa[i];
+  const float2 ai = make_float2(own.z, own.w);
+  float acc[1] = {0.f};
+  sweep_row_lanes<kSweepBLanes>(P, B.kv, rr, i, B.xa, acc, [&](const float4& r, float cx, float cy, float(&t)[1]) {
+    t[0] = (r.z - ai.x) * cx + (r.w - ai.y) * cy;
+  });
+  if ((threadIdx.x & (kSweepBLanes - 1)) == 0)
+    errs[threadIdx.x / kSweepBLanes] = valid ? sweep_b_finish(B, i, acc[0], make_float2(own.x, own.y)) : 0.0;
+  __syncthreads();
+  // block_sum_d over the 256 rows
+  const int wid = threadIdx.x >> 6;
+  if (threadIdx.x < kBlock) {
+    const double v = wave_sum_d(errs[threadIdx.x]);
+    if ((threadIdx.x & 63) == 0) sh[wid] = v;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double t = 0.0;
+    for (int w = 0; w < kBlock / 64; ++w) t += sh[w];
+    B.partials[blockIdx.x] = t;
+  }
+}
+
+// Rows up to which the lanes forms are the faster ones.  A + B in us, lanes
+// against tiles: 2.3k rows 4.8 + 11.0 / 16.4 + 16.5, 8.1k 5.9 + 11.4 / 16.4 +
+// 16.7, 33k 8.8 + 11.2 / 16.4 + 16.7, 131k 15.2 + 15.8 / 20.6 + 21.1; A with
+// 16 lanes against 4: 16k 7.6 / 7.4, 33k 12.0 / 8.8.
+constexpr int kSweepA16 = 1 << 13, kSweepLanes = 1 << 17;
+
+// Sweep launches: lanes per row for few rows, else over neighbor tiles when
+// the list carries them and the sweep gathers records.
 static void launch_sweep_a(const PairsDev& P, const SweepAArgs& A, const SolveCtrl* ctrl, int nb, hipStream_t st) {
-  if (P.tslot && A.kv && A.xp)
+  if (A.kv && A.xp && P.nq <= kSweepA16)
+    k_dfsph_sweep_a_lanes<16><<<grid_for(P.nq, kBlock / 16), kBlock, 0, st>>>(P, A, ctrl);
+  else if (A.kv && A.xp && P.nq <= kSweepLanes)
+    k_dfsph_sweep_a_lanes<4><<<grid_for(P.nq, kBlock / 4), kBlock, 0, st>>>(P, A, ctrl);
+  else if (P.tslot && A.kv && A.xp)
     k_dfsph_sweep_a_tiled<<<nb, kBlock, (size_t)P.tcap * sizeof(float4), st>>>(P, A, ctrl);
   else
     k_dfsph_sweep_a<<<nb, kBlock, 0, st>>>(P, A.kv, A.vol, A.rho, A.p, A.acc, ctrl, A.diff, A.xp, A.xa);
 }
 
 static void launch_sweep_b(const PairsDev& P, const SweepBArgs& B, int nb, hipStream_t st) {
-  if (P.tslot && B.kv && B.xa)
+  if (B.kv && B.xa && P.nq <= kSweepLanes)
+    k_dfsph_sweep_b_lanes<<<nb, kBlock * kSweepBLanes, 0, st>>>(P, B);
+  else if (P.tslot && B.kv && B.xa)
     k_dfsph_sweep_b_tiled<<<nb, kBlock, (size_t)P.tcap * sizeof(float4), st>>>(P, B);
   else
     k_dfsph_sweep_b<<<nb, kBlock, 0, st>>>(P, B);

@@ -130,8 +130,8 @@ __device__ __forceinline__ void add_lanes(float (&acc)[K], const float (&t)[K]) 
 // consecutive lanes of a wave: lane g evaluates the entries n0 + g, then all
 // lanes add the L terms one after the other (a DPP operand of the add), so
 // the sum is that of one thread.  terms(d, t) fills t[u] for U entries with
-// data d[u] = load(entry); entries past the row's end load `self` and
-// count as zero (no sum is -0, so adding +0 keeps its bits).  All lanes of the
+// data d[u] = load(neighbor, list position); entries past the row's end load `self`
+// (position -1) and count as zero (no sum is -0, so adding +0 keeps its bits).  All lanes of the
 // wave call it.
 template <int L, int U, int K, class Load, class Terms>
 __device__ __forceinline__ void sum_row(const int32_t* __restrict__ nbr, const RowRef& rr, int self, float (&acc)[K],
@@ -139,19 +139,20 @@ __device__ __forceinline__ void sum_row(const int32_t* __restrict__ nbr, const R
   const int g = L == 1 ? 0 : (int)(threadIdx.x & (L - 1));
   // the next group's entries are read ahead of the current group's work: the
   // list streams from HBM and a group's data loads wait for its entries
-  int j[U];
+  int j[U], at[U];
   auto entries = [&](int n0) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int n = n0 + u * L + g;
-      j[u] = n < rr.cnt ? __builtin_nontemporal_load(nbr + rr.base + n * rr.step) : self;
+      at[u] = n < rr.cnt ? rr.base + n * rr.step : -1;
+      j[u] = n < rr.cnt ? __builtin_nontemporal_load(nbr + at[u]) : self;
     }
   };
   entries(0);
   for (int n0 = 0; __builtin_amdgcn_ballot_w64(n0 < rr.cnt); n0 += U * L) {
-    decltype(load(0)) d[U];
+    decltype(load(0, 0)) d[U];
 #pragma unroll
-    for (int u = 0; u < U; ++u) d[u] = load(j[u]);
+    for (int u = 0; u < U; ++u) d[u] = load(j[u], at[u]);
     entries(n0 + U * L);
     float t[U][K];
     terms(d, t);
