@@ -10,6 +10,7 @@
 // list order.  A quantity is either per particle (the reference's (q_i, q_j)
 // tuple: qa indexed by i, qb by j) or per pair (a single tensor).
 #include "common.h"
+#include "near_math.h"
 
 namespace dsph {
 
@@ -70,31 +71,40 @@ __device__ __forceinline__ void pp_q(const PpArgs& a, int i, int64_t j, int64_t 
   (void)c;
 }
 
-__global__ void __launch_bounds__(kBlock) k_pp_operation(PpArgs a) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= a.n) return;
-  float acc[8];
+// Sixteen lanes per row: a row's pairs are consecutive, so the lanes read
+// whole lines (one thread per row read 64 rows ~200 B apart and missed on
+// every array), and the terms are added in pair order (add_lanes).  kOut:
+// outputs per row, rounded up.  5.1M pairs: 147 -> 25 to 33 us an
+// operation.
+constexpr int kPpLanes = 16;
+template <int kOut>
+__global__ void __launch_bounds__(kBlock) k_pp_operation(PpArgs a, int ow) {
+  const int row = (int)((blockIdx.x * (unsigned)kBlock + threadIdx.x) / kPpLanes);
+  const bool valid = row < a.n;
+  const int i = valid ? row : a.n - 1;
+  const int g = threadIdx.x & (kPpLanes - 1);
+  float acc[kOut];
 #pragma unroll
-  for (int t = 0; t < 8; ++t) acc[t] = 0.0f;
+  for (int t = 0; t < kOut; ++t) acc[t] = 0.0f;
   int64_t b = a.off[i], e = a.off[i + 1];
   if (b < 0) b = 0;
   if (e > a.np) e = a.np;
+  if (!valid) e = b;
   const float rho_i = a.ra ? a.ra[i] : 1.0f;
   const bool sym = a.mode == PM_SYMMETRIC;
   const float inv_ri2 = sym ? 1.0f / (rho_i * rho_i) : 0.0f;
-  for (int64_t k = b; k < e; ++k) {
-    const int64_t j = a.j[k];
-    if (j < 0 || j >= a.nb) continue;
+  // v[t]: the pair's term of output t
+  auto terms = [&](int64_t k, int64_t j, float(&v)[8]) {
     float q[4] = {0.f, 0.f, 0.f, 0.f};
     switch (a.op) {
       case PP_DENSITY: {
-        acc[0] += a.mb[j] * a.W[k];
+        v[0] = a.mb[j] * a.W[k];
         break;
       }
       case PP_INTERPOLATE: {
         const float kk = a.mb[j] / a.rb[j] * a.W[k];
         for (int t = 0; t < a.qw; ++t) q[t] = a.qp ? a.qp[k * a.qw + t] : a.qb[j * a.qw + t];
-        for (int t = 0; t < a.qw; ++t) acc[t] += q[t] * kk;
+        for (int t = 0; t < a.qw; ++t) v[t] = q[t] * kk;
         break;
       }
       case PP_GRADIENT:
@@ -118,21 +128,21 @@ __global__ void __launch_bounds__(kBlock) k_pp_operation(PpArgs a) {
         }
         if (a.op == PP_GRADIENT) {
           for (int t = 0; t < a.qw; ++t) {
-            acc[2 * t] += q[t] * kx;
-            acc[2 * t + 1] += q[t] * ky;
+            v[2 * t] = q[t] * kx;
+            v[2 * t + 1] = q[t] * ky;
           }
         } else if (a.op == PP_CURL) {
-          acc[0] += q[1] * kx - q[0] * ky;
+          v[0] = q[1] * kx - q[0] * ky;
         } else if (a.qw == 2) {
-          acc[0] += q[0] * kx + q[1] * ky;
+          v[0] = q[0] * kx + q[1] * ky;
         } else {
           // a 2x2 tensor field: 'div' contracts the last axis, 'dot' the first
           if (!a.dot) {
-            acc[0] += q[0] * kx + q[1] * ky;
-            acc[1] += q[2] * kx + q[3] * ky;
+            v[0] = q[0] * kx + q[1] * ky;
+            v[1] = q[2] * kx + q[3] * ky;
           } else {
-            acc[0] += q[0] * kx + q[2] * ky;
-            acc[1] += q[1] * kx + q[3] * ky;
+            v[0] = q[0] * kx + q[2] * ky;
+            v[1] = q[1] * kx + q[3] * ky;
           }
         }
         break;
@@ -144,7 +154,7 @@ __global__ void __launch_bounds__(kBlock) k_pp_operation(PpArgs a) {
           A[t] = a.qp ? a.qp[k * a.qw + t] : a.qa[(int64_t)i * a.qw + t] - a.qb[j * a.qw + t];
         if (a.mode == PM_NAIVE) {
           const float lk = -V * a.lap[k];
-          for (int t = 0; t < a.qw; ++t) acc[t] += lk * A[t];
+          for (int t = 0; t < a.qw; ++t) v[t] = lk * A[t];
           break;
         }
         const float h = a.hij[k];
@@ -153,39 +163,61 @@ __global__ void __launch_bounds__(kBlock) k_pp_operation(PpArgs a) {
         const float gx = a.gW[2 * k], gy = a.gW[2 * k + 1];
         const float kA = (gx * -ex + gy * -ey) / quot;
         if (a.qw == 1) {
-          acc[0] += -A[0] * V * 2.0f * kA;
+          v[0] = -A[0] * V * 2.0f * kA;
         } else if (a.mode == PM_CONSERVING) {
           const float qq = V * kA * (A[0] * ex + A[1] * ey);
-          acc[0] += -qq * ex;
-          acc[1] += -qq * ey;
+          v[0] = -qq * ex;
+          v[1] = -qq * ey;
         } else if (a.mode == PM_DIVFREE) {
           const float dd = (A[0] * ex + A[1] * ey) / quot;
           const float qq = 2.0f * 4.0f * V * dd;  // 2 (d + 2), d = 2
-          acc[0] += qq * gx;
-          acc[1] += qq * gy;
+          v[0] = qq * gx;
+          v[1] = qq * gy;
         } else if (a.mode == PM_DOT) {
           const float s = -4.0f * (A[0] * ex + A[1] * ey);  // -(d + 2) (A . x)
           const float f = V * kA;
-          acc[0] += (s * ex - A[0]) * f;
-          acc[1] += (s * ey - A[1]) * f;
+          v[0] = (s * ex - A[0]) * f;
+          v[1] = (s * ey - A[1]) * f;
         } else {
           const float qq = -2.0f * V * kA;
-          acc[0] += A[0] * qq;
-          acc[1] += A[1] * qq;
+          v[0] = A[0] * qq;
+          v[1] = A[1] * qq;
         }
         break;
       }
       default:
         break;
     }
+  };
+  for (int64_t k0 = b; __builtin_amdgcn_ballot_w64(k0 < e); k0 += kPpLanes) {
+    const int64_t k = k0 + g;
+    float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    if (k < e) {
+      const int64_t j = a.j[k];
+      if (j >= 0 && j < a.nb) terms(k, j, v);
+    }
+    float t[kOut];
+#pragma unroll
+    for (int c = 0; c < kOut; ++c) t[c] = v[c];
+    add_lanes<kPpLanes, kOut>(acc, t);
   }
+  if (!valid || g != 0) return;
+  const float scale = (sym && a.op != PP_DENSITY && a.op != PP_INTERPOLATE && a.op != PP_LAPLACIAN) ? rho_i : 1.0f;
+#pragma unroll
+  for (int t = 0; t < kOut; ++t)
+    if (t < ow) a.out[(int64_t)i * ow + t] = sym ? scale * acc[t] : acc[t];
+}
+
+static int launch_pp_operation(const PpArgs& a, hipStream_t st) {
   int ow = 1;
   if (a.op == PP_INTERPOLATE) ow = a.qw;
   else if (a.op == PP_GRADIENT) ow = 2 * a.qw;
   else if (a.op == PP_DIVERGENCE || a.op == PP_DIVERGENCE_CONSISTENT) ow = a.qw / 2;
   else if (a.op == PP_LAPLACIAN) ow = a.qw;
-  const float scale = (sym && a.op != PP_DENSITY && a.op != PP_INTERPOLATE && a.op != PP_LAPLACIAN) ? rho_i : 1.0f;
-  for (int t = 0; t < ow; ++t) a.out[(int64_t)i * ow + t] = sym ? scale * acc[t] : acc[t];
+  auto go = [&](auto kernel) { kernel<<<grid_for(a.n, kBlock / kPpLanes), kBlock, 0, st>>>(a, ow); };
+  ow <= 1 ? go(k_pp_operation<1>)
+          : (ow <= 2 ? go(k_pp_operation<2>) : (ow <= 4 ? go(k_pp_operation<4>) : go(k_pp_operation<8>)));
+  return launch_status();
 }
 
 // Row offsets of a row-sorted pair list: off[r] = first pair of row r;
@@ -367,8 +399,7 @@ extern "C" int dsph_pp_operation(const dsph_pair_arrays* pa, int32_t op, int32_t
   a.mode = mode;
   a.dot = dot_mode != 0;
   a.out = out;
-  k_pp_operation<<<grid_for(a.n), kBlock, 0, as_stream(stream)>>>(a);
-  return launch_status();
+  return launch_pp_operation(a, as_stream(stream));
 }
 
 extern "C" int dsph_pp_dfsph_alpha(const dsph_pair_arrays* pa, const float* actual_area_a,
