@@ -737,25 +737,37 @@ __global__ void __launch_bounds__(kBlock) k_ghosts(const float2* __restrict__ bp
 
 // The reference's C++ mDBC op (mDBCDensityKernel, v2/cppSrc/mDBC.h:129-244):
 // x_gj = -(q h) xhat, b = sum m_j [W, gradW], Cramer's rule with
-// det + 1e-7, Shepard density for <= 5 neighbors, clamped at rho0.
-__device__ float mdbc_op_row(const PairsDev& G, int i, const float* __restrict__ mass,
-                             const float* __restrict__ rho, const float2* __restrict__ bpos, float rho0,
-                             float* __restrict__ shepard) {
+// det + 1e-7, Shepard density for <= 5 neighbors, clamped at rho0.  Sixteen
+// lanes per ghost (the terms of MdbcOpAcc::add in row order): a wall has a few
+// thousand ghosts, one thread each left most CUs idle (9k ghosts of the 131k
+// dam break: 33 -> 8.7 us).
+constexpr int kGhostLanes = 16;
+__global__ void __launch_bounds__(kBlock) k_mdbc_op(PairsDev G, const float* __restrict__ mass,
+                                                    const float* __restrict__ rho, const float2* __restrict__ bpos,
+                                                    float rho0, float* __restrict__ rho_b,
+                                                    float* __restrict__ shepard) {
+  const int row = (int)((blockIdx.x * (unsigned)kBlock + threadIdx.x) / kGhostLanes);
+  const bool valid = row < G.nq;
+  const int i = valid ? row : G.nq - 1;
   const float2 xg = G.qpos[i];
   const float hi = h_of(G.qh, i, G.h0);
+  RowRef rr = row_ref(G, i);
+  if (!valid) rr.cnt = 0;
+  float a[12] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  sum_row<kGhostLanes, 1>(
+      G.nbr, rr, 0, a, [&](int j, int) { return j; }, [&](const int(&d)[1], float(&t)[1][12]) {
+        const int j = d[0];
+        const float h = pick_h(G.mode, hi, h_of(G.rh, j, G.h0));
+        const Geom g = pair_geom(xg, G.rpos[j], h, G.dom);
+        MdbcOpAcc::terms(mass[j], rho[j], g.w, g.gx, g.gy, ((-g.q) * g.h) * g.ex, ((-g.q) * g.h) * g.ey, t[0]);
+      });
+  if (!valid || (threadIdx.x & (kGhostLanes - 1)) != 0) return;
   MdbcOpAcc acc;
-  const RowRef rr = row_ref(G, i);
-  for (int n = 0, k = rr.base; n < rr.cnt; ++n, k += rr.step) {
-    const int j = G.nbr[k];
-    const float h = pick_h(G.mode, hi, h_of(G.rh, j, G.h0));
-    const Geom g = pair_geom(xg, G.rpos[j], h, G.dom);
-    acc.add(mass[j], rho[j], g.w, g.gx, g.gy, ((-g.q) * g.h) * g.ex, ((-g.q) * g.h) * g.ey);
-  }
+  acc.set(a);
   const float2 xb = bpos[i];
   float shep;
-  const float out = acc.finish(rr.cnt, xb.x - xg.x, xb.y - xg.y, rho0, &shep);
+  rho_b[i] = acc.finish(rr.cnt, xb.x - xg.x, xb.y - xg.y, rho0, &shep);
   if (shepard) shepard[i] = shep;
-  return out;
 }
 
 // mDBC wall density (mDBCDensity, v2/modules/mDBC.py:50-136): per ghost g
@@ -765,17 +777,12 @@ __device__ float mdbc_op_row(const PairsDev& G, int i, const float* __restrict__
 //        reference fills A_g], b = [sum m_j W, sum m_j gradW]
 //   rho_b = rho0 (no neighbors), rho_S (1..5 neighbors), else
 //   c = pinv(A) b (pinv only for > 4 neighbors) and rho_b = c0 + (x_b - x_g) . c[1:].
-// variant 1 is the C++ op above.
 __global__ void __launch_bounds__(kBlock) k_mdbc(PairsDev G, const float* __restrict__ mass,
                                                  const float* __restrict__ rho, const float2* __restrict__ bpos,
-                                                 float rho0, float support, int variant, float* __restrict__ rho_b,
+                                                 float rho0, float support, float* __restrict__ rho_b,
                                                  float* __restrict__ shepard) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= G.nq) return;
-  if (variant == 1) {
-    rho_b[i] = mdbc_op_row(G, i, mass, rho, bpos, rho0, shepard);
-    return;
-  }
   const float2 xg = G.qpos[i];
   const float hi = h_of(G.qh, i, G.h0);
   float nom = 0.f, vol = 0.f, gsx = 0.f, gsy = 0.f, vgx = 0.f, vgy = 0.f, psx = 0.f, psy = 0.f;
@@ -1258,8 +1265,12 @@ extern "C" int dsph_mdbc(const dsph_pairs* ghost_pairs, const float* fluid_mass,
   if (ghost_pairs->nq == 0) return DSPH_OK;
   if (!boundary_pos || !boundary_rho || (ghost_pairs->nr > 0 && (!fluid_mass || !fluid_rho))) return DSPH_ERR_ARG;
   PairsDev G = make_pairs(*ghost_pairs);
-  k_mdbc<<<grid_for(G.nq), kBlock, 0, as_stream(stream)>>>(G, fluid_mass, fluid_rho,
-                                                            reinterpret_cast<const float2*>(boundary_pos), rho0,
-                                                            support, variant, boundary_rho, shepard);
+  const float2* xb = reinterpret_cast<const float2*>(boundary_pos);
+  hipStream_t st = as_stream(stream);
+  if (variant == 1)
+    k_mdbc_op<<<grid_for(G.nq, kBlock / kGhostLanes), kBlock, 0, st>>>(G, fluid_mass, fluid_rho, xb, rho0,
+                                                                       boundary_rho, shepard);
+  else
+    k_mdbc<<<grid_for(G.nq), kBlock, 0, st>>>(G, fluid_mass, fluid_rho, xb, rho0, support, boundary_rho, shepard);
   return launch_status();
 }

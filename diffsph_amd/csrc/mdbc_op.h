@@ -42,6 +42,40 @@ struct MdbcOpAcc {
     bz += m_j * gy;
   }
 
+  // The terms of add() (nom and bx, den and m00 are the same sums), and the
+  // accumulator of their sums.
+  static __device__ __forceinline__ void terms(float m_j, float rho_j, float w, float gx, float gy, float xx, float xy,
+                                               float (&t)[12]) {
+    const float V = m_j / rho_j;
+    const float vw = V * w, vgx = V * gx, vgy = V * gy;
+    t[0] = m_j * w;
+    t[1] = vw;
+    t[2] = vgx;
+    t[3] = vgy;
+    t[4] = vw * xx;
+    t[5] = vgx * xx;
+    t[6] = vgx * xy;
+    t[7] = vw * xy;
+    t[8] = vgy * xx;
+    t[9] = vgy * xy;
+    t[10] = m_j * gx;
+    t[11] = m_j * gy;
+  }
+  __device__ __forceinline__ void set(const float (&t)[12]) {
+    nom = bx = t[0];
+    den = m00 = t[1];
+    m10 = t[2];
+    m20 = t[3];
+    m01 = t[4];
+    m11 = t[5];
+    m21 = t[6];
+    m02 = t[7];
+    m12 = t[8];
+    m22 = t[9];
+    by = t[10];
+    bz = t[11];
+  }
+
   // Shepard density nom / (den + 1e-7); with <= 5 neighbors the wall density
   // is the Shepard density, else Cramer's rule on A c = b (det + 1e-7) and
   // c0 + (x_b - x_g) . c[1:]; both clamped below at rho0.
