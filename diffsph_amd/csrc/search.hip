@@ -244,6 +244,14 @@ __device__ __forceinline__ void scan_queries(const SearchArgs& a, const Queries<
 // Supports that differ between particles.
 static bool varied_support(const SearchArgs& a) { return a.rh || a.qh; }
 
+// Few enough queries for the 16-query workgroups: with supports per particle
+// (a Verlet search, ~36 particles a cell, rows staged 128 deep) a query is
+// several times the work and the larger workgroups leave a tail for longer
+// (102k queries, count + fill: 55 + 139 us with 16, 87 + 183 with 64).
+static bool small_query_set(const SearchArgs& a) {
+  return a.nq < (varied_support(a) ? (1 << 18) : kRowSmall);
+}
+
 template <int kRows, bool kH>
 __global__ void __launch_bounds__(kBlock) k_neighbor_count(SearchArgs a, int32_t* __restrict__ counts) {
   __shared__ Queries<kRows> Q;
@@ -456,7 +464,7 @@ static void launch_fill_rows(const SearchArgs& a, const FillOut& F, const FillTi
 static int launch_fill(const SearchArgs& a, FillOut F, const FillTiles* tiles, hipStream_t st) {
   F.depth = F.width > 0 ? (F.width < kRowStage ? F.width : kRowStage) : (F.slice ? kRowStage : 0);
   const bool vary = varied_support(a);
-  if (a.nq < kRowSmall)
+  if (small_query_set(a))
     vary ? launch_fill_rows<16, true>(a, F, tiles, st) : launch_fill_rows<16, false>(a, F, tiles, st);
   else
     vary ? launch_fill_rows<64, true>(a, F, tiles, st) : launch_fill_rows<64, false>(a, F, tiles, st);
@@ -653,7 +661,7 @@ extern "C" int dsph_neighbor_count(const dsph_domain* domain, const dsph_grid* g
   hipStream_t st = as_stream(stream);
   const bool vary = varied_support(a);
   auto launch = [&](auto kernel, int rows) { kernel<<<grid_for(nq, rows), kBlock, 0, st>>>(a, counts); };
-  if (nq < kRowSmall)
+  if (small_query_set(a))
     vary ? launch(k_neighbor_count<16, true>, 16) : launch(k_neighbor_count<16, false>, 16);
   else
     vary ? launch(k_neighbor_count<64, true>, 64) : launch(k_neighbor_count<64, false>, 64);
