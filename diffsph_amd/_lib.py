@@ -222,6 +222,7 @@ SIGNATURES = {
     "dsph_grid_dims": (C.c_int, [P(Domain), F32, P(Grid)]),
     "dsph_grid_build_workspace": (SZ, [I64, P(Grid)]),
     "dsph_grid_build": (C.c_int, [P(Domain), P(Grid), V, V, I64, V, V, V, V, V, V, SZ, V]),
+    "dsph_grid_build_wrapped": (C.c_int, [P(Domain), P(Grid), V, V, I64, V, V, V, V, V, V, V, SZ, V]),
     "dsph_neighbor_count": (C.c_int, [P(Domain), P(Grid), V, V, V, I64, V, V, I64, I32, F32, I32, V, V]),
     "dsph_neighbor_fill": (C.c_int, [P(Domain), P(Grid), V, V, V, I64, V, V, I64, I32, F32, I32, V, V, I64, V, I64,
                                      V]),
@@ -230,6 +231,8 @@ SIGNATURES = {
     "dsph_neighbor_fill_fixed": (C.c_int, [P(Domain), P(Grid), V, V, V, I64, V, V, I64, I32, F32, I32, I32, V, V,
                                            V, I64, V, V, V, V]),
     "dsph_neighbor_fill_fixed_map": (C.c_int, [P(Domain), P(Grid), V, V, V, I64, V, V, I64, I32, F32, I32, I32, V,
+                                               V, V, I64, V, V, V]),
+    "dsph_neighbor_fill_fixed_or": (C.c_int, [P(Domain), P(Grid), V, V, V, I64, V, V, I64, I32, F32, I32, I32, V,
                                                V, V, I64, V, V, V]),
     "dsph_neighbor_fill_fixed_tiles": (C.c_int, [P(Domain), P(Grid), V, V, V, I64, V, V, I64, I32, F32, I32, I32,
                                                  V, V, V, I64, V, V, I32, V, I64, V, V, V, V]),

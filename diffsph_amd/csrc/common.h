@@ -355,22 +355,27 @@ __device__ __forceinline__ RowRef row_ref(const PairsDev& P, int i) {
 
 // slot = atomicAdd(&count[key], 1) for every valid lane of the wave, with one
 // atomic per distinct key: lanes sharing a key take consecutive slots in lane
-// order.  All 64 lanes must call it (invalid lanes pass valid = false).
+// order.  The keys' atomics are issued together (one after the other their
+// latencies added up).  All 64 lanes must call it (invalid lanes pass valid =
+// false).
 __device__ __forceinline__ int wave_slot(int32_t* __restrict__ count, int key, bool valid) {
   const int lane = threadIdx.x & 63;
   unsigned long long remaining = __ballot(valid);
-  int slot = 0;
+  int first = lane, before = 0, total = 0;
   while (remaining) {
     const int leader = __ffsll((long long)remaining) - 1;
     const int lkey = __shfl(key, leader, 64);
     const unsigned long long same = __ballot(valid && key == lkey);
-    int base = 0;
-    if (lane == leader) base = atomicAdd(&count[lkey], __popcll(same));
-    base = __shfl(base, leader, 64);
-    if (valid && key == lkey) slot = base + __popcll(same & ((1ull << lane) - 1ull));
+    if (valid && key == lkey) {
+      first = leader;
+      before = __popcll(same & ((1ull << lane) - 1ull));
+      total = __popcll(same);
+    }
     remaining &= ~same;
   }
-  return slot;
+  int base = 0;
+  if (valid && lane == first) base = atomicAdd(&count[key], total);
+  return __shfl(base, first, 64) + before;
 }
 
 // body(j, load(j)) for j = b .. e-1 in order; the loads of U consecutive j

@@ -225,20 +225,27 @@ __global__ void __launch_bounds__(kBlock) k_dsph_normalization_near(PairsDev P, 
   constexpr int U = 4;
   float acc[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   sum_row<kLanes, U>(P.nbr, rr, i, acc, ld, [&](const NbrXMR(&d)[U], float(&t)[U][6]) {
-    float dx[U], dy[U], V[U];
+    float dx[U], dy[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       dx[u] = xi.x - d[u].x.x;
       dy[u] = xi.y - d[u].x.y;
-      V[u] = kVol ? d[u].m : d[u].m / d[u].r;
     }
     wrap_offsets(dx, dy, dm);
     NearRange range;
 #pragma unroll
-    for (int u = 0; u < U; ++u) put(pair_geom_near(dx[u], dy[u], h, kc, range), V[u], d[u].r, t[u]);
+    for (int u = 0; u < U; ++u) {
+      float V = d[u].m;
+      if (!kVol) {
+        range.operand(d[u].m);
+        V = div_near(d[u].m, d[u].r, range.divisor(d[u].r));
+      }
+      put(pair_geom_near(dx[u], dy[u], h, kc, range), V, d[u].r, t[u]);
+    }
     if (range.odd()) {
 #pragma unroll
-      for (int u = 0; u < U; ++u) put(pair_geom(xi, d[u].x, h, kc, dm), V[u], d[u].r, t[u]);
+      for (int u = 0; u < U; ++u)
+        put(pair_geom(xi, d[u].x, h, kc, dm), kVol ? d[u].m : d[u].m / d[u].r, d[u].r, t[u]);
     }
   });
   float bx = 0.f, by = 0.f;

@@ -109,16 +109,17 @@ __global__ void __launch_bounds__(kBlock) k_scan_final(const int32_t* __restrict
     out[n] = (int32_t)(uint32_t)(uint64_t)(block_offsets[blockIdx.x] + tot);
 }
 
-// Up to kScanOne elements in one workgroup: the three launches above are each
-// a few microseconds of latency for a grid of 256 to 16k cells (7.2 -> 2.7
+// Up to kScanOne elements in one workgroup (16k elements: 9.4 us, the three
+// launches 8.7): the launches above are each
+// a few microseconds of latency for a grid of 256 to 4k cells (7.2 -> 2.7
 // us for the 256 cells of a 64^2 box).
-constexpr int kScanOne = 1 << 14;
+constexpr int kScanOne = 1 << 12;
 constexpr int kScanOneBlock = 1024;
 __global__ void __launch_bounds__(kScanOneBlock) k_scan_one(const int32_t* __restrict__ in, int n,
                                                             int32_t* __restrict__ out,
                                                             ScanHeader* __restrict__ hdr) {
   __shared__ int64_t wsum[kScanOneBlock / 64];
-  int per = 1;  // elements per thread, a power of two up to 16
+  int per = 1;  // elements per thread, a power of two up to 4
   while (per * kScanOneBlock < n) per *= 2;
   const int base = threadIdx.x * per;
   int v[kScanOne / kScanOneBlock];

@@ -33,7 +33,8 @@ __device__ __forceinline__ int cell_coord(float x, const Dom& d, int k, const Gr
 
 __global__ void __launch_bounds__(kBlock) k_cell_keys(const float2* __restrict__ pos, int n, Dom d, GridDev g,
                                                       int32_t* __restrict__ keys, int32_t* __restrict__ slot,
-                                                      int32_t* __restrict__ cell_count) {
+                                                      int32_t* __restrict__ cell_count,
+                                                      float2* __restrict__ wrapped) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   const bool valid = i < n;
   int key = 0;
@@ -43,6 +44,7 @@ __global__ void __launch_bounds__(kBlock) k_cell_keys(const float2* __restrict__
     int cx = cell_coord(wx, d, 0, g), cy = cell_coord(wy, d, 1, g);
     key = cy * g.nc[0] + cx;
     keys[i] = key;
+    if (wrapped) wrapped[i] = make_float2(wx, wy);
   }
   const int sl = wave_slot(cell_count, key, valid);
   if (valid) slot[i] = sl;
@@ -318,6 +320,9 @@ struct FillOut {
   int32_t* row_ovf;
   const int32_t* map;
   int depth;  // staged entries per row (0: CSR)
+  // fixed width without a pass before the fill: the slice offsets are written
+  // here, and the overflow bits are OR-ed into *row_ovf (not cleared)
+  int32_t* slices_out;
 };
 
 // Neighbor rows [blockIdx * kRows, + kRows).  In the sliced layouts the first
@@ -404,7 +409,13 @@ __global__ void __launch_bounds__(kBlock) k_neighbor_fill(SearchArgs a, FillOut 
       },
       [&](int r, int n) { found[r] = n; });
   if (kTiles && tbad) T.n[tile] = -1;
-  if (F.width > 0 && over) atomicMax(F.row_ovf, 2);
+  auto overflow = [&](int bit) { F.slices_out ? atomicOr(F.row_ovf, bit) : atomicMax(F.row_ovf, bit); };
+  if (F.width > 0 && over) overflow(2);
+  if (F.slices_out && threadIdx.x == 0) {
+    if ((i0 & 63) == 0) F.slices_out[i0 >> 6] = (i0 >> 6) * 64 * F.width;
+    const int last = (a.nq + 63) >> 6;
+    if (blockIdx.x == 0) F.slices_out[last] = last * 64 * F.width;
+  }
   __syncthreads();
   const int r = threadIdx.x % kRows, i = i0 + r;
   if (i < a.nq) {
@@ -414,7 +425,7 @@ __global__ void __launch_bounds__(kBlock) k_neighbor_fill(SearchArgs a, FillOut 
     if (F.width > 0 && threadIdx.x < kRows) {
       // entries past the row's count are never read: no padding
       F.counts[i] = n < len ? n : (int32_t)len;
-      if (n > len) atomicMax(F.row_ovf, 1);
+      if (n > len) overflow(1);
     }
     if (F.depth > 0) {
       const int staged = (int)(n < F.depth ? (n < len ? n : len) : (F.depth < len ? F.depth : len));
@@ -476,7 +487,7 @@ __global__ void __launch_bounds__(kBlock) k_fixed_slices(int nslices, int width,
                                                          int32_t* __restrict__ d16_ovf) {
   const int s = blockIdx.x * blockDim.x + threadIdx.x;
   if (s == 0) {
-    *row_ovf = 0;
+    if (row_ovf) *row_ovf = 0;
     if (d16_ovf) *d16_ovf = 0;
   }
   if (s <= nslices) slice_off[s] = s * 64 * width;
@@ -603,9 +614,10 @@ extern "C" size_t dsph_grid_build_workspace(int64_t n, const dsph_grid* grid) {
   return align256((size_t)n * 4) * 3 + align256((size_t)ncell * 4) + scan_ws(ncell);
 }
 
-extern "C" int dsph_grid_build(const dsph_domain* domain, const dsph_grid* grid, const float* pos, const float* h,
-                               int64_t n, int32_t* cell_start, int32_t* sort_index, int32_t* rank,
-                               float* sorted_pos, float* sorted_h, void* ws, size_t ws_bytes, void* stream) {
+extern "C" int dsph_grid_build_wrapped(const dsph_domain* domain, const dsph_grid* grid, const float* pos,
+                                       const float* h, int64_t n, int32_t* cell_start, int32_t* sort_index,
+                                       int32_t* rank, float* sorted_pos, float* sorted_h, float* wrapped, void* ws,
+                                       size_t ws_bytes, void* stream) {
   if (!domain || check_grid(grid) != DSPH_OK || n < 0 || n >= INT32_MAX) return DSPH_ERR_ARG;
   if (!cell_start || (n > 0 && (!pos || !sort_index || !sorted_pos))) return DSPH_ERR_ARG;
   if (sorted_h && !h) return DSPH_ERR_ARG;
@@ -633,7 +645,8 @@ extern "C" int dsph_grid_build(const dsph_domain* domain, const dsph_grid* grid,
   // a fill kernel rather than a memset node, so the call can be captured
   k_zero_i32<<<grid_for(ncell > 0 ? ncell : 1), kBlock, 0, st>>>(count, ncell);
   if (n > 0) {
-    k_cell_keys<<<grid_for(n), kBlock, 0, st>>>(reinterpret_cast<const float2*>(pos), (int)n, d, g, keys, slot, count);
+    k_cell_keys<<<grid_for(n), kBlock, 0, st>>>(reinterpret_cast<const float2*>(pos), (int)n, d, g, keys, slot, count,
+                                              reinterpret_cast<float2*>(wrapped));
     DSPH_LAUNCH_CHECK();
   }
   int s = scan_exclusive(count, ncell, cell_start, scan_w, scan_b, st);
@@ -646,6 +659,13 @@ extern "C" int dsph_grid_build(const dsph_domain* domain, const dsph_grid* grid,
     DSPH_LAUNCH_CHECK();
   }
   return DSPH_OK;
+}
+
+extern "C" int dsph_grid_build(const dsph_domain* domain, const dsph_grid* grid, const float* pos, const float* h,
+                               int64_t n, int32_t* cell_start, int32_t* sort_index, int32_t* rank,
+                               float* sorted_pos, float* sorted_h, void* ws, size_t ws_bytes, void* stream) {
+  return dsph_grid_build_wrapped(domain, grid, pos, h, n, cell_start, sort_index, rank, sorted_pos, sorted_h, nullptr,
+                                 ws, ws_bytes, stream);
 }
 
 extern "C" int dsph_neighbor_count(const dsph_domain* domain, const dsph_grid* grid, const int32_t* cell_start,
@@ -710,7 +730,8 @@ static int fill_fixed(const dsph_domain* domain, const dsph_grid* grid, const in
                       const float* sorted_pos, const float* sorted_h, int64_t nref, const float* qpos, const float* qh,
                       int64_t nq, int32_t qpos_wrapped, float h_uniform, int32_t mode, int32_t width, int32_t* counts,
                       int32_t* slice_off, int32_t* nbr, int64_t capacity, int16_t* nbr16, int32_t* delta_overflow,
-                      int32_t* row_overflow, const int32_t* map, const FillTiles* tiles, void* stream) {
+                      int32_t* row_overflow, const int32_t* map, const FillTiles* tiles, void* stream,
+                      bool accumulate = false) {
   SearchArgs a;
   int s = make_search(a, domain, grid, cell_start, sorted_pos, sorted_h, nref, qpos, qh, nq, qpos_wrapped,
                       h_uniform, mode);
@@ -722,9 +743,11 @@ static int fill_fixed(const dsph_domain* domain, const dsph_grid* grid, const in
   if (nslices * 64 * (int64_t)width >= INT32_MAX) return DSPH_ERR_ARG;
   if (capacity < nslices * 64 * (int64_t)width) return DSPH_ERR_CAPACITY;
   hipStream_t st = as_stream(stream);
-  k_fixed_slices<<<grid_for(nslices + 1), kBlock, 0, st>>>((int)nslices, width, slice_off, row_overflow,
-                                                          delta_overflow);
-  DSPH_LAUNCH_CHECK();
+  if (!accumulate || nq == 0) {
+    k_fixed_slices<<<grid_for(nslices + 1), kBlock, 0, st>>>((int)nslices, width, slice_off,
+                                                            accumulate ? nullptr : row_overflow, delta_overflow);
+    DSPH_LAUNCH_CHECK();
+  }
   if (nq == 0) return DSPH_OK;
   if (!counts || !nbr) return DSPH_ERR_ARG;
   if (tiles) {
@@ -732,7 +755,8 @@ static int fill_fixed(const dsph_domain* domain, const dsph_grid* grid, const in
     if (s2 != DSPH_OK) return s2;
   }
   return launch_fill(a,
-                     FillOut{nullptr, nullptr, nbr, capacity, nbr16, delta_overflow, width, counts, row_overflow, map},
+                     FillOut{nullptr, nullptr, nbr, capacity, nbr16, delta_overflow, width, counts, row_overflow, map,
+                             0, accumulate ? slice_off : nullptr},
                      tiles, st);
 }
 }  // namespace dsph
@@ -758,6 +782,17 @@ extern "C" int dsph_neighbor_fill_fixed_map(const dsph_domain* domain, const dsp
   if (nref > 0 && !map) return DSPH_ERR_ARG;
   return fill_fixed(domain, grid, cell_start, sorted_pos, sorted_h, nref, qpos, qh, nq, qpos_wrapped, h_uniform, mode,
                     width, counts, slice_off, nbr, capacity, nullptr, nullptr, row_overflow, map, nullptr, stream);
+}
+
+extern "C" int dsph_neighbor_fill_fixed_or(const dsph_domain* domain, const dsph_grid* grid,
+                                           const int32_t* cell_start, const float* sorted_pos, const float* sorted_h,
+                                           int64_t nref, const float* qpos, const float* qh, int64_t nq,
+                                           int32_t qpos_wrapped, float h_uniform, int32_t mode, int32_t width,
+                                           int32_t* counts, int32_t* slice_off, int32_t* nbr, int64_t capacity,
+                                           const int32_t* map, int32_t* row_overflow, void* stream) {
+  return fill_fixed(domain, grid, cell_start, sorted_pos, sorted_h, nref, qpos, qh, nq, qpos_wrapped, h_uniform, mode,
+                    width, counts, slice_off, nbr, capacity, nullptr, nullptr, row_overflow, map, nullptr, stream,
+                    true);
 }
 
 extern "C" int dsph_neighbor_fill_fixed_tiles(const dsph_domain* domain, const dsph_grid* grid,

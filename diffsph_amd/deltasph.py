@@ -28,7 +28,7 @@ import torch
 
 from . import _lib
 from ._lib import DsphError, check, lib, ptr
-from .neighborhood import WORKSPACE, CellGrid, search, wrap_positions
+from .neighborhood import WORKSPACE, CellGrid, search
 
 VISCOSITY = {None: -1, "none": -1, "deltaSPH_inviscid": 0, "deltaSPH_viscid": 1}
 EOS = {"isoThermal": 0, "Tait": 1}
@@ -325,8 +325,9 @@ class DeltaSPHSolver:
         mapped to state indices; returns (NeighborList, pairs descriptor,
         wrapped positions, grid)."""
         cfg = self.cfg
-        grid = CellGrid.build(pos, None, self.domain, cfg.support * cfg.cell_scale, h_uniform=cfg.support)
-        wpos = wrap_positions(pos, self.domain)
+        wpos = torch.empty_like(pos)
+        grid = CellGrid.build(pos, None, self.domain, cfg.support * cfg.cell_scale, h_uniform=cfg.support,
+                              wrapped=wpos)
         nl = self._search("fluid", grid, wpos, remap=True)
         pr = nl.pairs()
         pr.rpos = ptr(wpos)
@@ -365,9 +366,12 @@ class DeltaSPHSolver:
         bp = C.byref(bnd) if bnd is not None else None
         L_ = lib()
         if self.cfg.diffusion or L is not None or eigvals is not None:
-            # V_j = m_j / rho_j once per particle for the normalization pass
-            check(L_.dsph_volume(self.n, ptr(self.mass), ptr(rho), ptr(self._vol), st), "volume")
-            check(L_.dsph_deltasph_normalization_v(C.byref(pr), bp, ptr(self.mass), ptr(rho), ptr(self._vol),
+            # V_j = m_j / rho_j once per particle for the normalization pass;
+            # up to 64k particles the launch costs more than the quotients
+            vol = self._vol if self.n > 1 << 16 else None
+            if vol is not None:
+                check(L_.dsph_volume(self.n, ptr(self.mass), ptr(rho), ptr(vol), st), "volume")
+            check(L_.dsph_deltasph_normalization_v(C.byref(pr), bp, ptr(self.mass), ptr(rho), ptr(vol),
                                                    ptr(L), ptr(eigvals), ptr(self._grad), st),
                   "deltasph_normalization")
         check(L_.dsph_deltasph_rhs(C.byref(pr), bp, C.byref(self.prm), ptr(vel), ptr(self.mass), ptr(rho),
@@ -382,16 +386,14 @@ class DeltaSPHSolver:
         self.last_sort = si
         st = _lib.stream_handle(self.pos.device)
 
-        def perm(t):
-            out = torch.empty_like(t)
-            if t.dtype == torch.float32:
-                w = 1 if t.dim() == 1 else t.shape[1]
-                check(lib().dsph_gather_f32(ptr(t), ptr(si), self.n, w, ptr(out), st), "gather")
-                return out
-            return t[si.long()]
-
-        self.pos, self.vel, self.mass, self.rho, self.uid = (perm(t) for t in
-                                                             (self.pos, self.vel, self.mass, self.rho, self.uid))
+        src = [t.contiguous() for t in (self.pos, self.vel, self.mass, self.rho, self.uid)]
+        dst = [torch.empty_like(t) for t in src]
+        k = len(src)
+        words = [t.element_size() * (t.numel() // max(self.n, 1)) // 4 for t in src]
+        check(lib().dsph_gather_set(ptr(si), self.n, k, (C.c_void_p * k)(*[t.data_ptr() for t in src]),
+                                    (C.c_void_p * k)(*[t.data_ptr() for t in dst]), (C.c_int32 * k)(*words), st),
+              "gather_set")
+        self.pos, self.vel, self.mass, self.rho, self.uid = dst
 
     # -- one step ------------------------------------------------------------
     def step(self) -> float:
@@ -404,20 +406,22 @@ class DeltaSPHSolver:
         dt = float(np.float32(self.dt))
         half = float(np.float32(dt) * np.float32(0.5))
         x0, u0, r0 = self.pos, self.vel, self.rho
-        xs, us, rs = self._stage
+        xs, _, rs = self._stage
         x, u, r = x0, u0, r0
+        dxdt = [None] * 4
         for s, c in enumerate([half, half, dt, None]):
-            kx, ku, kr = self._k[s]
-            kx.copy_(u)                     # dx/dt of this stage = its velocity
+            _, ku, kr = self._k[s]
+            kx = dxdt[s] = u                # dx/dt of this stage = its velocity
             self.rhs(x, u, r, ku, kr)
             self._last_nl = self._keep[0]
             if c is not None:
+                us = self._k[s + 1][0]      # a buffer of its own: the combination reads it
                 check(L_.dsph_rk_update(self.n, ptr(x0), ptr(kx), ptr(xs), ptr(u0), ptr(ku), ptr(us), ptr(r0),
                                         ptr(kr), ptr(rs), C.c_float(c), st), "rk_update")
                 x, u, r = xs, us, rs
         stages = _lib.RK4Stages()
         for s in range(4):
-            stages.dxdt[s] = ptr(self._k[s][0])
+            stages.dxdt[s] = ptr(dxdt[s])
             stages.dudt[s] = ptr(self._k[s][1])
             stages.drhodt[s] = ptr(self._k[s][2])
         if self.dudt is None:
@@ -454,20 +458,22 @@ class DeltaSPHSolver:
         dt_dev, time_dev = self._device_clock()
         self._sort()
         x0, u0, r0 = self.pos, self.vel, self.rho
-        xs, us, rs = self._stage
+        xs, _, rs = self._stage
         x, u, r = x0, u0, r0
+        dxdt = [None] * 4
         for k, half in enumerate((1, 1, 0, None)):
-            kx, ku, kr = self._k[k]
-            kx.copy_(u)
+            _, ku, kr = self._k[k]
+            kx = dxdt[k] = u
             self.rhs(x, u, r, ku, kr)
             self._last_nl = self._keep[0]
             if half is not None:
+                us = self._k[k + 1][0]
                 check(L_.dsph_rk_update_dev(self.n, ptr(x0), ptr(kx), ptr(xs), ptr(u0), ptr(ku), ptr(us), ptr(r0),
                                             ptr(kr), ptr(rs), ptr(dt_dev), half, st), "rk_update_dev")
                 x, u, r = xs, us, rs
         stages = _lib.RK4Stages()
         for k in range(4):
-            stages.dxdt[k] = ptr(self._k[k][0])
+            stages.dxdt[k] = ptr(dxdt[k])
             stages.dudt[k] = ptr(self._k[k][1])
             stages.drhodt[k] = ptr(self._k[k][2])
         check(L_.dsph_rk4_combine_dev(self.n, C.byref(stages), ptr(self.pos), ptr(self.vel), ptr(self.rho),

@@ -94,7 +94,8 @@ class CellGrid:
 
     @staticmethod
     def build(positions: torch.Tensor, supports: torch.Tensor | None, domain: _lib.Domain,
-              hsearch: float, h_uniform: float = 0.0) -> "CellGrid":
+              hsearch: float, h_uniform: float = 0.0, wrapped: torch.Tensor | None = None) -> "CellGrid":
+        """`wrapped` (optional, [n, 2]): receives the wrapped positions in input order."""
         _check_f32(positions, "positions", (2,))
         n = positions.shape[0]
         dev = positions.device
@@ -111,10 +112,10 @@ class CellGrid:
             sorted_h = torch.empty(n, dtype=torch.float32, device=dev)
         wsb = lib().dsph_grid_build_workspace(n, C.byref(grid))
         ws = WORKSPACE.get(wsb, dev)
-        check(lib().dsph_grid_build(C.byref(domain), C.byref(grid), ptr(positions), ptr(supports), n,
-                                    ptr(cell_start), ptr(sort_index), ptr(rank), ptr(sorted_pos),
-                                    ptr(sorted_h), ptr(ws), ws.numel(), _lib.stream_handle(dev)),
-              "grid_build")
+        check(lib().dsph_grid_build_wrapped(C.byref(domain), C.byref(grid), ptr(positions), ptr(supports), n,
+                                            ptr(cell_start), ptr(sort_index), ptr(rank), ptr(sorted_pos),
+                                            ptr(sorted_h), ptr(wrapped), ptr(ws), ws.numel(),
+                                            _lib.stream_handle(dev)), "grid_build")
         return CellGrid(domain, grid, n, cell_start, sort_index, rank, sorted_pos, sorted_h,
                         float(h_uniform))
 
@@ -346,6 +347,13 @@ def _search_fixed(L, args, grid, qpos, qh, m, qpos_wrapped, counts, delta16, wid
     cap = max(nsl * 64 * width, 1)
     slice_off = torch.empty(nsl + 1, dtype=torch.int32, device=dev)
     nbr = torch.empty(cap, dtype=torch.int32, device=dev)
+    if deferred is not None and delta16 is None and tiles is None:
+        # the pair kernels read the sliced rows (counts + slice offsets): the
+        # CSR offsets are built only if asked for (NeighborList.ensure_offsets)
+        check(L.dsph_neighbor_fill_fixed_or(*args, width, ptr(counts), ptr(slice_off), ptr(nbr), cap, ptr(remap),
+                                            ptr(deferred), st), "neighbor_fill_fixed_or")
+        wq = qpos if qpos_wrapped else wrap_positions(qpos, grid.domain)
+        return NeighborList(counts, None, nbr, None, wq, qh, grid, m, slice_off, cap, None, None, width)
     info = torch.empty(2, dtype=torch.int32, device=dev)   # [row overflow, pair total]
     buf16 = flag16 = None
     if delta16 is not None:
@@ -362,8 +370,6 @@ def _search_fixed(L, args, grid, qpos, qh, m, qpos_wrapped, counts, delta16, wid
         check(L.dsph_neighbor_fill_fixed(*args, width, ptr(counts), ptr(slice_off), ptr(nbr), cap, ptr(buf16),
                                          ptr(flag16), ptr(info), st), "neighbor_fill_fixed")
     if deferred is not None:
-        # the pair kernels read the sliced rows (counts + slice offsets): the
-        # CSR offsets are built only if asked for (NeighborList.ensure_offsets)
         torch.bitwise_or(deferred, info[:1], out=deferred)
         offsets, npairs = None, None
     else:

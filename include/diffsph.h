@@ -200,6 +200,15 @@ int dsph_grid_build(const dsph_domain* domain, const dsph_grid* grid,
                     float* sorted_pos, float* sorted_h,
                     void* workspace, size_t workspace_bytes, void* stream);
 
+/* dsph_grid_build that also writes the wrapped positions in input order
+ * (wrapped[n,2], NULL: not written), as dsph_wrap_positions makes them. */
+int dsph_grid_build_wrapped(const dsph_domain* domain, const dsph_grid* grid,
+                            const float* pos, const float* h, int64_t n,
+                            int32_t* cell_start, int32_t* sort_index,
+                            int32_t* rank, float* sorted_pos, float* sorted_h,
+                            float* wrapped, void* workspace,
+                            size_t workspace_bytes, void* stream);
+
 /* Count, for each query particle, the reference particles within its support
  * (replaces countNeighbors, neighborhood.cpp:65-227, and the counting pass
  * of computeNeighborhood, v2/cppSrc/computeNeighborhood.h:115-146).
@@ -265,6 +274,19 @@ int dsph_neighbor_fill_fixed_map(const dsph_domain* domain, const dsph_grid* gri
                                  int32_t width, int32_t* counts, int32_t* slice_off,
                                  int32_t* nbr, int64_t capacity, const int32_t* map,
                                  int32_t* row_overflow, void* stream);
+
+/* dsph_neighbor_fill_fixed (map NULL) or dsph_neighbor_fill_fixed_map whose
+ * overflow bits are OR-ed into *row_overflow instead of replacing it: several
+ * searches share one flag that the caller clears and reads.  No 16-bit
+ * deltas.  No counterpart in the reference. */
+int dsph_neighbor_fill_fixed_or(const dsph_domain* domain, const dsph_grid* grid,
+                                const int32_t* cell_start, const float* sorted_pos,
+                                const float* sorted_h, int64_t nref,
+                                const float* qpos, const float* qh, int64_t nq,
+                                int32_t qpos_wrapped, float h_uniform, int32_t mode,
+                                int32_t width, int32_t* counts, int32_t* slice_off,
+                                int32_t* nbr, int64_t capacity, const int32_t* map,
+                                int32_t* row_overflow, void* stream);
 
 /* dsph_neighbor_fill_fixed that also builds the list's neighbor tiles (the
  * tile_* fields of dsph_pairs; the list must be square: nq == nref and

@@ -35,8 +35,8 @@ def test_scan_matches_numpy(n):
     assert np.array_equal(out.astype(np.int64), ref) and tot == ref[-1]
 
 
-# the one-workgroup form: per-thread counts 1 to 16 and its last size
-@pytest.mark.parametrize("n", [1023, 1025, 4097, 8191, 16384, 16385])
+# around the per-thread counts (1, 2, 4) and the last size of the one-workgroup form
+@pytest.mark.parametrize("n", [1023, 1025, 2049, 4095, 4096, 4097, 16385])
 def test_scan_one_workgroup_matches_numpy(n):
     c = np.random.default_rng(n).integers(0, 200, n).astype(np.int64)
     out, tot = _scan(c)
