@@ -86,6 +86,18 @@ __global__ void __launch_bounds__(kBlock) k_mlp_pack(const float* __restrict__ p
   pk[t] = v;
 }
 
+typedef __bf16 bf16p2 __attribute__((ext_vector_type(2)));
+typedef float f32p2 __attribute__((ext_vector_type(2)));
+
+// Four floats to bf16 by the hardware conversion (round to nearest even, two
+// per instruction; f2bf is five operations each).
+__device__ __forceinline__ short4v f2bf4(float a, float b, float c, float d) {
+  const bf16p2 lo = __builtin_convertvector((f32p2{a, b}), bf16p2);
+  const bf16p2 hi = __builtin_convertvector((f32p2{c, d}), bf16p2);
+  const uint2 v = make_uint2(__builtin_bit_cast(uint32_t, lo), __builtin_bit_cast(uint32_t, hi));
+  return __builtin_bit_cast(short4v, v);
+}
+
 struct MlpTile {
   // C-layout fp32 pre-activations (z + b) and bf16 post-activations of the
   // three hidden layers: [layer][nt] -> 4 rows (4q + j) of column 16nt + c.
@@ -94,10 +106,29 @@ struct MlpTile {
   float y[4];
 };
 
+// What a training wave keeps for all its tiles: the biases and output weights
+// of its columns.
+struct MlpCols {
+  float b[3][4], w4[4], b4;
+};
+
+// The inputs of one 16-sample tile: row c (layer 1's A operand), column c (the
+// weight gradient's) and the targets.  Rows >= n read as 0.
+struct MlpIn {
+  float a[4], t[4], y[4];
+};
+
 // LDS transpose: C layout (rows 4q+j, col 16nt+c) -> A layout (row c, cols
 // 16kt+4q+j).  buf holds 16 x 64 bf16 for this wave (row stride 68 to keep
-// the 16 rows of a column in distinct banks).
+// the 16 rows of a column in distinct banks).  The buffer is the wave's own
+// and its LDS operations complete in order, so no workgroup barrier is
+// needed, only their order in the program.
 constexpr int kLdsStride = 68;
+
+__device__ __forceinline__ void lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
 
 __device__ __forceinline__ void c_to_a(const short4v (&in)[4], short4v (&out)[4], short* buf) {
   const int l = threadIdx.x & 63, c = l & 15, q = l >> 4;
@@ -105,73 +136,71 @@ __device__ __forceinline__ void c_to_a(const short4v (&in)[4], short4v (&out)[4]
   for (int nt = 0; nt < 4; ++nt)
 #pragma unroll
     for (int j = 0; j < 4; ++j) buf[(4 * q + j) * kLdsStride + 16 * nt + c] = in[nt][j];
-  __syncthreads();
+  lds_order();
 #pragma unroll
-  for (int kt = 0; kt < 4; ++kt)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) out[kt][j] = buf[c * kLdsStride + 16 * kt + 4 * q + j];
-  __syncthreads();
+  for (int kt = 0; kt < 4; ++kt) out[kt] = *reinterpret_cast<const short4v*>(buf + c * kLdsStride + 16 * kt + 4 * q);
+  lds_order();
 }
 
-// Forward of one 16-sample tile starting at row m0 (rows >= n read as 0).
-__device__ __forceinline__ void mlp_forward_tile(const float* __restrict__ X, int n, int m0,
-                                                 const float* __restrict__ prm, const short4v* __restrict__ pk,
-                                                 short* lds, MlpTile& T) {
+__device__ __forceinline__ MlpIn mlp_load_tile(const float* __restrict__ X, const float* __restrict__ Tg, int n,
+                                               int m0) {
   const int l = threadIdx.x & 63, c = l & 15, q = l >> 4;
-  short4v xa;
-  {
-    const int m = m0 + c;
+  MlpIn v;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) xa[j] = f2bf(m < n ? X[(int64_t)m * kFin + 4 * q + j] : 0.0f);
+  for (int j = 0; j < 4; ++j) {
+    const int m = m0 + c, r = m0 + 4 * q + j;
+    v.a[j] = m < n ? X[(int64_t)m * kFin + 4 * q + j] : 0.0f;
+    v.t[j] = r < n ? X[(int64_t)r * kFin + c] : 0.0f;
+    v.y[j] = r < n ? Tg[r] : 0.0f;
   }
-  // layer 1
-#pragma unroll
-  for (int nt = 0; nt < 4; ++nt) {
-    float4v acc = {0.f, 0.f, 0.f, 0.f};
-    acc = mfma16(xa, pk[kPkW1 + nt * 64 + l], acc);
-    const float b = prm[kOffB1 + 16 * nt + c];
+  return v;
+}
+
+// Forward of one 16-sample tile; pk: the packed weights in LDS.
+__device__ __forceinline__ void mlp_forward_tile(const MlpIn& in, const MlpCols& W, const short4v* pk, short* lds,
+                                                 MlpTile& T) {
+  const int l = threadIdx.x & 63;
+  const short4v xa = f2bf4(in.a[0], in.a[1], in.a[2], in.a[3]);
+  auto activate = [&](int L, int nt, const float4v& acc) {
+    float r[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const float zz = acc[j] + b;
-      T.z[0][nt][j] = zz;
-      T.h[0][nt][j] = f2bf(zz > 0.0f ? zz : 0.0f);
+      const float zz = acc[j] + W.b[L][nt];
+      T.z[L][nt][j] = zz;
+      r[j] = zz > 0.0f ? zz : 0.0f;
     }
-  }
+    T.h[L][nt] = f2bf4(r[0], r[1], r[2], r[3]);
+  };
+  // layer 1
+#pragma unroll
+  for (int nt = 0; nt < 4; ++nt) activate(0, nt, mfma16(xa, pk[kPkW1 + nt * 64 + l], float4v{0.f, 0.f, 0.f, 0.f}));
   // layers 2, 3
 #pragma unroll
   for (int L = 1; L < 3; ++L) {
     short4v a[4];
     c_to_a(T.h[L - 1], a, lds);
     const int pkb = L == 1 ? kPkW2 : kPkW3;
-    const int bo = L == 1 ? kOffB2 : kOffB3;
 #pragma unroll
     for (int nt = 0; nt < 4; ++nt) {
       float4v acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int kt = 0; kt < 4; ++kt) acc = mfma16(a[kt], pk[pkb + (kt * 4 + nt) * 64 + l], acc);
-      const float b = prm[bo + 16 * nt + c];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const float zz = acc[j] + b;
-        T.z[L][nt][j] = zz;
-        T.h[L][nt][j] = f2bf(zz > 0.0f ? zz : 0.0f);
-      }
+      activate(L, nt, acc);
     }
   }
   // output layer (VALU): y[4q+j] = sum_k h3[4q+j][k] w4[k] + b4
   float s[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int nt = 0; nt < 4; ++nt) {
-    const float w = bf2f(f2bf(prm[kOffW4 + 16 * nt + c]));
 #pragma unroll
-    for (int j = 0; j < 4; ++j) s[j] += bf2f(T.h[2][nt][j]) * w;
+    for (int j = 0; j < 4; ++j) s[j] += bf2f(T.h[2][nt][j]) * W.w4[nt];
   }
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     float v = s[j];
 #pragma unroll
     for (int o = 1; o < 16; o <<= 1) v += __shfl_xor(v, o, 64);
-    T.y[j] = v + prm[kOffB4];
+    T.y[j] = v + W.b4;
   }
 }
 
@@ -344,8 +373,14 @@ __global__ void __launch_bounds__(kBlock) k_mlp_train(const float* __restrict__ 
                                                       int n, float lw, const float* __restrict__ prm,
                                                       const short4v* __restrict__ pk, float* __restrict__ gpart,
                                                       float* __restrict__ lpart) {
-  __shared__ short lds[4][16 * kLdsStride];
+  // The packed weights live in LDS for the launch: 68 fragment reads per tile
+  // from L1 were a latency chain that one wave per SIMD (the weight gradients
+  // fill the registers) could not hide.
+  __shared__ short4v wl[kPkTotal];
+  __shared__ __align__(8) short lds[4][16 * kLdsStride];
   __shared__ float red[4][1024];
+  for (int k = threadIdx.x; k < kPkTotal; k += kBlock) wl[k] = pk[k];
+  __syncthreads();
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63, c = l & 15, q = l >> 4;
   float4v gW1[4], gW2[4][4], gW3[4][4];
   float gb1[4] = {0, 0, 0, 0}, gb2[4] = {0, 0, 0, 0}, gb3[4] = {0, 0, 0, 0}, gw4[4] = {0, 0, 0, 0};
@@ -359,21 +394,31 @@ __global__ void __launch_bounds__(kBlock) k_mlp_train(const float* __restrict__ 
       gW3[a][b] = float4v{0.f, 0.f, 0.f, 0.f};
     }
   }
-  float w4b[4];
+  MlpCols C;
 #pragma unroll
-  for (int nt = 0; nt < 4; ++nt) w4b[nt] = bf2f(f2bf(prm[kOffW4 + 16 * nt + c]));
+  for (int nt = 0; nt < 4; ++nt) {
+    C.b[0][nt] = prm[kOffB1 + 16 * nt + c];
+    C.b[1][nt] = prm[kOffB2 + 16 * nt + c];
+    C.b[2][nt] = prm[kOffB3 + 16 * nt + c];
+    C.w4[nt] = bf2f(f2bf(prm[kOffW4 + 16 * nt + c]));
+  }
+  C.b4 = prm[kOffB4];
 
   const int ntiles = (n + 63) / 64;
+  // the next tile's inputs are loaded while this one computes
+  MlpIn next = mlp_load_tile(X, Tg, n, blockIdx.x * 64 + w * 16);
   for (int bt = blockIdx.x; bt < ntiles; bt += gridDim.x) {
     const int m0 = bt * 64 + w * 16;
+    const MlpIn in = next;
+    if (bt + (int)gridDim.x < ntiles) next = mlp_load_tile(X, Tg, n, (bt + gridDim.x) * 64 + w * 16);
     MlpTile T;
-    mlp_forward_tile(X, n, m0, prm, pk, lds[w], T);
+    mlp_forward_tile(in, C, wl, lds[w], T);
     // dL/dy
     float dy[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int m = m0 + 4 * q + j;
-      const float e = m < n ? T.y[j] - Tg[m] : 0.0f;
+      const float e = m < n ? T.y[j] - in.y[j] : 0.0f;
       dy[j] = m < n ? 2.0f * lw * e : 0.0f;
       if (c == 0) loss += lw * e * e;
       if (c == 0) gb4 += dy[j];
@@ -386,11 +431,11 @@ __global__ void __launch_bounds__(kBlock) k_mlp_train(const float* __restrict__ 
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         gw4[nt] += dy[j] * bf2f(T.h[2][nt][j]);
-        const float d = T.z[2][nt][j] > 0.0f ? dy[j] * w4b[nt] : 0.0f;
+        const float d = T.z[2][nt][j] > 0.0f ? dy[j] * C.w4[nt] : 0.0f;
         dz[nt][j] = d;
-        dzb[nt][j] = f2bf(d);
         gb3[nt] += d;
       }
+      dzb[nt] = f2bf4(dz[nt][0], dz[nt][1], dz[nt][2], dz[nt][3]);
     }
     // layers 3, 2, 1
 #pragma unroll
@@ -413,26 +458,21 @@ __global__ void __launch_bounds__(kBlock) k_mlp_train(const float* __restrict__ 
       for (int nt = 0; nt < 4; ++nt) {
         float4v acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int kt = 0; kt < 4; ++kt) acc = mfma16(a[kt], pk[pkb + (kt * 4 + nt) * 64 + l], acc);
+        for (int kt = 0; kt < 4; ++kt) acc = mfma16(a[kt], wl[pkb + (kt * 4 + nt) * 64 + l], acc);
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           const float d = T.z[L - 1][nt][j] > 0.0f ? acc[j] : 0.0f;
           dz[nt][j] = d;
-          dzb[nt][j] = f2bf(d);
           if (L == 2)
             gb2[nt] += d;
           else
             gb1[nt] += d;
         }
+        dzb[nt] = f2bf4(dz[nt][0], dz[nt][1], dz[nt][2], dz[nt][3]);
       }
     }
     // dW1 += X^T dZ1: X in C layout (rows 4q+j, column c)
-    short4v xc;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int m = m0 + 4 * q + j;
-      xc[j] = f2bf(m < n ? X[(int64_t)m * kFin + c] : 0.0f);
-    }
+    const short4v xc = f2bf4(in.t[0], in.t[1], in.t[2], in.t[3]);
 #pragma unroll
     for (int nt = 0; nt < 4; ++nt) gW1[nt] = mfma16(xc, dzb[nt], gW1[nt]);
   }
@@ -442,16 +482,14 @@ __global__ void __launch_bounds__(kBlock) k_mlp_train(const float* __restrict__ 
   float* out = gpart + (int64_t)blockIdx.x * kNumParams;
   float* r = red[w];
   // Helper lambdas write this wave's contribution of a [rows x 64] matrix
-  // chunk into r (indexed by row*64 + col), then wave 0 sums.
+  // chunk into r (indexed by row*64 + col), then all threads sum.
   auto reduce_chunk = [&](int count, int dst) {
     __syncthreads();
-    if (w == 0) {
-      for (int k = l; k < count; k += 64) {
-        float v = red[0][k] + red[1][k];
-        v = v + red[2][k];
-        v = v + red[3][k];
-        out[dst + k] = v;
-      }
+    for (int k = threadIdx.x; k < count; k += kBlock) {
+      float v = red[0][k] + red[1][k];
+      v = v + red[2][k];
+      v = v + red[3][k];
+      out[dst + k] = v;
     }
     __syncthreads();
   };
@@ -592,9 +630,12 @@ extern "C" int dsph_mlp_pack(const float* params, void* packed, void* stream) {
   return launch_status();
 }
 
+// One training workgroup per CU (its weight gradients fill the registers):
+// more of them run one after the other, and each pays the weights' staging
+// and the reduction of its 9473 partial gradients.
 static int mlp_grid(int64_t n) {
   int64_t tiles = (n + 63) / 64;
-  int64_t g = tiles < 1024 ? tiles : 1024;
+  int64_t g = tiles < 256 ? tiles : 256;
   return (int)(g < 1 ? 1 : g);
 }
 
