@@ -101,6 +101,33 @@ struct PrepNb {
   float h, vol, c2;
 };
 
+// alpha, divergence source and viscosity of row i from its sums: k1 x / y, k2,
+// divergence, viscosity x / y.
+__device__ __forceinline__ void finish_prepare(const PrepArgs& A, int i, float hi, const float (&s6)[6],
+                                               float* __restrict__ alpha_div, float* __restrict__ alpha_den,
+                                               float* __restrict__ div_src, float2* __restrict__ visc_acc) {
+  const float Vi = A.vol[i];
+  const float mass_i = A.areas[i] * A.rho0;
+  const float k1sq = s6[0] * s6[0] + s6[1] * s6[1];
+  {
+    const float fac = -A.dt2 * Vi;
+    alpha_den[i] = fac / mass_i * k1sq + fac * s6[2];
+  }
+  {
+    const float fac = -A.dt * Vi;
+    alpha_div[i] = fac / mass_i * k1sq + fac * s6[2];
+  }
+  div_src[i] = s6[3];
+  if (A.visc_on && visc_acc) {
+    float s;
+    if (A.visc_scheme == 0)
+      s = A.visc_alpha * hi * A.visc_cs * A.visc_rho0 / A.rho[i];
+    else
+      s = A.visc_factor / A.rho[i];
+    visc_acc[i] = make_float2(s * s6[4], s * s6[5]);
+  }
+}
+
 // One row of the prepare pass: neighbors by index idx(k) and data src(j),
 // four entries' loads ahead of their sums (the sums run in entry order).
 template <class Idx, class Src>
@@ -155,26 +182,8 @@ __device__ __forceinline__ void prepare_row(const PairsDev& P, const PrepArgs& A
     for (int u = 0; u < 4; ++u) body(k + u * rr.step, d[u]);
   }
   for (; n < rr.cnt; ++n, k += rr.step) body(k, src(idx(k)));
-  const float Vi = A.vol[i];
-  const float mass_i = A.areas[i] * A.rho0;
-  const float k1sq = k1x * k1x + k1y * k1y;
-  {
-    const float fac = -A.dt2 * Vi;
-    alpha_den[i] = fac / mass_i * k1sq + fac * k2;
-  }
-  {
-    const float fac = -A.dt * Vi;
-    alpha_div[i] = fac / mass_i * k1sq + fac * k2;
-  }
-  div_src[i] = dv;
-  if (A.visc_on && visc_acc) {
-    float s;
-    if (A.visc_scheme == 0)
-      s = A.visc_alpha * hi * A.visc_cs * A.visc_rho0 / A.rho[i];
-    else
-      s = A.visc_factor / A.rho[i];
-    visc_acc[i] = make_float2(s * vsx, s * vsy);
-  }
+  const float sums[6] = {k1x, k1y, k2, dv, vsx, vsy};
+  finish_prepare(A, i, hi, sums, alpha_div, alpha_den, div_src, visc_acc);
 }
 
 // The neighbor data of particle j from the global arrays.
@@ -229,6 +238,78 @@ __global__ void __launch_bounds__(kBlock) k_dfsph_prepare_tiled(PairsDev P, Prep
     prepare_row(
         P, A, i, [&](int k) { return P.nbr[k]; }, [&](int j) { return prep_nb(P, A, j); }, alpha_div, alpha_den,
         div_src, visc_acc, kv_out);
+}
+
+// The prepare pass of few rows (uniform support): kLanes lanes per row, in row
+// order, with the forms of near_math.h (pair_geom for a group out of their
+// range).  2304 rows: 29.8 us over tiles, now 7.0.
+struct PrepAt {
+  PrepNb d;
+  int at;
+};
+template <int kLanes>
+__global__ void __launch_bounds__(kBlock) k_dfsph_prepare_lanes(PairsDev P, PrepArgs A, float* __restrict__ alpha_div,
+                                                                float* __restrict__ alpha_den,
+                                                                float* __restrict__ div_src,
+                                                                float2* __restrict__ visc_acc,
+                                                                float* __restrict__ kv_out) {
+  const int row = (int)((blockIdx.x * (unsigned)kBlock + threadIdx.x) / kLanes);
+  const bool valid = row < P.nq;
+  const int i = valid ? row : P.nq - 1;
+  const float2 xi = P.qpos[i];
+  const float2 vi = A.vel[i];
+  const float h = P.h0;
+  const KConst kc = kconst(h);
+  const float eps = A.visc_eps * h * h;
+  RowRef rr = row_ref(P, i);
+  if (!valid) rr.cnt = 0;
+  constexpr int U = 4;
+  float acc[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  sum_row<kLanes, U>(
+      P.nbr, rr, i, acc, [&](int j, int at) { return PrepAt{prep_nb(P, A, j), at}; },
+      [&](const PrepAt(&e)[U], float(&t)[U][6]) {
+        float dx[U], dy[U];
+        Geom g[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          dx[u] = xi.x - e[u].d.x.x;
+          dy[u] = xi.y - e[u].d.x.y;
+        }
+        wrap_offsets(dx, dy, P.dom);
+        NearRange range;
+#pragma unroll
+        for (int u = 0; u < U; ++u) g[u] = pair_geom_near(dx[u], dy[u], h, kc, range);
+        if (range.odd()) {
+#pragma unroll
+          for (int u = 0; u < U; ++u) g[u] = pair_geom(xi, e[u].d.x, h, kc, P.dom);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const PrepNb& d = e[u].d;
+          const float s = dfsph_t(g[u]);
+          const float sv = d.vol * s;
+          const float kx = g[u].dx * sv, ky = g[u].dy * sv;
+          if (kv_out && e[u].at >= 0) kv_out[e[u].at] = sv;
+          t[u][0] = kx;
+          t[u][1] = ky;
+          const float gx = g[u].dx * s, gy = g[u].dy * s;
+          t[u][2] = d.c2 * (gx * gx + gy * gy);
+          t[u][3] = (d.v.x - vi.x) * kx + (d.v.y - vi.y) * ky;
+          t[u][4] = t[u][5] = 0.f;
+          if (A.visc_on) {
+            const float vx = vi.x - d.v.x, vy = vi.y - d.v.y;
+            const float rij = g[u].q * h;
+            const float vr = vx * g[u].ex + vy * g[u].ey;
+            float pi = vr / (rij + eps);
+            if (A.pi_switch) pi = vr < 0.0f ? pi : 0.0f;
+            const float f = d.vol * pi;
+            t[u][4] = f * g[u].gx;
+            t[u][5] = f * g[u].gy;
+          }
+        }
+      });
+  if (!valid || (threadIdx.x & (kLanes - 1)) != 0) return;
+  finish_prepare(A, i, h, acc, alpha_div, alpha_den, div_src, visc_acc);
 }
 
 // Source of a solve with advection adv (may be NULL = 0): div(v*) with
@@ -1084,6 +1165,27 @@ __device__ __forceinline__ void sweep_row_lanes(const PairsDev& P, const float* 
       });
 }
 
+// The divergence source of few rows from the (x, y, v*) records.
+template <int kLanes>
+__global__ void __launch_bounds__(kBlock) k_dfsph_source_lanes(PairsDev P, const float* __restrict__ kv,
+                                                               const float4* __restrict__ rec,
+                                                               const float* __restrict__ vol,
+                                                               const float* __restrict__ areas, float dt, int density,
+                                                               float* __restrict__ src) {
+  const int row = (int)((blockIdx.x * (unsigned)kBlock + threadIdx.x) / kLanes);
+  const bool valid = row < P.nq;
+  const int i = valid ? row : P.nq - 1;
+  RowRef rr = row_ref(P, i);
+  if (!valid) rr.cnt = 0;
+  const float4 own = rec[i];
+  float acc[1] = {0.f};
+  sweep_row_lanes<kLanes>(P, kv, rr, i, rec, acc, [&](const float4& r, float cx, float cy, float(&t)[1]) {
+    t[0] = (r.z - own.z) * cx + (r.w - own.w) * cy;
+  });
+  if (!valid || (threadIdx.x & (kLanes - 1)) != 0) return;
+  src[i] = density ? (1.0f - areas[i] / vol[i]) - dt * acc[0] : acc[0];
+}
+
 template <int kLanes>
 __global__ void __launch_bounds__(kBlock) k_dfsph_sweep_a_lanes(PairsDev P, SweepAArgs A, const SolveCtrl* ctrl) {
   if (ctrl && ctrl->done) return;
@@ -1148,7 +1250,7 @@ __global__ void __launch_bounds__(kBlock* kSweepBLanes) k_dfsph_sweep_b_lanes(Pa
 // against tiles: 2.3k rows 4.8 + 11.0 / 16.4 + 16.5, 8.1k 5.9 + 11.4 / 16.4 +
 // 16.7, 33k 8.8 + 11.2 / 16.4 + 16.7, 131k 15.2 + 15.8 / 20.6 + 21.1; A with
 // 16 lanes against 4: 16k 7.6 / 7.4, 33k 12.0 / 8.8.
-constexpr int kSweepA16 = 1 << 13, kSweepLanes = 1 << 17;
+constexpr int kSweepA16 = kLanes16Rows, kSweepLanes = kLanes4Rows;
 
 // Sweep launches: lanes per row for few rows, else over neighbor tiles when
 // the list carries them and the sweep gathers records.
@@ -1544,7 +1646,15 @@ extern "C" int dsph_dfsph_prepare(const dsph_pairs* pairs, const float* vel, con
   A.visc_eps = visc ? visc->eps : 0.f;
   A.pi_switch = visc ? visc->pi_switch : 0;
   A.visc_factor = visc ? (float)(2.0 * (2 + 2) * (double)visc->alpha * (double)visc->rho0) : 0.f;
-  if (P.tslot && !P.qh && !P.rh)
+  auto lanes = [&](auto kernel, int per_row) {
+    kernel<<<grid_for(P.nq, kBlock / per_row), kBlock, 0, as_stream(stream)>>>(
+        P, A, alpha_div, alpha_den, div_src, reinterpret_cast<float2*>(visc_acc), kgrad);
+  };
+  if (near_support(P) && P.nq == P.nr && P.nq <= kLanes16Rows)
+    lanes(k_dfsph_prepare_lanes<16>, 16);
+  else if (near_support(P) && P.nq == P.nr && P.nq <= kLanes4Rows)
+    lanes(k_dfsph_prepare_lanes<4>, 4);
+  else if (P.tslot && !P.qh && !P.rh)
     k_dfsph_prepare_tiled<<<grid_for(P.nq), kBlock, (size_t)P.tcap * (sizeof(float4) + sizeof(float2)),
                             as_stream(stream)>>>(P, A, alpha_div, alpha_den, div_src,
                                                  reinterpret_cast<float2*>(visc_acc), kgrad);
@@ -1603,7 +1713,15 @@ extern "C" int dsph_dfsph_solve(const dsph_pairs* pairs, const dsph_dfsph_params
                                         reinterpret_cast<const float2*>(adv), prm->dt, (int)n, xv);
       DSPH_LAUNCH_CHECK();
     }
-    if (P.tslot && kv && xv)
+    auto lanes = [&](auto kernel, int per_row) {
+      kernel<<<grid_for(P.nq, kBlock / per_row), kBlock, 0, st>>>(P, kv, xv, vol, areas, prm->dt,
+                                                                  prm->source_density, src);
+    };
+    if (kv && xv && P.nq <= kLanes16Rows)
+      lanes(k_dfsph_source_lanes<16>, 16);
+    else if (kv && xv && P.nq <= kLanes4Rows)
+      lanes(k_dfsph_source_lanes<4>, 4);
+    else if (P.tslot && kv && xv)
       k_dfsph_source_tiled<<<nb, kBlock, (size_t)P.tcap * sizeof(float4), st>>>(
           P, kv, reinterpret_cast<const float2*>(vel), reinterpret_cast<const float2*>(adv), vol, areas, prm->dt,
           prm->source_density, src, xv);

@@ -168,4 +168,8 @@ __device__ __forceinline__ void sum_row(const int32_t* __restrict__ nbr, const R
   }
 }
 
+// Lanes per row of the DFSPH passes: few rows are a matter of latency (their
+// figures stand at the passes), from 131k rows on the tiled forms fill the chip.
+constexpr int kLanes16Rows = 1 << 13, kLanes4Rows = 1 << 17;
+
 }  // namespace dsph

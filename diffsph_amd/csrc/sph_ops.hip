@@ -2,6 +2,7 @@
 // values are evaluated on the fly from positions (no per-pair arrays).
 // One thread per query particle, neighbors in CSR order, no atomics.
 #include "common.h"
+#include "near_math.h"
 
 namespace dsph {
 
@@ -110,11 +111,69 @@ __global__ void __launch_bounds__(kBlock) k_density_tiled(PairsDev P, const floa
   if (vol) vol[i] = qmass[i] / acc;
 }
 
-// The density launch: over neighbor tiles when the list carries them and
-// the support is uniform.
+// Density of few rows (uniform support): kLanes lanes per row, in row order,
+// with the square root of near_math.h.
+struct NbrXM {
+  float2 x;
+  float m;
+  int at;
+};
+template <int kLanes>
+__global__ void __launch_bounds__(kBlock) k_density_lanes(PairsDev P, const float* __restrict__ rmass,
+                                                          const float* __restrict__ qmass, float* __restrict__ rho,
+                                                          float* __restrict__ vol, float* __restrict__ w_out) {
+  const int row = (int)((blockIdx.x * (unsigned)kBlock + threadIdx.x) / kLanes);
+  const bool valid = row < P.nq;
+  const int i = valid ? row : P.nq - 1;
+  const float2 xi = P.qpos[i];
+  const KConst kk = kconst(P.h0);
+  RowRef rr = row_ref(P, i);
+  if (!valid) rr.cnt = 0;
+  float acc[1] = {0.f};
+  // entries past the row's end read particle 0 (their terms are dropped)
+  sum_row<kLanes, 4>(
+      P.nbr, rr, 0, acc, [&](int j, int at) { return NbrXM{P.rpos[j], rmass[j], at}; },
+      [&](const NbrXM(&d)[4], float(&t)[4][1]) {
+        float dx[4], dy[4], d2[4], r[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          dx[u] = xi.x - d[u].x.x;
+          dy[u] = xi.y - d[u].x.y;
+        }
+        wrap_offsets(dx, dy, P.dom);
+        NearRange range;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          d2[u] = dist2_exact(dx[u], dy[u]);
+          range.d2(d2[u]);
+          r[u] = sqrt_near(d2[u]);
+        }
+        if (range.odd()) {
+#pragma unroll
+          for (int u = 0; u < 4; ++u) r[u] = sqrt_rn(d2[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const float w = wendland_w(r[u] * kk.ih, kk);
+          if (w_out && d[u].at >= 0) w_out[d[u].at] = w;
+          t[u][0] = d[u].m * w;
+        }
+      });
+  if (!valid || (threadIdx.x & (kLanes - 1)) != 0) return;
+  rho[i] = acc[0];
+  if (vol) vol[i] = qmass[i] / acc[0];
+}
+
+// The density launch: lanes per row for few rows (2304 rows: 24.8 us over
+// tiles, now about 5), else over neighbor tiles when the list carries them,
+// both for a uniform support.
 static void launch_density(const PairsDev& P, const float* rmass, const float* qmass, float* rho, float* vol,
                            float* w_out, hipStream_t st) {
-  if (P.tslot && !P.qh && !P.rh)
+  if (near_support(P) && P.nq <= kLanes16Rows)
+    k_density_lanes<16><<<grid_for(P.nq, kBlock / 16), kBlock, 0, st>>>(P, rmass, qmass, rho, vol, w_out);
+  else if (near_support(P) && P.nq <= kLanes4Rows)
+    k_density_lanes<4><<<grid_for(P.nq, kBlock / 4), kBlock, 0, st>>>(P, rmass, qmass, rho, vol, w_out);
+  else if (P.tslot && !P.qh && !P.rh)
     k_density_tiled<<<grid_for(P.nq), kBlock, (size_t)P.tcap * sizeof(float4), st>>>(P, rmass, qmass, rho, vol,
                                                                                       w_out);
   else

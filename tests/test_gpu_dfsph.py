@@ -63,6 +63,24 @@ def test_dfsph_steps_match_oracle(orc, nside, seed, steps):
         assert abs(stats.den_error - info["err_den"]) <= 1e-6 * max(1e-12, abs(info["err_den"])) + 1e-9
 
 
+# 16 lanes per row, 4 lanes (from 8193 rows), and the tiled passes (from 131073)
+@pytest.mark.parametrize("nside", [33, 91, 131, 363])
+def test_dfsph_lane_passes_equal_oracle_bits(orc, nside):
+    d, dt = _setup(nside, 5, 0.4)
+    print(f"case nside={nside}", flush=True)
+    s = _solver(d, dt, min_iters=3, max_iters=3)
+    dom = orc.make_domain((-1, -1), (1, 1), (True, True))
+    n = d["pos"].shape[0]
+    ost = orc.DfsphState(d["pos"].copy(), d["vel"].copy(), d["mass"].copy(), d["area"].copy(),
+                         np.arange(n, dtype=np.int32))
+    s.step()
+    ost, info = orc.dfsph_step(ost, dom, d["h"], dt, min_iters=3, max_iters=3)
+    for name, gpu, ref in [("rho", s.rho, info["rho"]), ("alpha_den", s.alpha_den, info["alpha_den"]),
+                           ("visc", s.visc, info["visc"]), ("p_div", s.p_div, info["p_div"]),
+                           ("p_den", s.p_den, info["p_den"]), ("vel", s.vel, ost.vel), ("pos", s.pos, ost.pos)]:
+        np.testing.assert_array_equal(gpu.cpu().numpy(), ref, err_msg=name)
+
+
 def test_dfsph_1m_steps_match_oracle(orc):
     """The 1M-particle headline workload (1024^2, seed 0) through the HIP
     path against the oracle: the first step (p = 0 warm start) and the
