@@ -166,8 +166,9 @@ __global__ void __launch_bounds__(kBlock) k_bscatter(int n, const int32_t* __res
   order[cell_start[keys[i]] + slot[i]] = i;
 }
 
-// The final order, by particle index within each cell (cell_rank); with
-// `dst`, dst[slot] = src[particle] in the same pass.
+// The final order, by particle index within each cell (cell_rank, cells of any
+// size: a batch has no report of an overfull one); with `dst`, dst[slot] =
+// src[particle] in the same pass.
 __global__ void __launch_bounds__(kBlock) k_bcellrank(int n, const int32_t* __restrict__ keys,
                                                       const int32_t* __restrict__ slot,
                                                       const int32_t* __restrict__ cell_start,
@@ -175,7 +176,7 @@ __global__ void __launch_bounds__(kBlock) k_bcellrank(int n, const int32_t* __re
                                                       const float2* __restrict__ src, float2* __restrict__ dst) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  const int p = cell_rank(i, keys[i], slot, cell_start, order);
+  const int p = cell_rank(i, keys[i], slot, cell_start, order, INT32_MAX);
   si[p] = i;
   if (dst) dst[p] = src[i];
 }

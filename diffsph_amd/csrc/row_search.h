@@ -94,12 +94,13 @@ struct LaneTest {
 // count of smaller indices among its particles order[cell_start[key] ..].  One
 // thread per particle with eight loads in flight; one thread per cell (a
 // serial sort of 16 to 36 entries) took 14 us at 4k particles and 365 us on a
-// grid of 36 a cell.  A cell over DSPH_CELL_MAX stays in provisional order (a
-// diverged state: the search reports it).
+// grid of 36 a cell.  A cell of more than `longest` particles stays in
+// provisional order.
 __device__ __forceinline__ int cell_rank(int i, int key, const int32_t* __restrict__ slot,
-                                         const int32_t* __restrict__ cell_start, const int32_t* __restrict__ order) {
+                                         const int32_t* __restrict__ cell_start, const int32_t* __restrict__ order,
+                                         int longest) {
   const int b = cell_start[key], e = cell_start[key + 1];
-  if (e - b > DSPH_CELL_MAX) return b + slot[i];
+  if (e - b > longest) return b + slot[i];
   int r = 0;
   for (int a = b; a < e; a += 8) {
     int v[8];

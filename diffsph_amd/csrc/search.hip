@@ -62,7 +62,8 @@ __global__ void __launch_bounds__(kBlock) k_cell_scatter(int n, const int32_t* _
 
 // The final order, by original index within each cell: particle i goes to its
 // rank in the cell (cell_rank, row_search.h), with its sorted position,
-// support and rank in the same pass.
+// support and rank in the same pass.  A cell over DSPH_CELL_MAX is a diverged
+// state that the search reports: it is left unranked.
 __global__ void __launch_bounds__(kBlock) k_cell_rank(int n, Dom d, const int32_t* __restrict__ keys,
                                                       const int32_t* __restrict__ slot,
                                                       const int32_t* __restrict__ cell_start,
@@ -72,7 +73,7 @@ __global__ void __launch_bounds__(kBlock) k_cell_rank(int n, Dom d, const int32_
                                                       float* __restrict__ sh, int32_t* __restrict__ rank) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  const int p = cell_rank(i, keys[i], slot, cell_start, order);
+  const int p = cell_rank(i, keys[i], slot, cell_start, order, DSPH_CELL_MAX);
   const float2 x = pos[i];
   sort_index[p] = i;
   spos[p] = make_float2(wrap_coord(x.x, d, 0), wrap_coord(x.y, d, 1));

@@ -116,6 +116,25 @@ def test_batched_width_overflow_is_reported():
     assert b.status() == (0, 0)
 
 
+def test_batched_crowded_cell_is_sorted_by_index():
+    """A cell far beyond the usual occupancy (5000 particles) is ranked in
+    full: its particles keep their input order, whatever order the histogram
+    atomics arrived in."""
+    B = _batched()
+    ens = B.make_ensemble(sizes=[90, 33], dx=DX, seed=2, device="cuda")
+    heavy = torch.cat([torch.arange(0, 3000, 3), torch.arange(3000, 7000)]).cuda()
+    lo = torch.tensor(ens.boxes[0][0], device="cuda", dtype=torch.float32)
+    ens.pos[heavy] = lo + 0.3 * ens.cfg.support + 1e-3 * DX * torch.rand(heavy.numel(), 2, device="cuda")
+    print(f"crowded cell: {heavy.numel()} particles", flush=True)
+    assert heavy.numel() > 4096
+    b = B.BatchedDeltaSPH(ens.boxes, ens.counts, ens.pos, ens.vel, ens.mass, ens.rho, replace(ens.cfg, dt=1e-9),
+                          width=64)
+    b.step(1)
+    uid = b.uid.cpu().numpy()
+    mine = uid[np.isin(uid, heavy.cpu().numpy())]
+    np.testing.assert_array_equal(mine, heavy.cpu().numpy())
+
+
 def test_batched_autotune_returns_measured_candidate():
     B = _batched()
     ens = B.make_ensemble(sizes=[30, 45, 60], dx=DX, seed=2, device="cuda")
