@@ -212,7 +212,7 @@ __global__ void __launch_bounds__(kBlock) k_bpermute(int n, const int32_t* __res
 // 7.8M particles, and only dsph_batch_probe reads it).  A wave takes the rows
 // of one cell together (row_search.h); the first `depth` entries are staged in LDS and written
 // column by column, whole lines at a time, as in the single-domain fill.
-template <int kRows, int kTurns>
+template <int kRows, int kTurns, bool kMaySparse>
 __global__ void __launch_bounds__(kBlock) k_bfill(int n, const int32_t* __restrict__ dom_of,
                                                   const Dom* __restrict__ doms, const BGrid* __restrict__ grids,
                                                   const float2* __restrict__ q, const float2* __restrict__ spos,
@@ -276,21 +276,21 @@ __global__ void __launch_bounds__(kBlock) k_bfill(int n, const int32_t* __restri
     const int own = r0 + (lane < kMine ? lane : 0);
     const float2 mine = qs[own];
     const int cell = lane < kMine ? cells[own] : -1;
-    auto d2 = [&](const float2& x, int k, bool seam) {
-      float dx = lane_value(mine.x, k) - x.x, dy = lane_value(mine.y, k) - x.y;
+    auto d2 = [&](const float2& x, const auto& qk, bool seam) {
+      float dx = qk.x() - x.x, dy = qk.y() - x.y;
       if (seam) {
-        const Dom d = doms[ds[r0 + k]];
+        const Dom d = doms[ds[r0 + qk.k]];
         dx = mod_offset(dx, d, 0);
         dy = mod_offset(dy, d, 1);
       }
       return dist2_exact(dx, dy);
     };
-    const int mine_found = scan_rows_by_cell(
-        (uint32_t)__builtin_amdgcn_ballot_w64(cell >= 0), cell, depth,
-        [&](int p, int k) { return rows[p][r0 + k]; }, [&](int j) { return spos[j]; },
-        [](int, int, bool, int j) { return j; },
-        [&](const float2& x, int k, bool seam) { return within(d2(x, k, seam)); },
-        [&](const float2& x, int k, bool seam) { return within.exact(d2(x, k, seam)); },
+    const int mine_found = scan_rows<kMine, false, kMaySparse>(
+        cell, depth, [&](int p, int k) { return rows[p][r0 + k]; },
+        WaveQuery{mine.x, mine.y, 0.f, 0},
+        [&](int j) { return spos[j]; }, [](int, int, bool, int j) { return j; },
+        [&](const float2& x, const auto& qk, bool seam) { return within(d2(x, qk, seam)); },
+        [&](const float2& x, const auto& qk, bool seam) { return within.exact(d2(x, qk, seam)); },
         [&](int k, int pos, int j) { stage[__umul24(pos, kRows + 1) + r0 + k] = j; },
         [&](int k, int pos, int j) {
           const int i = i0 + r0 + k;
@@ -506,10 +506,13 @@ int fill_rows(const Ctx& c, const float2* q, const float2* spos, const int32_t* 
         c.b->support, c.b->width, depth, c.p<int32_t>(L.nbr), c.p<int32_t>(L.cnt), c.p<int32_t>(L.status),
         count_pairs);
   };
+  // the path for sparse cells takes ~20 registers (two waves per SIMD): left
+  // out where the mean cell is too full for it
+  const bool may = (int64_t)c.n * 9 < (int64_t)c.ncell * kSparse;
   if (c.n < kRowSmall)
-    launch(k_bfill<16, 1>, 16, 1);
+    may ? launch(k_bfill<16, 1, true>, 16, 1) : launch(k_bfill<16, 1, false>, 16, 1);
   else
-    launch(k_bfill<64, 4>, 64, 4);
+    may ? launch(k_bfill<64, 4, true>, 64, 4) : launch(k_bfill<64, 4, false>, 64, 4);
   return launch_status();
 }
 

@@ -34,6 +34,12 @@ constexpr int kRowStage = 128;  // deepest staged row of the layouts without a f
 // 72 / 46).
 constexpr int kRowSmall = 1 << 15;
 
+// Candidates of a query (its three cell rows) up to which its wave takes
+// scan_rows_sparse: 9 cells of 5 to 10.  Count and CSR fill in us, queries in
+// cell order, bounds of 48 / 96 / 128: 1M at 5 a cell 85 + 181 / 60 + 93 / -,
+// 1M at 16 a cell 88 + 206 / 88 + 207 / 90 + 206 (144 candidates: above).
+constexpr int kSparse = 96;
+
 // The candidates of one row of cells, at most two runs of sorted slots (two
 // when the row wraps around the periodic x boundary), in scan order.  `len1`
 // carries the seam flag: pairs of these ranges may cross a periodic seam.
@@ -139,23 +145,45 @@ __device__ __forceinline__ unsigned long long first_lanes(int n) {
   return n >= 64 ? ~0ull : (n <= 0 ? 0ull : (1ull << n) - 1ull);
 }
 
+// Query k of the wave (the same k in all lanes) whose values lie in lane k, as
+// scalars where they are used.
+struct WaveQuery {
+  float vx, vy, vh;
+  int k;
+  __device__ __forceinline__ float x() const { return lane_value(vx, k); }
+  __device__ __forceinline__ float y() const { return lane_value(vy, k); }
+  __device__ __forceinline__ float h() const { return lane_value(vh, k); }
+};
+
+// The query of this lane.
+struct LaneQuery {
+  float vx, vy, vh;
+  int k;
+  __device__ __forceinline__ float x() const { return vx; }
+  __device__ __forceinline__ float y() const { return vy; }
+  __device__ __forceinline__ float h() const { return vh; }
+};
+
 // The neighbor rows of the queries in `todo` (bit k: the query of lane k,
 // k < 32, whose cell is `cell` there); returns each query's row length in its
-// lane.  rows(p, k): cell row p = 0..2 of query k; load(j): candidate j;
+// lane.  mine: the query of this lane (lanes without one: any); rows(p, k):
+// cell row p = 0..2 of query k; load(j): candidate j;
 // value(p, k, first, j): what a row gets for candidate j of cell row p of the
-// queries in query k's cell (first: of its first range); test(c, k, seam): a
-// LaneTest of every lane's candidate c against query k (uniform), exact(c, k,
-// seam) the expression itself; put(k, pos, value): entry pos < depth of row
-// k, spill(k, pos, value): entry pos >= depth.  All 64 lanes call it; no
+// queries in query k's cell (first: of its first range); test(c, q, seam): a
+// LaneTest of every lane's candidate c against its query q (WaveQuery or
+// LaneQuery), exact(c, q, seam) the expression itself; put(k, pos, value): entry pos < depth of row
+// k, spill(k, pos, value): entry pos >= depth (kDirect: every entry).  All 64 lanes call it; no
 // barrier inside.
 //
 // Vector and scalar issue are about equal here (~35 and ~33 a row), so the
 // masks of a row's three cell rows are formed first and the checks that are
 // rarely true (a pair in the band, a row past `depth`) made once per row.
-template <class Rows, class Load, class Value, class Test, class Exact, class Put, class Spill>
+template <bool kDirect, class Rows, class Load, class Value, class Test, class Exact, class Put,
+          class Spill>
 __device__ __forceinline__ int scan_rows_by_cell(uint32_t todo, int cell, int depth, const Rows& rows,
-                                                 const Load& load, const Value& value, const Test& test,
-                                                 const Exact& exact, const Put& put, const Spill& spill) {
+                                                 const WaveQuery& own, const Load& load, const Value& value,
+                                                 const Test& test, const Exact& exact, const Put& put,
+                                                 const Spill& spill) {
   using Cand = decltype(load(0));
   const int lane = threadIdx.x & 63;
   int found = 0;
@@ -181,12 +209,13 @@ __device__ __forceinline__ int scan_rows_by_cell(uint32_t todo, int cell, int de
     auto place_of = [](unsigned long long m, int n) {
       return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, n));
     };
-    auto decide = [&](LaneTest t, const Cand& cd, int k, bool at_seam) {
-      return t.in | (__builtin_amdgcn_ballot_w64(exact(cd, k, at_seam)) & t.band);
+    auto decide = [&](LaneTest t, const Cand& cd, const auto& q, bool at_seam) {
+      return t.in | (__builtin_amdgcn_ballot_w64(exact(cd, q, at_seam)) & t.band);
     };
     // one query, candidates read as they come: any cell row
-    auto general = [&](int k, bool stage) {
+    auto general = [&](int k) {
       int n = 0;
+      const WaveQuery qk{own.vx, own.vy, own.vh, k};
       for (int p = 0; p < 3; ++p) {
         const CellRow v = rows(p, f);
         const int b0 = __builtin_amdgcn_readfirstlane(v.b0), l0 = __builtin_amdgcn_readfirstlane(v.len0);
@@ -196,12 +225,12 @@ __device__ __forceinline__ int scan_rows_by_cell(uint32_t todo, int cell, int de
         for (int t0 = 0; t0 < total; t0 += 64) {
           const int t = t0 + lane, j = t + (t < l0 ? b0 : b1 - l0);
           const Cand cd = load(t < total ? j : 0);
-          const unsigned long long m = decide(test(cd, k, at_seam), cd, k, at_seam) & first_lanes(total - t0);
+          const unsigned long long m = decide(test(cd, qk, at_seam), cd, qk, at_seam) & first_lanes(total - t0);
           const int pos = place_of(m, n);
           if (__builtin_amdgcn_inverse_ballot_w64(m)) {
-            if (pos >= depth)
+            if (kDirect || pos >= depth)
               spill(k, pos, value(p, k, t < l0, j));
-            else if (stage)
+            else
               put(k, pos, value(p, k, t < l0, j));
           }
           n += __popcll(m);
@@ -230,6 +259,7 @@ __device__ __forceinline__ int scan_rows_by_cell(uint32_t todo, int cell, int de
       while (same) {
         const int k = __ffs(same) - 1;
         same &= same - 1;
+        const WaveQuery qk{own.vx, own.vy, own.vh, k};
         unsigned long long m[3][NC];
         unsigned long long band = 0;
 #pragma unroll
@@ -237,7 +267,7 @@ __device__ __forceinline__ int scan_rows_by_cell(uint32_t todo, int cell, int de
 #pragma unroll
           for (int q = 0; q < NC; ++q) {
             const unsigned long long live = first_lanes(tot[p] - q * 64);
-            const LaneTest t = test(cand[p][q], k, kSeam && (R[p].len1 & kSeamBit));
+            const LaneTest t = test(cand[p][q], qk, kSeam && (R[p].len1 & kSeamBit));
             m[p][q] = t.in & live;
             band |= t.band & live;
           }
@@ -248,7 +278,7 @@ __device__ __forceinline__ int scan_rows_by_cell(uint32_t todo, int cell, int de
 #pragma unroll
             for (int q = 0; q < NC; ++q) {
               const bool at_seam = kSeam && (R[p].len1 & kSeamBit);
-              m[p][q] = decide(test(cand[p][q], k, at_seam), cand[p][q], k, at_seam) & first_lanes(tot[p] - q * 64);
+              m[p][q] = decide(test(cand[p][q], qk, at_seam), cand[p][q], qk, at_seam) & first_lanes(tot[p] - q * 64);
             }
           }
         }
@@ -259,8 +289,8 @@ __device__ __forceinline__ int scan_rows_by_cell(uint32_t todo, int cell, int de
           for (int q = 0; q < NC; ++q) n += __popcll(m[p][q]);
         }
         found = lane == k ? n : found;
-        if (n > depth) {
-          general(k, true);
+        if (!kDirect && n > depth) {
+          general(k);
           continue;
         }
         n = 0;
@@ -269,7 +299,12 @@ __device__ __forceinline__ int scan_rows_by_cell(uint32_t todo, int cell, int de
 #pragma unroll
           for (int q = 0; q < NC; ++q) {
             const int pos = place_of(m[p][q], n);
-            if (__builtin_amdgcn_inverse_ballot_w64(m[p][q])) put(k, pos, val[p][q]);
+            if (__builtin_amdgcn_inverse_ballot_w64(m[p][q])) {
+              if (kDirect)
+                spill(k, pos, val[p][q]);
+              else
+                put(k, pos, val[p][q]);
+            }
             n += __popcll(m[p][q]);
           }
         }
@@ -282,7 +317,7 @@ __device__ __forceinline__ int scan_rows_by_cell(uint32_t todo, int cell, int de
       while (same) {
         const int k = __ffs(same) - 1;
         same &= same - 1;
-        const int n = general(k, true);
+        const int n = general(k);
         found = lane == k ? n : found;
       }
     } else if (longest > 64) {
@@ -297,6 +332,90 @@ __device__ __forceinline__ int scan_rows_by_cell(uint32_t todo, int cell, int de
     }
   }
   return found;
+}
+
+// scan_rows_by_cell for queries whose cell rows hold few candidates (up to
+// kSparse each): all kMine queries of the wave at once, 64 / kMine lanes each
+// over the candidates of the three cell rows end to end, four loads in flight.
+// A cell's candidates in registers leave most lanes idle there, and its set-up
+// (~330 cycles) comes with every one or two queries.  1M queries in cell order,
+// count + CSR fill + fixed-width fill in us, by cell only / this: 0.5 a cell
+// 157 + 256 + 225 / 32 + 42 + 49, 2 a cell 120 + 228 + 186 / 42 + 60 + 65, 5 a
+// cell 92 + 204 + 156 / 60 + 93 + 89 (one thread per query: 29 + 45 + 47, 42 +
+// 72 + 72, 57 + 127 + 108).
+template <int kMine, bool kDirect, class Rows, class Load, class Value, class Test, class Exact, class Put,
+          class Spill>
+__device__ __forceinline__ int scan_rows_sparse(int end0, int end1, int total, bool seam, int depth, const Rows& rows,
+                                                const LaneQuery& q, const Load& load, const Value& value,
+                                                const Test& test, const Exact& exact, const Put& put,
+                                                const Spill& spill) {
+  constexpr int kLanes = 64 / kMine;
+  const int lane = threadIdx.x & 63, k = lane / kLanes, g = lane % kLanes;
+  int n = 0;
+  using Cand = decltype(load(0));
+  constexpr int U = 4;
+  for (int t0 = 0; __builtin_amdgcn_ballot_w64(t0 < total); t0 += U * kLanes) {
+    Cand c[U];
+    int p[U], j[U];
+    bool first[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int t = t0 + u * kLanes + g;
+      p[u] = t < end0 ? 0 : (t < end1 ? 1 : 2);
+      const CellRow v = rows(p[u], k);
+      const int w = t - (p[u] == 0 ? 0 : (p[u] == 1 ? end0 : end1));
+      first[u] = w < v.len0;
+      j[u] = w + (first[u] ? v.b0 : v.b1 - v.len0);
+      c[u] = load(t < total ? j[u] : 0);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const LaneTest in = test(c[u], q, seam);
+      unsigned long long m = in.in;
+      if (in.band) m |= __builtin_amdgcn_ballot_w64(exact(c[u], q, seam)) & in.band;
+      m &= __builtin_amdgcn_ballot_w64(t0 + u * kLanes + g < total);
+      const uint32_t mine = (uint32_t)(m >> (lane & ~(kLanes - 1))) & ((1u << kLanes) - 1u);
+      if ((mine >> g) & 1u) {
+        const int pos = n + __popc(mine & ((1u << g) - 1u));
+        if (kDirect || pos >= depth)
+          spill(k, pos, value(p[u], k, first[u], j[u]));
+        else
+          put(k, pos, value(p[u], k, first[u], j[u]));
+      }
+      n += __popc(mine);
+    }
+  }
+  return __shfl(n, (lane % kMine) * kLanes, 64);
+}
+
+// The neighbor rows of a wave's kMine queries, by whichever of the two suits
+// their candidates; arguments as for scan_rows_by_cell.
+template <int kMine, bool kDirect, bool kMaySparse, class Rows, class Load, class Value, class Test, class Exact,
+          class Put, class Spill>
+__device__ __forceinline__ int scan_rows(int cell, int depth, const Rows& rows, const WaveQuery& own, const Load& load,
+                                         const Value& value, const Test& test, const Exact& exact, const Put& put,
+                                         const Spill& spill) {
+  if constexpr (kMaySparse) {
+    const int k = (threadIdx.x & 63) / (64 / kMine);
+    int end[3], flags = 0, total = 0;
+#pragma unroll
+    for (int p = 0; p < 3; ++p) {
+      const CellRow v = rows(p, k);
+      total += v.len0 + (v.len1 & (kSeamBit - 1));
+      end[p] = total;
+      flags |= v.len1;
+    }
+    if (__builtin_amdgcn_ballot_w64(total > kSparse) == 0) {
+      // off a seam the min-image is the plain difference: all lanes take it
+      // when one needs it
+      const bool seam = __builtin_amdgcn_ballot_w64((flags & kSeamBit) != 0) != 0;
+      const LaneQuery q{__shfl(own.vx, k, 64), __shfl(own.vy, k, 64), __shfl(own.vh, k, 64), k};
+      return scan_rows_sparse<kMine, kDirect>(end[0], end[1], total, seam, depth, rows, q, load, value, test, exact,
+                                              put, spill);
+    }
+  }
+  const uint32_t todo = (uint32_t)__builtin_amdgcn_ballot_w64(cell >= 0);
+  return scan_rows_by_cell<kDirect>(todo, cell, depth, rows, own, load, value, test, exact, put, spill);
 }
 
 }  // namespace dsph

@@ -195,12 +195,12 @@ __device__ __forceinline__ void load_queries(const SearchArgs& a, int i0, Querie
 }
 
 // The rows of this wave's quarter of the workgroup's queries: value / put /
-// spill as scan_rows_by_cell takes them, with the row's number in the
+// spill as scan_rows takes them, with the row's number in the
 // workgroup; done(r, n): row r has n entries (one lane per row).  The
 // min-image is evaluated only for cell rows at a periodic seam (elsewhere the
 // plain difference is the offset).  kH: supports per particle (else the
 // uniform a.h0).
-template <int kRows, bool kH, class Value, class Put, class Spill, class Done>
+template <int kRows, bool kH, bool kDirect, class Value, class Put, class Spill, class Done>
 __device__ __forceinline__ void scan_queries(const SearchArgs& a, const Queries<kRows>& Q, int depth,
                                              const Value& value, const Put& put, const Spill& spill,
                                              const Done& done) {
@@ -210,36 +210,37 @@ __device__ __forceinline__ void scan_queries(const SearchArgs& a, const Queries<
   const int own = r0 + (lane < kMine ? lane : 0);
   const float qx = Q.x[own], qy = Q.y[own], qh = Q.h[own];
   const int cell = lane < kMine ? Q.cell[own] : -1;
-  const uint32_t todo = (uint32_t)__builtin_amdgcn_ballot_w64(cell >= 0);
   auto rows = [&](int p, int k) { return Q.rows[p][r0 + k]; };
+  const WaveQuery mine{qx, qy, qh, 0};
   auto val = [&](int p, int k, bool first, int j) { return value(p, r0 + k, first, j); };
   auto in = [&](int k, int pos, int v) { put(r0 + k, pos, v); };
   auto out = [&](int k, int pos, int v) { spill(r0 + k, pos, v); };
   int n;
   if (kH) {
-    auto keep = [&](const Cand& c, int k, bool seam) {
-      const float2 qi = make_float2(lane_value(qx, k), lane_value(qy, k));
-      const float hi = lane_value(qh, k);
-      return seam ? keep_pair(qi, hi, c.x, c.h, a) : keep_pair_near(qi, hi, c.x, c.h, a);
+    auto keep = [&](const Cand& c, const auto& q, bool seam) {
+      const float2 qi = make_float2(q.x(), q.y());
+      return seam ? keep_pair(qi, q.h(), c.x, c.h, a) : keep_pair_near(qi, q.h(), c.x, c.h, a);
     };
-    n = scan_rows_by_cell(
-        todo, cell, depth, rows, [&](int j) { return Cand{a.rpos[j], h_of(a.rh, j, a.h0)}; }, val,
-        [&](const Cand& c, int k, bool seam) { return LaneTest{__builtin_amdgcn_ballot_w64(keep(c, k, seam)), 0}; },
-        [](const Cand&, int, bool) { return false; }, in, out);
+    n = scan_rows<kMine, kDirect, true>(
+        cell, depth, rows, mine, [&](int j) { return Cand{a.rpos[j], h_of(a.rh, j, a.h0)}; }, val,
+        [&](const Cand& c, const auto& q, bool seam) {
+          return LaneTest{__builtin_amdgcn_ballot_w64(keep(c, q, seam)), 0};
+        },
+        [](const Cand&, const auto&, bool) { return false; }, in, out);
   } else {
     const NearTest within(a.h0);
-    auto d2 = [&](const float2& x, int k, bool seam) {
-      float dx = lane_value(qx, k) - x.x, dy = lane_value(qy, k) - x.y;
+    auto d2 = [&](const float2& x, const auto& q, bool seam) {
+      float dx = q.x() - x.x, dy = q.y() - x.y;
       if (seam) {
         dx = mod_offset(dx, a.d, 0);
         dy = mod_offset(dy, a.d, 1);
       }
       return dist2_exact(dx, dy);
     };
-    n = scan_rows_by_cell(
-        todo, cell, depth, rows, [&](int j) { return a.rpos[j]; }, val,
-        [&](const float2& x, int k, bool seam) { return within(d2(x, k, seam)); },
-        [&](const float2& x, int k, bool seam) { return within.exact(d2(x, k, seam)); }, in, out);
+    n = scan_rows<kMine, kDirect, true>(
+        cell, depth, rows, mine, [&](int j) { return a.rpos[j]; }, val,
+        [&](const float2& x, const auto& q, bool seam) { return within(d2(x, q, seam)); },
+        [&](const float2& x, const auto& q, bool seam) { return within.exact(d2(x, q, seam)); }, in, out);
   }
   if (cell >= 0) done(own, n);
 }
@@ -262,7 +263,7 @@ __global__ void __launch_bounds__(kBlock) k_neighbor_count(SearchArgs a, int32_t
   bool over = false;  // counted without the skipped ranges; the host checks the cells
   load_queries<kRows>(a, i0, Q, over, [](int, int, const CellRow&) {});
   __syncthreads();
-  scan_queries<kRows, kH>(
+  scan_queries<kRows, kH, false>(
       a, Q, INT32_MAX, [](int, int, bool, int) { return 0; }, [](int, int, int) {}, [](int, int, int) {},
       [&](int r, int n) { counts[i0 + r] = n; });
 }
@@ -336,15 +337,17 @@ struct FillOut {
 // the run of the candidate range, as ~j for a range outside the tile's runs
 // (tile_n = -1 then); a tile that does not fit T.cap (or kFillTileMax) is
 // filled without slots.
-template <int kRows, bool kTiles, bool kH>
+template <int kRows, bool kTiles, bool kH, bool kCsr>
 __global__ void __launch_bounds__(kBlock) k_neighbor_fill(SearchArgs a, FillOut F, FillTiles T) {
   extern __shared__ int32_t stage[];
   __shared__ Queries<kRows> Q;
   __shared__ int2 run_add[kTiles ? 3 : 1][kTiles ? kRows : 1];
   __shared__ int found[kRows];
   __shared__ int rt_s[kTileMaxRuns], rt_e[kTileMaxRuns], rt_d[kTileMaxRuns];
+  __shared__ int offs[kCsr ? kRows + 1 : 1];  // the rows' first entries
   const int i0 = blockIdx.x * kRows;
   const int tile = i0 / kBlock;
+  if (kCsr && threadIdx.x <= kRows) offs[threadIdx.x] = F.off[i0 + (int)threadIdx.x < a.nq ? i0 + threadIdx.x : a.nq];
   bool fit = false;
   int R = 0;
   if (kTiles) {
@@ -372,25 +375,25 @@ __global__ void __launch_bounds__(kBlock) k_neighbor_fill(SearchArgs a, FillOut 
   __syncthreads();
   const bool slots = kTiles && fit;
   auto row_of = [&](int i, int64_t& base, int64_t& step, int64_t& len) {
-    if (F.width > 0) {
+    if (kCsr) {
+      base = offs[i - i0];
+      step = 1;
+      len = (int64_t)offs[i - i0 + 1] - base;
+    } else if (F.width > 0) {
       base = (int64_t)(i >> 6) * 64 * F.width + (i & 63);
       step = 64;
       len = F.width;
-    } else if (F.slice) {
+    } else {
       const int s = i >> 6;
       base = (int64_t)F.slice[s] + (i & 63);
       step = 64;
       len = ((int64_t)F.slice[s + 1] - F.slice[s]) >> 6;
-    } else {
-      base = F.off[i];
-      step = 1;
-      len = (int64_t)F.off[i + 1] - F.off[i];
     }
   };
   // slot of the reference particle a staged value stands for
   auto ref_of = [&](int v) { return !slots ? v : (v >= 0 ? (v & 0xfff) - rt_d[v >> 12] : ~v); };
-  scan_queries<kRows, kH>(
-      a, Q, F.depth,
+  scan_queries<kRows, kH, kCsr>(
+      a, Q, kCsr ? 0 : F.depth,
       [&](int p, int r, bool first, int j) {
         if (!slots) return j;
         const int2 add = run_add[kTiles ? p : 0][kTiles ? r : 0];
@@ -417,6 +420,10 @@ __global__ void __launch_bounds__(kBlock) k_neighbor_fill(SearchArgs a, FillOut 
     const int last = (a.nq + 63) >> 6;
     if (blockIdx.x == 0) F.slices_out[last] = last * 64 * F.width;
   }
+  if (kCsr) {
+    if (bad) *F.ovf = 1;
+    return;
+  }
   __syncthreads();
   const int r = threadIdx.x % kRows, i = i0 + r;
   if (i < a.nq) {
@@ -428,7 +435,7 @@ __global__ void __launch_bounds__(kBlock) k_neighbor_fill(SearchArgs a, FillOut 
       F.counts[i] = n < len ? n : (int32_t)len;
       if (n > len) overflow(1);
     }
-    if (F.depth > 0) {
+    {
       const int staged = (int)(n < F.depth ? (n < len ? n : len) : (F.depth < len ? F.depth : len));
       constexpr int kStep = kBlock / kRows;
       int c = threadIdx.x / kRows;
@@ -468,9 +475,11 @@ template <int kRows, bool kH>
 static void launch_fill_rows(const SearchArgs& a, const FillOut& F, const FillTiles* tiles, hipStream_t st) {
   const size_t lds = (size_t)F.depth * (kRows + 1) * sizeof(int32_t);
   if (tiles)
-    k_neighbor_fill<kRows, true, kH><<<grid_for(a.nq, kRows), kBlock, lds, st>>>(a, F, *tiles);
+    k_neighbor_fill<kRows, true, kH, false><<<grid_for(a.nq, kRows), kBlock, lds, st>>>(a, F, *tiles);
+  else if (F.depth > 0)
+    k_neighbor_fill<kRows, false, kH, false><<<grid_for(a.nq, kRows), kBlock, lds, st>>>(a, F, FillTiles{});
   else
-    k_neighbor_fill<kRows, false, kH><<<grid_for(a.nq, kRows), kBlock, lds, st>>>(a, F, FillTiles{});
+    k_neighbor_fill<kRows, false, kH, true><<<grid_for(a.nq, kRows), kBlock, 0, st>>>(a, F, FillTiles{});
 }
 
 static int launch_fill(const SearchArgs& a, FillOut F, const FillTiles* tiles, hipStream_t st) {

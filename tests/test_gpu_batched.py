@@ -61,6 +61,20 @@ def test_batched_domains_match_single_domain_bitexact(cell_scale, block):
         _assert_domain_equal(b, _single_run(ens, d, cfg, steps), d, f"cs={cell_scale}")
 
 
+def test_batched_sparse_cells_match_single_domain_bitexact():
+    """A support of ~7 neighbors (two particles a cell): the batched fill takes
+    the queries of sparse cells side by side."""
+    B = _batched()
+    ens = B.make_ensemble(sizes=[200, 23, 30], dx=DX, seed=4, device="cuda", target_neighbors=7.0)
+    print(f"sparse batch: sizes {ens.counts}", flush=True)
+    b = B.BatchedDeltaSPH(ens.boxes, ens.counts, ens.pos, ens.vel, ens.mass, ens.rho, ens.cfg)
+    b.step(2)
+    torch.cuda.synchronize()
+    b.check_rows()
+    for d in range(len(ens.counts)):
+        _assert_domain_equal(b, _single_run(ens, d, ens.cfg, 2), d, "sparse")
+
+
 def test_batched_graph_replays_eager_steps_bitexact():
     B = _batched()
     ens = B.make_ensemble(sizes=[18, 33, 26], dx=DX, seed=3, device="cuda")

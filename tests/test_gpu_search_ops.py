@@ -397,13 +397,14 @@ def test_grid_cell_order_matches_oracle(orc, nside, hscale):
     np.testing.assert_array_equal(g.sort_index.cpu().numpy(), g_o.sort_index)
 
 
-# 33^2: a last workgroup of one row; 364^2 = 132496: the 64-row
-# workgroups.
+# 33^2: a last workgroup of one row; 364^2 = 132496 and, with supports per
+# particle, 513^2 = 263169: the 64-row workgroups.
 # Cells of 1.6 h and 2.4 h: cell rows beyond 64 and 128 candidates; 2.4 h of
 # 33^2 is a periodic grid under 7 cells (every row at the seam).
 @pytest.mark.parametrize("nside,hscale,per,vary", [
     (33, 1.0, (True, True), False), (33, 2.4, (True, True), True), (33, 1.6, (False, True), False),
-    (364, 1.0, (True, False), True), (364, 1.6, (True, True), False), (364, 2.4, (False, False), False)])
+    (364, 1.0, (True, False), True), (364, 1.6, (True, True), False), (364, 2.4, (False, False), False),
+    (513, 1.5, (True, True), True)])
 def test_search_rows_by_cell_match_oracle(orc, nside, hscale, per, vary):
     """Rows of the search (a wave takes the queries of a cell together) equal
     the oracle's in every layout, also past the staged depth."""
@@ -425,6 +426,39 @@ def test_search_rows_by_cell_match_oracle(orc, nside, hscale, per, vary):
         nl = search(g, g.sorted_pos, qh, "scatter", qpos_wrapped=True, layout=layout, width=width)
         np.testing.assert_array_equal(nl.counts.cpu().numpy(), c_o)
         np.testing.assert_array_equal(nl.csr_nbr().cpu().numpy()[: nbr_o.size], nbr_o)
+
+
+# Cells of 0.4 to 8 particles on average (the waves of sparse cells take their
+# queries side by side, those with over 96 candidates the cell's), a cloud with
+# both (a quarter of the particles in a corner, 40 a cell), and queries in
+# random order; 40001 and 300001: the 64-row workgroups, uniform and varied.
+@pytest.mark.parametrize("n,per_cell,per,vary,corner", [
+    (1000, 0.4, (True, True), False, False), (1001, 3.0, (False, True), True, False),
+    (40001, 0.5, (True, True), False, False), (40001, 3.0, (True, False), False, True),
+    (40001, 8.0, (True, True), False, False), (30001, 8.0, (False, False), True, True),
+    (300001, 3.0, (True, True), True, True)])
+def test_search_of_sparse_cells_matches_oracle(orc, n, per_cell, per, vary, corner):
+    print(f"case {n} {per_cell} {per} {vary} {corner}", flush=True)
+    rng = np.random.default_rng(n)
+    pos = rng.uniform(-1.0, 1.0, (n, 2))
+    h = np.float32(2.0 * np.sqrt(per_cell / n))
+    if corner:
+        pos[: n // 4] = -1.0 + rng.uniform(0.0, 1.0, (n // 4, 2)) * h * np.sqrt(n / 4 / 40)
+    pos = pos.astype(np.float32)
+    dom_o, dom = orc.make_domain((-1, -1), (1, 1), per), _lib.make_domain((-1, -1), (1, 1), per)
+    hp = (h * (0.7 + 0.3 * rng.random(n))).astype(np.float32) if vary else None
+    T = lambda a: None if a is None else torch.from_numpy(np.ascontiguousarray(a)).cuda()  # noqa: E731
+    g_o = orc.grid_build(dom_o, pos, float(h))
+    g = CellGrid.build(T(pos), T(hp), dom, float(h), h_uniform=0.0 if vary else float(h))
+    sh = hp[g_o.sort_index] if vary else None
+    mix = rng.permutation(n)
+    for q, qh in ((g_o.sorted_pos, sh), (g_o.sorted_pos[mix], None if sh is None else sh[mix])):
+        c_o, off_o, nbr_o = orc.neighbors_cell(dom_o, g_o, q, qh, h0=float(h), sorted_h=sh)
+        longest = int(c_o.max())
+        for layout, width in [("csr", 0), ("sell", 0), ("fixed", longest), ("fixed", longest + 70)]:
+            nl = search(g, T(q), T(qh), "scatter", qpos_wrapped=True, layout=layout, width=width)
+            np.testing.assert_array_equal(nl.counts.cpu().numpy(), c_o)
+            np.testing.assert_array_equal(nl.csr_nbr().cpu().numpy()[: nbr_o.size], nbr_o)
 
 
 def test_gather_set_permutes_every_array():

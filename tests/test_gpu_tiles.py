@@ -171,9 +171,9 @@ def _entries(nl):
 # 96^2: workgroups span two rows of cells and wrap the seam; 272^2; a
 # 5 x 5 periodic grid (every candidate range takes the seam path); cap 0:
 # the median tile size, so that some tiles do not fit and get no slots;
-# cap 64: none fit
+# cap 64: none fit; 97: cells of about two particles
 @pytest.mark.parametrize("nside,seed,cap,d16", [(96, 0, 4096, True), (272, 3, 1152, False), (272, 3, 0, True),
-                                                 (24, 5, 4096, False), (96, 2, 64, False)])
+                                                 (24, 5, 4096, False), (96, 2, 64, False), (97, 6, 4096, False)])
 def test_fill_built_tiles_equal_two_pass_tiles(nside, seed, cap, d16):
     from diffsph_amd import _lib
     d, _ = _setup(nside, seed)
@@ -183,6 +183,8 @@ def test_fill_built_tiles_equal_two_pass_tiles(nside, seed, cap, d16):
     h = float(d["h"])
     if nside == 24:
         h = 0.34  # a 5 x 5 cell grid over [-1, 1]^2
+    if nside == 97:
+        h = 1.4 * float(d["dx"])
     domain = _lib.make_domain((-1.0, -1.0), (1.0, 1.0), (True, True))
     median = cap == 0
     if median:
