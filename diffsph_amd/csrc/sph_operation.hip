@@ -11,6 +11,7 @@
 // tuple: qa indexed by i, qb by j) or per pair (a single tensor).
 #include "common.h"
 #include "near_math.h"
+#include <type_traits>
 
 namespace dsph {
 
@@ -71,13 +72,12 @@ __device__ __forceinline__ void pp_q(const PpArgs& a, int i, int64_t j, int64_t 
   (void)c;
 }
 
-// Sixteen lanes per row: a row's pairs are consecutive, so the lanes read
-// whole lines (one thread per row read 64 rows ~200 B apart and missed on
+// kPpLanes lanes per row: a row's pairs are consecutive, so the lanes read
+// whole lines (one thread per row reads 64 rows ~200 B apart and misses on
 // every array), and the terms are added in pair order (add_lanes).  kOut:
-// outputs per row, rounded up.  5.1M pairs: 147 -> 25 to 33 us an
+// outputs per row, rounded up.  102k rows of 50 pairs: 147 -> 25 to 33 us an
 // operation.
-constexpr int kPpLanes = 16;
-template <int kOut>
+template <int kOut, int kPpLanes>
 __global__ void __launch_bounds__(kBlock) k_pp_operation(PpArgs a, int ow) {
   const int row = (int)((blockIdx.x * (unsigned)kBlock + threadIdx.x) / kPpLanes);
   const bool valid = row < a.n;
@@ -214,9 +214,26 @@ static int launch_pp_operation(const PpArgs& a, hipStream_t st) {
   else if (a.op == PP_GRADIENT) ow = 2 * a.qw;
   else if (a.op == PP_DIVERGENCE || a.op == PP_DIVERGENCE_CONSISTENT) ow = a.qw / 2;
   else if (a.op == PP_LAPLACIAN) ow = a.qw;
-  auto go = [&](auto kernel) { kernel<<<grid_for(a.n, kBlock / kPpLanes), kBlock, 0, st>>>(a, ow); };
-  ow <= 1 ? go(k_pp_operation<1>)
-          : (ow <= 2 ? go(k_pp_operation<2>) : (ow <= 4 ? go(k_pp_operation<4>) : go(k_pp_operation<8>)));
+  auto go = [&](auto kernel, int lanes) { kernel<<<grid_for(a.n, kBlock / lanes), kBlock, 0, st>>>(a, ow); };
+  auto by_width = [&](auto lanes) {
+    constexpr int L = decltype(lanes)::value;
+    ow <= 1 ? go(k_pp_operation<1, L>, L)
+            : (ow <= 2 ? go(k_pp_operation<2, L>, L)
+                       : (ow <= 4 ? go(k_pp_operation<4, L>, L) : go(k_pp_operation<8, L>, L)));
+  };
+  // Rows of fewer pairs than lanes leave most of the lanes idle, which shows
+  // once the rows fill the chip.  Density / gradient of 1M rows in us with 1, 4
+  // and 16 lanes: 1.6 pairs a row 17 + 49, 22 + 52, 64 + 126; 3.1 pairs 25 + 74,
+  // 25 + 64, 65 + 127; 9.4 pairs 175 + 313, 41 + 110, 71 + 142; 28 pairs 986 +
+  // 1155, 140 + 293, 147 + 322; 50 pairs - , 289 + 485, 218 + 482.  30k rows of
+  // 28 pairs: 20 + 62, 11 + 20, 12 + 14.
+  const int64_t rows = a.n;
+  if (rows <= (1 << 15) || a.np >= 24 * rows)
+    by_width(std::integral_constant<int, 16>{});
+  else if (a.np >= 3 * rows)
+    by_width(std::integral_constant<int, 4>{});
+  else
+    by_width(std::integral_constant<int, 1>{});
   return launch_status();
 }
 

@@ -3,7 +3,7 @@
 Drop-ins for ``sphOperation`` and ``sphOperationStates``
 (src/diffSPH/v2/sphOps.py:253-303): same names, argument order, argument
 meaning and return shapes.  Every operation runs as one HIP kernel
-(``dsph_pp_operation``: one thread per row, the row's pairs summed in list
+(``dsph_pp_operation``: 1 to 16 threads per row, its pairs summed in list
 order); there is no CPU path.
 
 Arguments follow the reference: ``masses`` and ``densities`` are (set A,

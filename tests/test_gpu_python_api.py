@@ -139,6 +139,40 @@ def test_sph_operation_states_and_per_pair_quantity(ops):
     _close(out, d["grad_difference_scalar"])
 
 
+@pytest.mark.parametrize("mean", [1.5, 8.0, 30.0])
+@pytest.mark.parametrize("operation,width", [("density", 1), ("interpolate", 1), ("gradient", 1), ("gradient", 4),
+                                             ("divergence", 2), ("divergence", 4), ("curl", 2), ("laplacian", 2)])
+def test_sph_operation_short_rows_equal_split_rows(mean, operation, width):
+    """Many rows of few pairs (1 or 4 threads a row) give the bits of the same
+    rows in calls of up to 32768 rows (16 threads a row); empty rows and a
+    last workgroup that is not full among them."""
+    from diffsph_amd.sphops import sphOperation
+    print(f"case {mean} {operation} {width}", flush=True)
+    rng = np.random.default_rng(int(mean) * 10 + width)
+    n, nb = 40003, 5000
+    counts = rng.poisson(mean, n)
+    P = int(counts.sum())
+    f = lambda *sh: torch.from_numpy(rng.standard_normal(sh).astype(np.float32)).cuda()  # noqa: E731
+    i = torch.from_numpy(np.repeat(np.arange(n), counts)).cuda()
+    j = torch.from_numpy(rng.integers(0, nb, P)).cuda()
+    W, gW, r, x, h = f(P).abs(), f(P, 2), f(P).abs() + 0.1, f(P, 2), f(P).abs() + 0.5
+    ma, mb, ra, rb = f(n).abs() + 0.5, f(nb).abs() + 0.5, f(n).abs() + 0.5, f(nb).abs() + 0.5
+    shape = {1: (), 2: (2,), 4: (2, 2)}[width]
+    qa, qb = f(n, *shape), f(nb, *shape)
+
+    def run(lo, hi):
+        s = (i >= lo) & (i < hi)
+        return sphOperation((ma[lo:hi].contiguous(), mb), (ra[lo:hi].contiguous(), rb),
+                            (qa[lo:hi].contiguous(), qb), ((i[s] - lo).contiguous(), j[s].contiguous()), W[s], gW[s],
+                            r[s], x[s], h[s], hi - lo, operation,
+                            gradientMode="conserving" if operation == "laplacian" else "difference")
+
+    whole = run(0, n)
+    split = torch.cat([run(0, 20000), run(20000, n)])
+    assert torch.isfinite(whole).all() and float(whole.abs().max()) > 0
+    assert torch.equal(whole, split)
+
+
 def test_sph_operation_rejects_unsorted_rows(ops):
     from diffsph_amd._lib import DsphError
     from diffsph_amd.sphops import sphOperation
