@@ -744,11 +744,11 @@ __global__ void __launch_bounds__(kBlock) k_ghosts(const float2* __restrict__ bp
 
 // The reference's C++ mDBC op (mDBCDensityKernel, v2/cppSrc/mDBC.h:129-244):
 // x_gj = -(q h) xhat, b = sum m_j [W, gradW], Cramer's rule with
-// det + 1e-7, Shepard density for <= 5 neighbors, clamped at rho0.  Sixteen
-// lanes per ghost (the terms of MdbcOpAcc::add in row order): a wall has a few
-// thousand ghosts, one thread each left most CUs idle (9k ghosts of the 131k
-// dam break: 33 -> 8.7 us).
-constexpr int kGhostLanes = 16;
+// det + 1e-7, Shepard density for <= 5 neighbors, clamped at rho0.
+// kGhostLanes lanes per ghost (the terms of MdbcOpAcc::add in row order): a
+// wall has a few thousand ghosts, one thread each leaves most CUs idle (9k
+// ghosts of the 131k dam break: 33 -> 8.7 us with 16).
+template <int kGhostLanes>
 __global__ void __launch_bounds__(kBlock) k_mdbc_op(PairsDev G, const float* __restrict__ mass,
                                                     const float* __restrict__ rho, const float2* __restrict__ bpos,
                                                     float rho0, float* __restrict__ rho_b,
@@ -1274,9 +1274,18 @@ extern "C" int dsph_mdbc(const dsph_pairs* ghost_pairs, const float* fluid_mass,
   PairsDev G = make_pairs(*ghost_pairs);
   const float2* xb = reinterpret_cast<const float2*>(boundary_pos);
   hipStream_t st = as_stream(stream);
-  if (variant == 1)
-    k_mdbc_op<<<grid_for(G.nq, kBlock / kGhostLanes), kBlock, 0, st>>>(G, fluid_mass, fluid_rho, xb, rho0,
-                                                                       boundary_rho, shepard);
+  auto go = [&](auto kernel, int lanes) {
+    kernel<<<grid_for(G.nq, kBlock / lanes), kBlock, 0, st>>>(G, fluid_mass, fluid_rho, xb, rho0, boundary_rho,
+                                                              shepard);
+  };
+  // ghosts of 50 neighbors in us with 16, 4 and 1 lanes: 10k 13.0 / 17.9 / 52,
+  // 30k 25 / 20 / 56, 100k 64 / 41 / 73, 300k 171 / 92 / 98, 1M 552 / 281 / 265
+  if (variant == 1 && G.nq <= (1 << 14))
+    go(k_mdbc_op<16>, 16);
+  else if (variant == 1 && G.nq <= (1 << 19))
+    go(k_mdbc_op<4>, 4);
+  else if (variant == 1)
+    go(k_mdbc_op<1>, 1);
   else
     k_mdbc<<<grid_for(G.nq), kBlock, 0, st>>>(G, fluid_mass, fluid_rho, xb, rho0, support, boundary_rho, shepard);
   return launch_status();

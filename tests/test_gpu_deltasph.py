@@ -273,6 +273,35 @@ def test_dam_break_config_properties():
     assert float((wr[under] - cfg.rho0).abs().max()) < 0.01 * cfg.rho0
 
 
+# 16, 4 (up to 2^19) and 1 lanes per ghost, each with a last workgroup that is not full
+@pytest.mark.parametrize("ghosts", [5, 16384, 16390, 524291])
+def test_mdbc_op_ghost_counts_match_oracle_bitexact(ghosts):
+    from diffsph_amd.neighborhood import CellGrid, search
+    print(f"case {ghosts}", flush=True)
+    rng = np.random.default_rng(ghosts)
+    nf, h, per = 1500, 0.13, (True, False)
+    f32 = lambda *sh: rng.uniform(-1.0, 1.0, sh).astype(np.float32)  # noqa: E731
+    fluid, gpos, wall = f32(nf, 2), f32(ghosts, 2), f32(ghosts, 2)
+    fluid[:, 1] *= 0.7  # ghosts without fluid and with up to five neighbors among them
+    mass, rho = (4.0 / nf * (1.0 + 0.1 * f32(nf))).astype(np.float32), (1.0 + 0.05 * f32(nf)).astype(np.float32)
+    dom_o, dom = orc.make_domain((-1, -1), (1, 1), per), _lib.make_domain((-1, -1), (1, 1), per)
+    T = lambda a: torch.from_numpy(a).cuda()  # noqa: E731
+    g = CellGrid.build(T(fluid), None, dom, h, h_uniform=h)
+    si = g.sort_index.long()
+    nl = search(g, T(gpos), None, "scatter", layout="sell")
+    pr = nl.pairs()
+    m, r, x = T(mass)[si].contiguous(), T(rho)[si].contiguous(), T(wall)
+    out, shep = torch.empty(ghosts, device="cuda"), torch.empty(ghosts, device="cuda")
+    P = _lib.ptr
+    _lib.check(_lib.lib().dsph_mdbc(C.byref(pr), P(m), P(r), P(x), C.c_float(1.0), C.c_float(h), 1, P(out), P(shep),
+                                    _lib.stream_handle(out.device)), "mdbc")
+    off = np.concatenate([[0], np.cumsum(nl.counts.cpu().numpy())]).astype(np.int32)
+    ref, rshep = orc.mdbc(dom_o, off, nl.csr_nbr().cpu().numpy(), nl.qpos.cpu().numpy(), g.sorted_pos.cpu().numpy(),
+                          h, m.cpu().numpy(), r.cpu().numpy(), wall, 1.0, h, variant=1)
+    np.testing.assert_array_equal(out.cpu().numpy(), ref)
+    np.testing.assert_array_equal(shep.cpu().numpy(), rshep)
+
+
 # rows of 16, 4 and 1 lanes, with a last workgroup that is not full
 @pytest.mark.parametrize("nside", [33, 91, 131, 363])
 @pytest.mark.parametrize("state", ["plain", "switch", "odd"])
