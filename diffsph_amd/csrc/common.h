@@ -460,6 +460,15 @@ inline int grid_for(int64_t n, int block = kBlock) {
   return (int)(g < 1 ? 1 : g);
 }
 
+// launch(row0, rows) for all n rows of a kernel that takes `threads` (a power of
+// two up to kBlock) threads per row: a launch holds less than 2^32 threads, so
+// more rows than that come in several.
+template <class F>
+inline void in_launches(int64_t n, int threads, F&& launch) {
+  const int64_t most = ((int64_t)1 << 31) / threads;
+  for (int64_t r = 0; r < n; r += most) launch((int)r, n - r < most ? n - r : most);
+}
+
 inline int launch_status() {
   hipError_t e = hipGetLastError();
   return e == hipSuccess ? DSPH_OK : DSPH_ERR_LAUNCH;

@@ -104,6 +104,14 @@ struct SearchArgs {
   int nref;
 };
 
+// The queries from row0 on, for a launch of their own.
+inline SearchArgs queries_from(SearchArgs a, int row0, int64_t rows) {
+  a.qpos += row0;
+  if (a.qh) a.qh += row0;
+  a.nq = (int)rows;
+  return a;
+}
+
 // A candidate reference particle: wrapped position and support.
 struct Cand {
   float2 x;
@@ -471,25 +479,42 @@ __global__ void __launch_bounds__(kBlock) k_neighbor_fill(SearchArgs a, FillOut 
   if (bad) *F.ovf = 1;
 }
 
+// The list's rows from row0 (a multiple of 256) on.
+static FillOut rows_from(FillOut F, int row0) {
+  if (F.off) F.off += row0;
+  if (F.slice) F.slice += row0 / 64;
+  if (F.slices_out) F.slices_out += row0 / 64;
+  if (F.width > 0) {
+    const int64_t o = (int64_t)row0 * F.width;
+    F.nbr += o;
+    F.cap -= o;
+    F.counts += row0;
+  }
+  return F;
+}
+
+static FillTiles tiles_from(FillTiles T, int row0, int width) {
+  T.runs += (int64_t)(row0 / kBlock) * kTileRunStride;
+  T.n += row0 / kBlock;
+  T.slot += (int64_t)row0 * width;
+  return T;
+}
+
 template <int kRows, bool kH>
 static void launch_fill_rows(const SearchArgs& a, const FillOut& F, const FillTiles* tiles, hipStream_t st) {
   const size_t lds = (size_t)F.depth * (kRows + 1) * sizeof(int32_t);
+  auto go = [&](auto kernel) {
+    in_launches(a.nq, kBlock / kRows, [&](int row0, int64_t rows) {
+      kernel<<<grid_for(rows, kRows), kBlock, lds, st>>>(queries_from(a, row0, rows), rows_from(F, row0),
+                                                         tiles ? tiles_from(*tiles, row0, F.width) : FillTiles{});
+    });
+  };
   if (tiles)
-    k_neighbor_fill<kRows, true, kH, false><<<grid_for(a.nq, kRows), kBlock, lds, st>>>(a, F, *tiles);
+    go(k_neighbor_fill<kRows, true, kH, false>);
   else if (F.depth > 0)
-    k_neighbor_fill<kRows, false, kH, false><<<grid_for(a.nq, kRows), kBlock, lds, st>>>(a, F, FillTiles{});
+    go(k_neighbor_fill<kRows, false, kH, false>);
   else
-    k_neighbor_fill<kRows, false, kH, true><<<grid_for(a.nq, kRows), kBlock, 0, st>>>(a, F, FillTiles{});
-}
-
-static int launch_fill(const SearchArgs& a, FillOut F, const FillTiles* tiles, hipStream_t st) {
-  F.depth = F.width > 0 ? (F.width < kRowStage ? F.width : kRowStage) : (F.slice ? kRowStage : 0);
-  const bool vary = varied_support(a);
-  if (small_query_set(a))
-    vary ? launch_fill_rows<16, true>(a, F, tiles, st) : launch_fill_rows<16, false>(a, F, tiles, st);
-  else
-    vary ? launch_fill_rows<64, true>(a, F, tiles, st) : launch_fill_rows<64, false>(a, F, tiles, st);
-  return launch_status();
+    go(k_neighbor_fill<kRows, false, kH, true>);
 }
 
 __global__ void __launch_bounds__(kBlock) k_fixed_slices(int nslices, int width, int32_t* __restrict__ slice_off,
@@ -503,13 +528,35 @@ __global__ void __launch_bounds__(kBlock) k_fixed_slices(int nslices, int width,
   if (s <= nslices) slice_off[s] = s * 64 * width;
 }
 
+__global__ void k_set_flag(int32_t* flag, int v) {
+  if (threadIdx.x == 0) *flag = v;
+}
+
+static int launch_fill(const SearchArgs& a, FillOut F, const FillTiles* tiles, hipStream_t st) {
+  F.depth = F.width > 0 ? (F.width < kRowStage ? F.width : kRowStage) : (F.slice ? kRowStage : 0);
+  const bool vary = varied_support(a);
+  // several launches (in_launches): their rows count from each one's first, so
+  // 16-bit deltas are given up as if one had not fitted, and the slice offsets
+  // are written once more
+  const bool several = (int64_t)a.nq * 4 > ((int64_t)1 << 31);
+  if (several && F.d16) {
+    k_set_flag<<<1, 64, 0, st>>>(F.ovf, 1);
+    F.d16 = nullptr;
+  }
+  if (small_query_set(a))
+    vary ? launch_fill_rows<16, true>(a, F, tiles, st) : launch_fill_rows<16, false>(a, F, tiles, st);
+  else
+    vary ? launch_fill_rows<64, true>(a, F, tiles, st) : launch_fill_rows<64, false>(a, F, tiles, st);
+  if (several && F.slices_out) {
+    const int nslices = (int)(((int64_t)a.nq + 63) / 64);
+    k_fixed_slices<<<grid_for(nslices + 1), kBlock, 0, st>>>(nslices, F.width, F.slices_out, nullptr, nullptr);
+  }
+  return launch_status();
+}
+
 __global__ void __launch_bounds__(kBlock) k_zero_i32(int32_t* __restrict__ a, int64_t n) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) a[i] = 0;
-}
-
-__global__ void k_fill_flag_clear(int32_t* flag) {
-  if (threadIdx.x == 0) *flag = 0;
 }
 
 // Longest row of every 64-row slice, times 64 (one wave per slice).
@@ -690,7 +737,11 @@ extern "C" int dsph_neighbor_count(const dsph_domain* domain, const dsph_grid* g
   if (nq == 0) return DSPH_OK;
   hipStream_t st = as_stream(stream);
   const bool vary = varied_support(a);
-  auto launch = [&](auto kernel, int rows) { kernel<<<grid_for(nq, rows), kBlock, 0, st>>>(a, counts); };
+  auto launch = [&](auto kernel, int per_block) {
+    in_launches(nq, kBlock / per_block, [&](int row0, int64_t rows) {
+      kernel<<<grid_for(rows, per_block), kBlock, 0, st>>>(queries_from(a, row0, rows), counts + row0);
+    });
+  };
   if (small_query_set(a))
     vary ? launch(k_neighbor_count<16, true>, 16) : launch(k_neighbor_count<16, false>, 16);
   else
@@ -727,7 +778,7 @@ extern "C" int dsph_neighbor_fill16(const dsph_domain* domain, const dsph_grid* 
   // the deltas are j - i modulo n: row i must be reference slot i
   if (nq != nref || !qpos_wrapped) return DSPH_ERR_ARG;
   hipStream_t st = as_stream(stream);
-  k_fill_flag_clear<<<1, 64, 0, st>>>(overflow);
+  k_set_flag<<<1, 64, 0, st>>>(overflow, 0);
   DSPH_LAUNCH_CHECK();
   if (nq == 0) return DSPH_OK;
   if ((!offsets && !slice_off) || (capacity > 0 && !nbr) || capacity < 0 || layout_total < 0) return DSPH_ERR_ARG;

@@ -78,8 +78,8 @@ __device__ __forceinline__ void pp_q(const PpArgs& a, int i, int64_t j, int64_t 
 // outputs per row, rounded up.  102k rows of 50 pairs: 147 -> 25 to 33 us an
 // operation.
 template <int kOut, int kPpLanes>
-__global__ void __launch_bounds__(kBlock) k_pp_operation(PpArgs a, int ow) {
-  const int row = (int)((blockIdx.x * (unsigned)kBlock + threadIdx.x) / kPpLanes);
+__global__ void __launch_bounds__(kBlock) k_pp_operation(PpArgs a, int ow, int row0) {
+  const int row = row0 + (int)((blockIdx.x * (unsigned)kBlock + threadIdx.x) / kPpLanes);
   const bool valid = row < a.n;
   const int i = valid ? row : a.n - 1;
   const int g = threadIdx.x & (kPpLanes - 1);
@@ -214,7 +214,11 @@ static int launch_pp_operation(const PpArgs& a, hipStream_t st) {
   else if (a.op == PP_GRADIENT) ow = 2 * a.qw;
   else if (a.op == PP_DIVERGENCE || a.op == PP_DIVERGENCE_CONSISTENT) ow = a.qw / 2;
   else if (a.op == PP_LAPLACIAN) ow = a.qw;
-  auto go = [&](auto kernel, int lanes) { kernel<<<grid_for(a.n, kBlock / lanes), kBlock, 0, st>>>(a, ow); };
+  auto go = [&](auto kernel, int lanes) {
+    in_launches(a.n, lanes, [&](int row0, int64_t rows) {
+      kernel<<<grid_for(rows, kBlock / lanes), kBlock, 0, st>>>(a, ow, row0);
+    });
+  };
   auto by_width = [&](auto lanes) {
     constexpr int L = decltype(lanes)::value;
     ow <= 1 ? go(k_pp_operation<1, L>, L)

@@ -303,8 +303,8 @@ __global__ void __launch_bounds__(kBlock) k_export_pairs(PairsDev P, const int32
                                                          const int32_t* __restrict__ r_sort,
                                                          const int32_t* __restrict__ out_off, int64_t* out_i,
                                                          int64_t* out_j, float* out_r, float* out_x, float* out_h,
-                                                         float* out_w, float* out_g) {
-  const int q = (int)((blockIdx.x * (unsigned)kBlock + threadIdx.x) / kExportLanes);
+                                                         float* out_w, float* out_g, int q0) {
+  const int q = q0 + (int)((blockIdx.x * (unsigned)kBlock + threadIdx.x) / kExportLanes);
   if (q >= P.nq) return;
   const int row = q_rank ? q_rank[q] : q;
   const float2 xi = P.qpos[row];
@@ -531,9 +531,11 @@ extern "C" int dsph_pairs_export(const dsph_pairs* pairs, const int32_t* q_sort_
   if (s != DSPH_OK) return s;
   if (P.nq == 0) return DSPH_OK;
   (void)q_sort_index;
-  k_export_pairs<<<grid_for(P.nq, kBlock / kExportLanes), kBlock, 0, st>>>(P, q_rank, r_sort_index, out_offsets, out_i,
-                                                                           out_j, out_distances, out_vectors,
-                                                                           out_supports, out_kernels, out_gradients);
+  in_launches(P.nq, kExportLanes, [&](int q0, int64_t rows) {
+    k_export_pairs<<<grid_for(rows, kBlock / kExportLanes), kBlock, 0, st>>>(
+        P, q_rank, r_sort_index, out_offsets, out_i, out_j, out_distances, out_vectors, out_supports, out_kernels,
+        out_gradients, q0);
+  });
   return launch_status();
 }
 
