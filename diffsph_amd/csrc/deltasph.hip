@@ -536,6 +536,7 @@ __global__ void __launch_bounds__(kBlock) k_dsph_rhs_near(PairsDev P, BoundaryDe
     }
     wrap_offsets(dx, dy, dm);
     NearRange range;
+    range.operand(rho_i);  // the density difference is a dividend
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const NbrRhs& e = d[u];

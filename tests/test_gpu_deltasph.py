@@ -304,12 +304,12 @@ def test_mdbc_op_ghost_counts_match_oracle_bitexact(ghosts):
 
 # rows of 16, 4 and 1 lanes, with a last workgroup that is not full
 @pytest.mark.parametrize("nside", [33, 91, 131, 363])
-@pytest.mark.parametrize("state", ["plain", "switch", "odd"])
+@pytest.mark.parametrize("state", ["plain", "switch", "odd", "rest"])
 def test_near_kernels_equal_general_kernels(nside, state):
     """The uniform-support kernels give the bits of the general ones (reached
     by passing the same support per particle), also for operands out of
     their fast range: zero, tiny and huge densities, infinities, NaN, pairs
-    closer than 2^-48."""
+    closer than 2^-48; at rest the own density meets no other operand."""
     print(f"case {nside} {state}", flush=True)
     rng = np.random.default_rng(3)
     pos, dx = sampling.sample_regular(nside)
@@ -317,6 +317,9 @@ def test_near_kernels_equal_general_kernels(nside, state):
     n = pos.shape[0]
     vel = rng.standard_normal((n, 2)).astype(np.float32)
     rho = (1.0 + 0.01 * rng.standard_normal(n)).astype(np.float32)
+    if state == "rest":
+        vel[:] = 0.0
+        rho[rng.permutation(n)[:6]] = [3e38, np.inf, 1e-30, -3e38, 2e37, 1e25]
     if state == "odd":
         pos[0] = (1e-16, 1e-17)
         pos[1] = (1e-16, 3e-16)
@@ -337,14 +340,16 @@ def test_near_kernels_equal_general_kernels(nside, state):
         pr.qh = pr.rh = _lib.ptr(hs) if general else None
         vol, g, m = torch.empty(n, device=dev), torch.empty(n, 2, device=dev), torch.empty(n, 4, device=dev)
         g2, du, dr = torch.empty(n, 2, device=dev), torch.empty(n, 2, device=dev), torch.empty(n, device=dev)
+        tm = torch.empty(n, 8, device=dev)
         P = _lib.ptr
         _lib.check(L.dsph_volume(n, P(sv.mass), P(sv.rho), P(vol), st), "volume")
         _lib.check(L.dsph_deltasph_normalization_v(C.byref(pr), None, P(sv.mass), P(sv.rho), P(vol), P(m), None, P(g),
                                                    st), "normalization")
         _lib.check(L.dsph_deltasph_normalization_v(C.byref(pr), None, P(sv.mass), P(sv.rho), None, None, None, P(g2),
                                                    st), "normalization")
-        _lib.check(L.dsph_deltasph_rhs(C.byref(pr), None, C.byref(sv.prm), P(sv.vel), P(sv.mass), P(sv.rho), P(g),
-                                       P(du), P(dr), None, st), "rhs")
-        out.append([t.cpu().numpy() for t in (m, g, g2, du, dr)])
-    for name, a, b in zip(("L", "grad", "grad, no volumes", "dudt", "drhodt"), *out):
+        gr = torch.zeros_like(g) if state == "rest" else g
+        _lib.check(L.dsph_deltasph_rhs(C.byref(pr), None, C.byref(sv.prm), P(sv.vel), P(sv.mass), P(sv.rho), P(gr),
+                                       P(du), P(dr), P(tm), st), "rhs")
+        out.append([t.cpu().numpy() for t in (m, g, g2, du, dr, tm)])
+    for name, a, b in zip(("L", "grad", "grad, no volumes", "dudt", "drhodt", "terms"), *out):
         np.testing.assert_array_equal(a, b, err_msg=name)
