@@ -387,12 +387,19 @@ class DeltaSPHSolver:
         st = _lib.stream_handle(self.pos.device)
 
         src = [t.contiguous() for t in (self.pos, self.vel, self.mass, self.rho, self.uid)]
-        dst = [torch.empty_like(t) for t in src]
-        k = len(src)
-        words = [t.element_size() * (t.numel() // max(self.n, 1)) // 4 for t in src]
-        check(lib().dsph_gather_set(ptr(si), self.n, k, (C.c_void_p * k)(*[t.data_ptr() for t in src]),
-                                    (C.c_void_p * k)(*[t.data_ptr() for t in dst]), (C.c_int32 * k)(*words), st),
-              "gather_set")
+        words = [t.element_size() * (t.numel() // max(self.n, 1)) / 4 for t in src]
+        # one pass over the arrays it takes (1, 2 or 4 words per particle, aligned
+        # to them); a caller's other ones are indexed
+        taken = [w in (1, 2, 4) and t.data_ptr() % int(4 * w) == 0 for t, w in zip(src, words)]
+        dst = [torch.empty_like(t) if ok else t[si.long()] for t, ok in zip(src, taken)]
+        k = sum(taken)
+
+        def those(v):
+            return [x for x, ok in zip(v, taken) if ok]
+
+        check(lib().dsph_gather_set(ptr(si), self.n, k, (C.c_void_p * k)(*[t.data_ptr() for t in those(src)]),
+                                    (C.c_void_p * k)(*[t.data_ptr() for t in those(dst)]),
+                                    (C.c_int32 * k)(*[int(w) for w in those(words)]), st), "gather_set")
         self.pos, self.vel, self.mass, self.rho, self.uid = dst
 
     # -- one step ------------------------------------------------------------

@@ -273,6 +273,27 @@ def test_dam_break_config_properties():
     assert float((wr[under] - cfg.rho0).abs().max()) < 0.01 * cfg.rho0
 
 
+def test_sort_takes_arrays_the_one_pass_permute_does_not():
+    """A state array put in place by the caller at an odd 4-byte offset, and
+    particle ids of 8 or 16 bits, are permuted as any other."""
+    pos, vel, mass, rho, cfg = taylor_green_state(24, torch.device("cuda:0"))
+    a, b = DeltaSPHSolver(pos, vel, mass, rho, cfg), DeltaSPHSolver(pos, vel, mass, rho, cfg)
+    n = a.n
+    buf = torch.zeros(2 * n + 1, device=pos.device)
+    buf[1:] = b.vel.flatten()
+    b.vel = buf[1:].view(n, 2)
+    b.uid = b.uid.to(torch.int16)
+    for _ in range(2):
+        a.step()
+        b.step()
+    assert b.uid.dtype == torch.int16 and torch.equal(a.uid, b.uid.to(torch.int32))
+    for name in ("pos", "vel", "mass", "rho"):
+        assert torch.equal(getattr(a, name), getattr(b, name)), name
+    b.uid = (b.uid % 100).to(torch.uint8)
+    b.step()
+    assert b.uid.dtype == torch.uint8
+
+
 # 16, 4 (up to 2^19) and 1 lanes per ghost, each with a last workgroup that is not full
 @pytest.mark.parametrize("ghosts", [5, 16384, 16390, 524291])
 def test_mdbc_op_ghost_counts_match_oracle_bitexact(ghosts):
