@@ -50,7 +50,7 @@ constexpr int kSeamBit = 1 << 30;
 
 // Ranges of the cells cx-1 .. cx+1 of the row whose first cell is cs[0].  A
 // slice longer than `longest` is left out and sets `over`, cell by cell in a
-// wrapping row.
+// wrapping row.  A periodic row has at least two cells (searches refuse one).
 __device__ __forceinline__ CellRow cell_row(const int32_t* __restrict__ cs, int ncx, int cx, bool periodic_x,
                                             bool seam, int longest, bool& over) {
   CellRow r;

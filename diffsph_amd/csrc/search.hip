@@ -596,6 +596,9 @@ static int make_search(SearchArgs& a, const dsph_domain* domain, const dsph_grid
                        const float* sorted_pos, const float* sorted_h, int64_t nref, const float* qpos,
                        const float* qh, int64_t nq, int32_t wrapped, float h0, int32_t mode) {
   if (!domain || check_grid(grid) != DSPH_OK) return DSPH_ERR_ARG;
+  // one periodic column: a cell row would be the same cell three times, which
+  // is no two runs of slots (cell_row)
+  if (domain->periodic[0] && grid->ncell[0] < 2) return DSPH_ERR_DIM;
   if (nq < 0 || nref < 0 || nq >= INT32_MAX || nref >= INT32_MAX) return DSPH_ERR_ARG;
   if (mode < 0 || mode > 2) return DSPH_ERR_ARG;
   if (nq > 0 && (!qpos || !cell_start)) return DSPH_ERR_ARG;

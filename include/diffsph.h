@@ -212,7 +212,8 @@ int dsph_grid_build_wrapped(const dsph_domain* domain, const dsph_grid* grid,
 /* Count, for each query particle, the reference particles within its support
  * (replaces countNeighbors, neighborhood.cpp:65-227, and the counting pass
  * of computeNeighborhood, v2/cppSrc/computeNeighborhood.h:115-146).
- * `qpos_wrapped` != 0 when qpos already holds wrapped positions.
+ * `qpos_wrapped` != 0 when qpos already holds wrapped positions.  A periodic
+ * x axis of one cell is refused (DSPH_ERR_DIM), here and by the fills.
  * The predicate is evaluated in float32 as
  *   d = mod(wrap(x_i) - wrap(x_j)); r = sqrt_rn(d.x*d.x + d.y*d.y) (no FMA);
  *   keep iff r /_rn h_mode <= 1

@@ -54,6 +54,23 @@ def test_host_only_entry_points_run_without_gpu():
                               C.c_void_p(0x4000), None) == 1
 
 
+def test_search_refuses_a_single_periodic_column():
+    """One column of cells on a periodic x axis (a grid dsph_grid_build refuses
+    for the domain): a query's cell row would not be two runs of cells.
+    Refused on the host (the pointers are never dereferenced)."""
+    from diffsph_amd import _lib
+    L = _lib.lib()
+    p = [C.c_void_p(0x1000 * (k + 1)) for k in range(8)]
+    for per, want in [((True, False), 2), ((True, True), 2)]:
+        dom = _lib.make_domain((-1, -1), (1, 1), per)
+        g = _lib.Grid()
+        g.ncell[0], g.ncell[1], g.hcell = 1, 4, 2.0
+        a = (C.byref(dom), C.byref(g), p[0], p[1], None, 10, p[2], None, 10, 1, C.c_float(0.5), 1)
+        assert L.dsph_neighbor_count(*a, p[3], None) == want
+        assert L.dsph_neighbor_fill(*a, p[3], None, 10, p[4], 10, None) == want
+        assert L.dsph_neighbor_fill_fixed_or(*a, 4, p[3], p[4], p[5], 256, None, p[6], None) == want
+
+
 def test_grid_dims_match_oracle(orc):
     from diffsph_amd import _lib
     L = _lib.lib()
