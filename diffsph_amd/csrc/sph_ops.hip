@@ -320,10 +320,16 @@ __global__ void __launch_bounds__(kBlock) k_export_pairs(PairsDev P, const int32
     if (out_i) out_i[o] = q;
     if (out_j) out_j[o] = r_sort ? r_sort[j] : j;
     if (out_r) out_r[o] = g.q;
-    if (out_x) *reinterpret_cast<float2*>(out_x + 2 * o) = make_float2(g.ex, g.ey);
+    if (out_x) {
+      out_x[2 * o] = g.ex;
+      out_x[2 * o + 1] = g.ey;
+    }
     if (out_h) out_h[o] = h;
     if (out_w) out_w[o] = g.w;
-    if (out_g) *reinterpret_cast<float2*>(out_g + 2 * o) = make_float2(g.gx, g.gy);
+    if (out_g) {
+      out_g[2 * o] = g.gx;
+      out_g[2 * o + 1] = g.gy;
+    }
   }
 }
 

@@ -29,14 +29,17 @@ def test_pairs_export_beyond_one_launch():
     pr.h_uniform, pr.mode = 0.5, 1
     pr.domain = _lib.make_domain((-1, -1), (1, 1), (False, False))
     i, j = torch.full((3,), -1, device=dev), torch.full((3,), -1, device=dev)
-    d, x = torch.zeros(3, device=dev), torch.zeros(3, 2, device=dev)
+    d = torch.zeros(3, device=dev)
+    x, gr = (torch.zeros(7, device=dev)[1:].view(3, 2) for _ in range(2))  # aligned to their floats only
     oo = torch.empty(n + 1, dtype=torch.int32, device=dev)
     L = _lib.lib()
     ws = torch.empty(L.dsph_pairs_export_workspace(n), dtype=torch.uint8, device=dev)
-    _lib.check(L.dsph_pairs_export(C.byref(pr), None, None, None, P(oo), P(i), P(j), P(d), P(x), None, None, None,
+    _lib.check(L.dsph_pairs_export(C.byref(pr), None, None, None, P(oo), P(i), P(j), P(d), P(x), None, None, P(gr),
                                    P(ws), ws.numel(), _lib.stream_handle(q.device)), "pairs_export")
     assert i.tolist() == [0, n - 1, n - 1] and j.tolist() == [0, 1, 2]
     torch.testing.assert_close(d.cpu(), torch.tensor([0.2, 0.1, 0.1]))
+    torch.testing.assert_close(x.cpu(), torch.tensor([[0.0, -1.0], [0.0, -1.0], [1.0, 0.0]]), rtol=0, atol=1e-5)
+    assert (gr[:, 0].abs().cpu() > 0).tolist() == [False, False, True]
 
 
 @pytest.mark.parametrize("what", ["count", "csr", "fixed"])
