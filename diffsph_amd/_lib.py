@@ -275,6 +275,7 @@ SIGNATURES = {
     "dsph_mlp_forward_affine": (C.c_int, [V, I64, V, V, V, F32, F32, I32, V, V]),
     "dsph_mlp_train_workspace": (SZ, [I64]),
     "dsph_mlp_loss_grad": (C.c_int, [V, V, I64, F32, V, V, V, V, V, SZ, V]),
+    "dsph_near_check": (C.c_int, [I32, C.c_uint32, I64, C.c_uint64, V, V]),
     "dsph_adam_step": (C.c_int, [V, V, V, V, I64, F32, F32, F32, F32, F32, I32, V]),
     "dsph_remap_neighbors": (C.c_int, [V, I64, V, I64, V]),
     "dsph_deltasph_normalization": (C.c_int, [P(Pairs), P(Boundary), V, V, V, V, V, V]),

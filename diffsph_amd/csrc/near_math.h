@@ -10,10 +10,11 @@
 // elementary functions on the IBM RISC System/6000 processor", IBM J. Res.
 // Dev. 34(1), 1990: q + y fma(-b, q, a) with y the rounded 1/b), the
 // reciprocal and the square root by comparison with the IEEE forms over
-// every float32 in range on this hardware (1.0e9 and 1.6e9 values, no
-// difference; 1.7e10 random quotients likewise).  So results are the same
-// bits; the kernels that use them test the range per group of entries and
-// evaluate the IEEE forms where it does not hold.
+// every float32 in range on this hardware (dsph_near_check: 1.0e9 and 1.6e9
+// values, no difference; 4e9 drawn quotients likewise).  So results are the
+// same bits, quotients below 2^-100 aside; the kernels that use them test the
+// range per group of entries and evaluate the IEEE forms where it does not
+// hold.
 #pragma once
 
 #include "common.h"
@@ -33,8 +34,9 @@ __device__ __forceinline__ float rcp_near(float x, float y) {
 }
 __device__ __forceinline__ float rcp_near(float x) { return rcp_near(x, __builtin_amdgcn_rcpf(x)); }
 
-// a / b with y = rcp_near(b), |a| < 2^60 (a quotient below 2^-100 may be one
-// ulp off, and a zero one positive; sums of pair terms do not show either).
+// a / b with y = rcp_near(b), |a| < 2^60.  A quotient below 2^-100 may be one
+// ulp off: it shows only in a row whose terms are all that small.  A zero one
+// is positive: no sum of terms shows that.
 __device__ __forceinline__ float div_near(float a, float b, float y) {
   const float q = a * y;
   return __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);

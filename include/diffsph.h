@@ -1351,6 +1351,16 @@ int dsph_hash_build_neighbors(const int32_t* offsets, int64_t capacity,
                               const uint8_t* periodicity, int32_t mode,
                               int32_t* out_i, int32_t* out_j, void* stream);
 
+/* The kernels of a uniform support take square roots, reciprocals and
+ * quotients in a short form that equals the IEEE one for operands in range on
+ * this hardware.  Counts (adds to *differ, device int64) the values for which
+ * it does not: op 0 square root and op 1 reciprocal of the floats with bits
+ * first .. first + n - 1 (0 or 2^-96 .. 2^96; 2^-60 .. 2^60), op 2 n drawn
+ * quotients (|a| 2^-40 .. 2^58, b 2^-58 .. 2^58).  No counterpart in the
+ * reference. */
+int dsph_near_check(int32_t op, uint32_t first, int64_t n, uint64_t seed,
+                    int64_t* differ, void* stream);
+
 #ifdef __cplusplus
 }
 #endif
