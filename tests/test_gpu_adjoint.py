@@ -22,12 +22,14 @@ GOLD = os.path.join(os.path.dirname(__file__), "golden", "reference_rollout_grad
 
 def _oprm(cfg):
     return orc.DeltaParams(rho0=cfg.rho0, cs=cfg.cs, delta=cfg.delta, kernel_scale=cfg.kernel_scale,
-                           viscosity=1 if cfg.viscosity == "deltaSPH_viscid" else 0,
-                           visc_coeff=cfg.nu if cfg.viscosity == "deltaSPH_viscid" else cfg.alpha, eps=cfg.eps)
+                           viscosity={"deltaSPH_viscid": 1, "deltaSPH_inviscid": 0, None: -1}[cfg.viscosity],
+                           visc_coeff=cfg.nu if cfg.viscosity == "deltaSPH_viscid" else cfg.alpha, eps=cfg.eps,
+                           kappa=cfg.kappa, pi_switch=cfg.pi_switch, eos=0 if cfg.eos == "isoThermal" else 1,
+                           diffusion=cfg.diffusion)
 
 
-def _check_vjp(ns, what, visc):
-    print(f"case {ns} {what} {visc}", flush=True)
+def _check_vjp(ns, what, visc, **options):
+    print(f"case {ns} {what} {visc} {options}", flush=True)
     rng = np.random.default_rng(11)
     pos, dx = sampling.sample_regular(ns)
     pos = sampling.jitter(pos, dx, 0.3, 11)
@@ -36,7 +38,7 @@ def _check_vjp(ns, what, visc):
     rho = (1.0 + 0.01 * rng.standard_normal(n)).astype(np.float32)
     mass = np.full(n, dx * dx, np.float32)
     h = sampling.volume_to_support(dx * dx, 50.0)
-    cfg = DeltaSPHConfig(support=h, dx=dx, viscosity=visc)
+    cfg = DeltaSPHConfig(support=h, dx=dx, viscosity=visc, **options)
     dev = torch.device("cuda:0")
     T = lambda a: torch.from_numpy(np.ascontiguousarray(a, np.float32)).to(dev)  # noqa: E731
     sv = DeltaSPHSolver(T(pos), T(vel), T(mass), T(rho), cfg)
@@ -78,6 +80,16 @@ def test_rhs_vjp_matches_float64_finite_differences(what, visc):
 @pytest.mark.parametrize("ns", [91, 131, 363])
 def test_rhs_vjp_lanes_match_float64_finite_differences(ns):
     _check_vjp(ns, "all", "deltaSPH_viscid")
+
+
+# the combined pair term's other branches (the bound as above)
+@pytest.mark.parametrize("ns", [32, 131])
+@pytest.mark.parametrize("visc,options", [("deltaSPH_inviscid", {"pi_switch": True}), (None, {}),
+                                          ("deltaSPH_viscid", {"diffusion": False}),
+                                          ("deltaSPH_viscid", {"eos": "Tait"}),
+                                          (None, {"diffusion": False, "eos": "Tait"})])
+def test_rhs_vjp_options_match_float64_finite_differences(ns, visc, options):
+    _check_vjp(ns, "all", visc, **options)
 
 
 def test_rollout_gradient_matches_reference_autograd():

@@ -170,13 +170,15 @@ def _odom(cfg):
     return orc.make_domain(cfg.domain_min, cfg.domain_max, cfg.periodic)
 
 
-@pytest.mark.parametrize("mdbc", ["mDBCDensity", "mDBC_op"])
-def test_rhs_with_walls_matches_oracle_bitexact(mdbc):
-    """Dam break at dx = 1/32 with perturbed velocity and density: mDBC wall
+# 2 res^2 rows: 16, 4 (18432) and 1 (135200) lanes per row
+@pytest.mark.parametrize("mdbc,res", [("mDBCDensity", 32), ("mDBC_op", 32), ("mDBC_op", 96), ("mDBC_op", 260)])
+def test_rhs_with_walls_matches_oracle_bitexact(mdbc, res):
+    """Dam break at dx = 1/res with perturbed velocity and density: mDBC wall
     densities (both variants), normalization, density gradient and every
     right-hand side term with the wall pairs, bit for bit."""
     from dataclasses import replace
-    pos, vel, mass, rho, cfg, walls = _dam(32)
+    print(f"case {mdbc} {res}", flush=True)
+    pos, vel, mass, rho, cfg, walls = _dam(res)
     cfg = replace(cfg, mdbc=mdbc)
     s = DeltaSPHSolver(pos, vel, mass, rho, cfg, walls=walls)
     n = s.n

@@ -243,14 +243,18 @@ def test_record_sweeps_match_separate_arrays():
     assert torch.equal(xp[:, 2], p2) and torch.equal(xp[:, :2], s.grid.sorted_pos)
 
 
-def test_dfsph_compact_index_paths_identical():
+# 363^2 = 131769: without tiles the sweeps read the 16-bit deltas (up to 131072
+# particles they take several lanes per row over the int32 list)
+@pytest.mark.parametrize("nside,steps,kw", [(96, 4, {}), (363, 2, {"tile_cap": 0, "max_iters": 4})])
+def test_dfsph_compact_index_paths_identical(nside, steps, kw):
     """16-bit deltas, the int32 list, the device-side fallback after an
     overflow, the two-pass neighbor list and the one-pass list's fallback
     (then widened) give the same trajectory bit for bit."""
-    d, dt = _setup(96, 4)
-    runs = [_solver(d, dt), _solver(d, dt, compact_index=False), _solver(d, dt, compact_limit=2),
-            _solver(d, dt, neighbor_width=0), _solver(d, dt, neighbor_width=8)]
-    for k in range(4):
+    d, dt = _setup(nside, 4)
+    print(f"case {nside}", flush=True)
+    runs = [_solver(d, dt, **kw), _solver(d, dt, compact_index=False, **kw), _solver(d, dt, compact_limit=2, **kw),
+            _solver(d, dt, neighbor_width=0, **kw), _solver(d, dt, neighbor_width=8, **kw)]
+    for k in range(steps):
         its = [r.step() for r in runs]
         assert len({(st.div_iters, st.den_iters) for st in its}) == 1, k
         assert len({st.num_pairs for st in its}) == 1, k

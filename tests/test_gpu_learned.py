@@ -39,12 +39,16 @@ def test_mlp_forward_matches_oracle(n):
     assert err < 2e-3
 
 
-def test_mlp_gradient_matches_oracle():
+# tiles of 64 samples, 256 workgroups: one sample, a tile and a sample, one turn
+# of some workgroups, a second turn of one (16385), three turns with a ragged
+# last tile; all 16 feature columns in use or the first 8
+@pytest.mark.parametrize("n,features", [(3000, 8), (1, 16), (65, 16), (16385, 16), (40007, 16)])
+def test_mlp_gradient_matches_oracle(n, features):
+    print(f"case {n} {features}", flush=True)
     net = _net(3)
     rng = np.random.default_rng(7)
-    n = 3000
     X = rng.standard_normal((n, 16)).astype(np.float32)
-    X[:, 8:] = 0.0
+    X[:, features:] = 0.0
     T = rng.standard_normal(n).astype(np.float32)
     loss = net.loss_grad(torch.from_numpy(X).cuda(), torch.from_numpy(T).cuda())
     g = net.grad.cpu().numpy().astype(np.float64)
