@@ -309,6 +309,12 @@ __global__ void __launch_bounds__(kBlock) k_vjp_main(PairsDev P, VjpConst K, Vjp
 
 using namespace dsph;
 
+// Lanes per row, where the times cross.  k_vjp_grad / k_vjp_main in us with 16
+// and 4 lanes: 4k rows 9 / 7, 12 / 14; 8.1k 12 / 9, 13 / 15; 12k 13 / 11, 11 / 13;
+// 16k 15 / 13, 11 / 13; 26k 18 / 20, 13 / 17; with 4 and 1: 132k 31 / 51, 36 / 63;
+// 202k 42 / 71, 46 / 85; 262k 53 / 87, 49 / 84; 640k 110 / 203, 101 / 202.
+constexpr int64_t kGrad16 = 1 << 13, kMain16 = 1 << 14, kVjp4 = 7 << 15;
+
 extern "C" size_t dsph_deltasph_vjp_workspace(int64_t n) {
   return ((size_t)n * 4 * sizeof(float) + 255) / 256 * 256 + 256;
 }
@@ -346,9 +352,8 @@ extern "C" int dsph_deltasph_rhs_vjp(const dsph_pairs* pairs, const dsph_deltasp
   K.diffusion = prm->diffusion;
   char* w = static_cast<char*>(ws);
   float4* lsg = reinterpret_cast<float4*>(w);
-  // lanes per row, as the forward passes choose them
-  const int lanes = n <= (1 << 14) ? 16 : (n <= (1 << 17) ? 4 : 1);
-  const int grad_lanes = n <= (1 << 13) ? 16 : (n <= (1 << 17) ? 4 : 1);
+  const int lanes = n <= kMain16 ? 16 : (n <= kVjp4 ? 4 : 1);
+  const int grad_lanes = n <= kGrad16 ? 16 : (n <= kVjp4 ? 4 : 1);
   if (prm->diffusion) {
     auto go = [&](auto kernel) {
       kernel<<<grid_for(n, kBlock / grad_lanes), kBlock, 0, st>>>(P, K, mass, rho, cot_drhodt,

@@ -946,13 +946,14 @@ extern "C" int dsph_volume(int64_t n, const float* mass, const float* rho, float
 // Lanes per row of the *_near kernels.  More lanes shorten a row's chain and
 // fill the chip with fewer rows, but each of them adds all terms, so the
 // fewest that keep ~4 waves on every SIMD win.  Normalization / right-hand
-// side, us, with 16, 4 and 1 lanes: 4k rows 10 / 6.2, 13.7 / 10.6 and 32.6 /
-// 36.9; 16k 16.0 / 9.9, 12.5 / 10.7; 27k 21.2 / 15.6, 15.3 / 13.8; 131k - ,
-// 33 / 38, 41 / 50; 262k - , 48 / 57, 42 / 51 (one thread per row with the
-// IEEE forms and no prefetch of the entries, before: 4k 33 / 39, 131k with
-// walls 48 / 58, 262k 51 / 68, 7.8M 1099 / 1597, now 890 / 1290).
-static int row_lanes(int64_t nq, int64_t up_to_16) { return nq <= up_to_16 ? 16 : (nq <= (1 << 17) ? 4 : 1); }
-constexpr int64_t kNorm16 = 1 << 13, kRhs16 = 1 << 14;
+// side in us with 16 and 4 lanes: 4k rows 8 / 7, 11 / 10; 8.1k 11 / 8, 12 / 10;
+// 12k 13 / 9, 11 / 10; 16k 15 / 10, 11 / 10; 26k 19 / 15, 13 / 12; with 4 and 1:
+// 132k 30 / 35, 33 / 39; 160k 34 / 39, 34 / 40; 202k 41 / 48, 41 / 51; 262k 50 /
+// 59, 44 / 52; 410k 71 / 87, 68 / 83 (one thread per row with the IEEE forms and
+// no prefetch of the entries: 4k 33 / 39, 262k 51 / 68, 7.8M 1099 / 1597, now
+// 890 / 1290).
+constexpr int64_t kNorm16 = 1 << 13, kRhs16 = 1 << 14, kNear4 = 7 << 15;
+static int row_lanes(int64_t nq, int64_t up_to_16) { return nq <= up_to_16 ? 16 : (nq <= kNear4 ? 4 : 1); }
 
 template <class DF>
 static int launch_normalization(const PairsDev& P, const BoundaryDev& B, const DF& dom, const float* mass,

@@ -1246,10 +1246,9 @@ __global__ void __launch_bounds__(kBlock* kSweepBLanes) k_dfsph_sweep_b_lanes(Pa
   }
 }
 
-// Rows up to which the lanes forms are the faster ones.  A + B in us, lanes
-// against tiles: 2.3k rows 4.8 + 11.0 / 16.4 + 16.5, 8.1k 5.9 + 11.4 / 16.4 +
-// 16.7, 33k 8.8 + 11.2 / 16.4 + 16.7, 131k 15.2 + 15.8 / 20.6 + 21.1; A with
-// 16 lanes against 4: 16k 7.6 / 7.4, 33k 12.0 / 8.8.
+// Rows up to which the lanes forms are the faster ones (near_math.h has A's
+// figures).  B in us, 4 lanes against tiles: 2.3k rows 11.0 / 16.5, 33k 11.2 /
+// 16.7, 132k 19.8 / 21.5, 160k 20.6 / 22.3, 202k 25.7 / 23.6, 262k 26.4 / 24.5.
 constexpr int kSweepA16 = kLanes16Rows, kSweepLanes = kLanes4Rows;
 
 // Sweep launches: lanes per row for few rows, else over neighbor tiles when

@@ -170,8 +170,13 @@ __device__ __forceinline__ void sum_row(const int32_t* __restrict__ nbr, const R
   }
 }
 
-// Lanes per row of the DFSPH passes: few rows are a matter of latency (their
-// figures stand at the passes), from 131k rows on the tiled forms fill the chip.
-constexpr int kLanes16Rows = 1 << 13, kLanes4Rows = 1 << 17;
+// Lanes per row of the DFSPH passes (16, 4, else tiles): few rows are a matter
+// of latency, many fill the chip by themselves, and the lines lie where the
+// times cross.  Density / prepare / source / sweep A in us: 8.1k rows with 16
+// lanes 8 / 9 / 5 / 6, with 4 12 / 13 / 7 / 8; 12k 7 / 11 / 6 / 7 and 9 / 13 / 7 /
+// 7; 16k 7 / 13 / 7 / 8 and 9 / 13 / 7 / 7; 160k with 4 lanes 22 / 41 / 20 / 19,
+// tiles 27 / 46 / 23 / 22; 202k 25 / 51 / 23 / 22 and 29 / 51 / 24 / 23; 262k 28 /
+// 61 / 27 / 26 and 28 / 53 / 25 / 24.
+constexpr int kLanes16Rows = 3 << 12, kLanes4Rows = 3 << 16;
 
 }  // namespace dsph

@@ -75,9 +75,9 @@ def test_rhs_vjp_matches_float64_finite_differences(what, visc):
     _check_vjp(32, what, visc)
 
 
-# the passes' 16, 4 and 1 lanes per row change at 8192, 16384 and 131072 rows
+# the passes' 16, 4 and 1 lanes per row change at 8192, 16384 and 229376 rows
 # (the bound of the small case: float32 sums, measured 3e-6)
-@pytest.mark.parametrize("ns", [91, 131, 363])
+@pytest.mark.parametrize("ns", [91, 131, 363, 481])
 def test_rhs_vjp_lanes_match_float64_finite_differences(ns):
     _check_vjp(ns, "all", "deltaSPH_viscid")
 

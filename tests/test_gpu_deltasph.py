@@ -170,8 +170,8 @@ def _odom(cfg):
     return orc.make_domain(cfg.domain_min, cfg.domain_max, cfg.periodic)
 
 
-# 2 res^2 rows: 16, 4 (18432) and 1 (135200) lanes per row
-@pytest.mark.parametrize("mdbc,res", [("mDBCDensity", 32), ("mDBC_op", 32), ("mDBC_op", 96), ("mDBC_op", 260)])
+# 2 res^2 rows: 16, 4 (18432) and 1 (233928) lanes per row
+@pytest.mark.parametrize("mdbc,res", [("mDBCDensity", 32), ("mDBC_op", 32), ("mDBC_op", 96), ("mDBC_op", 342)])
 def test_rhs_with_walls_matches_oracle_bitexact(mdbc, res):
     """Dam break at dx = 1/res with perturbed velocity and density: mDBC wall
     densities (both variants), normalization, density gradient and every
@@ -326,7 +326,7 @@ def test_mdbc_op_ghost_counts_match_oracle_bitexact(ghosts):
 
 
 # rows of 16, 4 and 1 lanes, with a last workgroup that is not full
-@pytest.mark.parametrize("nside", [33, 91, 131, 363])
+@pytest.mark.parametrize("nside", [33, 91, 131, 363, 481])
 @pytest.mark.parametrize("state", ["plain", "switch", "odd", "rest"])
 def test_near_kernels_equal_general_kernels(nside, state):
     """The uniform-support kernels give the bits of the general ones (reached

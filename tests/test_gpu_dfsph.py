@@ -63,8 +63,8 @@ def test_dfsph_steps_match_oracle(orc, nside, seed, steps):
         assert abs(stats.den_error - info["err_den"]) <= 1e-6 * max(1e-12, abs(info["err_den"])) + 1e-9
 
 
-# 16 lanes per row, 4 lanes (from 8193 rows), and the tiled passes (from 131073)
-@pytest.mark.parametrize("nside", [33, 91, 131, 363])
+# 16 lanes per row, 4 lanes (from 12289 rows), and the tiled passes (from 196609)
+@pytest.mark.parametrize("nside", [33, 91, 131, 363, 444])
 def test_dfsph_lane_passes_equal_oracle_bits(orc, nside):
     d, dt = _setup(nside, 5, 0.4)
     print(f"case nside={nside}", flush=True)
@@ -243,9 +243,9 @@ def test_record_sweeps_match_separate_arrays():
     assert torch.equal(xp[:, 2], p2) and torch.equal(xp[:, :2], s.grid.sorted_pos)
 
 
-# 363^2 = 131769: without tiles the sweeps read the 16-bit deltas (up to 131072
+# 444^2 = 197136: without tiles the sweeps read the 16-bit deltas (up to 196608
 # particles they take several lanes per row over the int32 list)
-@pytest.mark.parametrize("nside,steps,kw", [(96, 4, {}), (363, 2, {"tile_cap": 0, "max_iters": 4})])
+@pytest.mark.parametrize("nside,steps,kw", [(96, 4, {}), (444, 2, {"tile_cap": 0, "max_iters": 4})])
 def test_dfsph_compact_index_paths_identical(nside, steps, kw):
     """16-bit deltas, the int32 list, the device-side fallback after an
     overflow, the two-pass neighbor list and the one-pass list's fallback

@@ -90,11 +90,11 @@ def test_tile_runs_and_slots(nside, seed):
 
 
 # cap 0: the median neighbor count of the first step's workgroups, so that
-# some workgroups use their tile and the others gather.  Up to 131072 particles
+# some workgroups use their tile and the others gather.  Up to 196608 particles
 # the passes of a step take several lanes per row with and without tiles; from
-# 363^2 = 131769 on they read the tiles: all fit, some, none.
+# there on (444^2 = 197136) they read the tiles: all fit, some, none.
 @pytest.mark.parametrize("nside,seed,cap", [(96, 1, 2048), (272, 2, 1024), (272, 2, 0), (96, 1, 64),
-                                            (363, 3, 4096), (363, 3, 0), (363, 3, 64)])
+                                            (444, 3, 4096), (444, 3, 0), (444, 3, 64)])
 def test_tiled_steps_bit_identical(nside, seed, cap):
     d, dt = _setup(nside, seed)
     if cap == 0:
