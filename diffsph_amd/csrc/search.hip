@@ -208,7 +208,7 @@ __device__ __forceinline__ void load_queries(const SearchArgs& a, int i0, Querie
 // min-image is evaluated only for cell rows at a periodic seam (elsewhere the
 // plain difference is the offset).  kH: supports per particle (else the
 // uniform a.h0).
-template <int kRows, bool kH, bool kDirect, class Value, class Put, class Spill, class Done>
+template <int kRows, bool kH, bool kDirect, bool kMaySparse, class Value, class Put, class Spill, class Done>
 __device__ __forceinline__ void scan_queries(const SearchArgs& a, const Queries<kRows>& Q, int depth,
                                              const Value& value, const Put& put, const Spill& spill,
                                              const Done& done) {
@@ -229,7 +229,7 @@ __device__ __forceinline__ void scan_queries(const SearchArgs& a, const Queries<
       const float2 qi = make_float2(q.x(), q.y());
       return seam ? keep_pair(qi, q.h(), c.x, c.h, a) : keep_pair_near(qi, q.h(), c.x, c.h, a);
     };
-    n = scan_rows<kMine, kDirect, true>(
+    n = scan_rows<kMine, kDirect, kMaySparse>(
         cell, depth, rows, mine, [&](int j) { return Cand{a.rpos[j], h_of(a.rh, j, a.h0)}; }, val,
         [&](const Cand& c, const auto& q, bool seam) {
           return LaneTest{__builtin_amdgcn_ballot_w64(keep(c, q, seam)), 0};
@@ -245,7 +245,7 @@ __device__ __forceinline__ void scan_queries(const SearchArgs& a, const Queries<
       }
       return dist2_exact(dx, dy);
     };
-    n = scan_rows<kMine, kDirect, true>(
+    n = scan_rows<kMine, kDirect, kMaySparse>(
         cell, depth, rows, mine, [&](int j) { return a.rpos[j]; }, val,
         [&](const float2& x, const auto& q, bool seam) { return within(d2(x, q, seam)); },
         [&](const float2& x, const auto& q, bool seam) { return within.exact(d2(x, q, seam)); }, in, out);
@@ -264,14 +264,20 @@ static bool small_query_set(const SearchArgs& a) {
   return a.nq < (varied_support(a) ? (1 << 18) : kRowSmall);
 }
 
-template <int kRows, bool kH>
+// Whether most cells may be sparse enough for scan_rows_sparse: only then do
+// the kernels look for waves that are (0.25 us of a 10 us fill of a 64^2 box).
+static bool may_be_sparse(const SearchArgs& a) {
+  return (int64_t)a.nref * 9 < (int64_t)a.g.nc[0] * a.g.nc[1] * kSparse;
+}
+
+template <int kRows, bool kH, bool kMaySparse>
 __global__ void __launch_bounds__(kBlock) k_neighbor_count(SearchArgs a, int32_t* __restrict__ counts) {
   __shared__ Queries<kRows> Q;
   const int i0 = blockIdx.x * kRows;
   bool over = false;  // counted without the skipped ranges; the host checks the cells
   load_queries<kRows>(a, i0, Q, over, [](int, int, const CellRow&) {});
   __syncthreads();
-  scan_queries<kRows, kH, false>(
+  scan_queries<kRows, kH, false, kMaySparse>(
       a, Q, INT32_MAX, [](int, int, bool, int) { return 0; }, [](int, int, int) {}, [](int, int, int) {},
       [&](int r, int n) { counts[i0 + r] = n; });
 }
@@ -345,7 +351,7 @@ struct FillOut {
 // the run of the candidate range, as ~j for a range outside the tile's runs
 // (tile_n = -1 then); a tile that does not fit T.cap (or kFillTileMax) is
 // filled without slots.
-template <int kRows, bool kTiles, bool kH, bool kCsr>
+template <int kRows, bool kTiles, bool kH, bool kCsr, bool kMaySparse>
 __global__ void __launch_bounds__(kBlock) k_neighbor_fill(SearchArgs a, FillOut F, FillTiles T) {
   extern __shared__ int32_t stage[];
   __shared__ Queries<kRows> Q;
@@ -400,7 +406,7 @@ __global__ void __launch_bounds__(kBlock) k_neighbor_fill(SearchArgs a, FillOut 
   };
   // slot of the reference particle a staged value stands for
   auto ref_of = [&](int v) { return !slots ? v : (v >= 0 ? (v & 0xfff) - rt_d[v >> 12] : ~v); };
-  scan_queries<kRows, kH, kCsr>(
+  scan_queries<kRows, kH, kCsr, kMaySparse>(
       a, Q, kCsr ? 0 : F.depth,
       [&](int p, int r, bool first, int j) {
         if (!slots) return j;
@@ -500,7 +506,7 @@ static FillTiles tiles_from(FillTiles T, int row0, int width) {
   return T;
 }
 
-template <int kRows, bool kH>
+template <int kRows, bool kH, bool kMaySparse>
 static void launch_fill_rows(const SearchArgs& a, const FillOut& F, const FillTiles* tiles, hipStream_t st) {
   const size_t lds = (size_t)F.depth * (kRows + 1) * sizeof(int32_t);
   auto go = [&](auto kernel) {
@@ -510,11 +516,11 @@ static void launch_fill_rows(const SearchArgs& a, const FillOut& F, const FillTi
     });
   };
   if (tiles)
-    go(k_neighbor_fill<kRows, true, kH, false>);
+    go(k_neighbor_fill<kRows, true, kH, false, kMaySparse>);
   else if (F.depth > 0)
-    go(k_neighbor_fill<kRows, false, kH, false>);
+    go(k_neighbor_fill<kRows, false, kH, false, kMaySparse>);
   else
-    go(k_neighbor_fill<kRows, false, kH, true>);
+    go(k_neighbor_fill<kRows, false, kH, true, kMaySparse>);
 }
 
 __global__ void __launch_bounds__(kBlock) k_fixed_slices(int nslices, int width, int32_t* __restrict__ slice_off,
@@ -543,10 +549,14 @@ static int launch_fill(const SearchArgs& a, FillOut F, const FillTiles* tiles, h
     k_set_flag<<<1, 64, 0, st>>>(F.ovf, 1);
     F.d16 = nullptr;
   }
-  if (small_query_set(a))
-    vary ? launch_fill_rows<16, true>(a, F, tiles, st) : launch_fill_rows<16, false>(a, F, tiles, st);
-  else
-    vary ? launch_fill_rows<64, true>(a, F, tiles, st) : launch_fill_rows<64, false>(a, F, tiles, st);
+  auto go = [&](auto sparse) {
+    constexpr bool S = decltype(sparse)::value;
+    if (small_query_set(a))
+      vary ? launch_fill_rows<16, true, S>(a, F, tiles, st) : launch_fill_rows<16, false, S>(a, F, tiles, st);
+    else
+      vary ? launch_fill_rows<64, true, S>(a, F, tiles, st) : launch_fill_rows<64, false, S>(a, F, tiles, st);
+  };
+  may_be_sparse(a) ? go(std::true_type{}) : go(std::false_type{});
   if (several && F.slices_out) {
     const int nslices = (int)(((int64_t)a.nq + 63) / 64);
     k_fixed_slices<<<grid_for(nslices + 1), kBlock, 0, st>>>(nslices, F.width, F.slices_out, nullptr, nullptr);
@@ -745,10 +755,14 @@ extern "C" int dsph_neighbor_count(const dsph_domain* domain, const dsph_grid* g
       kernel<<<grid_for(rows, per_block), kBlock, 0, st>>>(queries_from(a, row0, rows), counts + row0);
     });
   };
-  if (small_query_set(a))
-    vary ? launch(k_neighbor_count<16, true>, 16) : launch(k_neighbor_count<16, false>, 16);
-  else
-    vary ? launch(k_neighbor_count<64, true>, 64) : launch(k_neighbor_count<64, false>, 64);
+  auto go = [&](auto sparse) {
+    constexpr bool S = decltype(sparse)::value;
+    if (small_query_set(a))
+      vary ? launch(k_neighbor_count<16, true, S>, 16) : launch(k_neighbor_count<16, false, S>, 16);
+    else
+      vary ? launch(k_neighbor_count<64, true, S>, 64) : launch(k_neighbor_count<64, false, S>, 64);
+  };
+  may_be_sparse(a) ? go(std::true_type{}) : go(std::false_type{});
   return launch_status();
 }
 
