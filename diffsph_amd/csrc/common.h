@@ -378,23 +378,6 @@ __device__ __forceinline__ int wave_slot(int32_t* __restrict__ count, int key, b
   return __shfl(base, first, 64) + before;
 }
 
-// body(j, load(j)) for j = b .. e-1 in order; the loads of U consecutive j
-// are issued before the first body of the group, so U gathers are in
-// flight at once.  The order of the bodies (and of any sums they form) is
-// that of the plain loop.
-template <int U, class Load, class Body>
-__device__ __forceinline__ void scan_range(int b, int e, Load&& load, Body&& body) {
-  int j = b;
-  for (; j + U <= e; j += U) {
-    decltype(load(j)) d[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) d[u] = load(j + u);
-#pragma unroll
-    for (int u = 0; u < U; ++u) body(j + u, d[u]);
-  }
-  for (; j < e; ++j) body(j, load(j));
-}
-
 // body(j, load(j)) over the entries j of a neighbor row, in row order, with
 // U entries and their gathers in flight (Stream: the entries are read with
 // non-temporal loads, for lists read once).

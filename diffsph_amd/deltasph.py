@@ -292,8 +292,10 @@ class DeltaSPHSolver:
         n = self.n
         self._grad = torch.empty(n, 2, **f)
         self._vol = torch.empty(n, **f)
-        self._k = [(torch.empty(n, 2, **f), torch.empty(n, 2, **f), torch.empty(n, **f)) for _ in range(4)]
-        self._stage = (torch.empty(n, 2, **f), torch.empty(n, 2, **f), torch.empty(n, **f))
+        # per stage: its velocity (the first stage's is the state's), dudt, drhodt
+        self._k = [(torch.empty(n, 2, **f) if k else None, torch.empty(n, 2, **f), torch.empty(n, **f))
+                   for k in range(4)]
+        self._stage = (torch.empty(n, 2, **f), torch.empty(n, **f))  # positions, densities
         self._widths = {}           # list kind -> row width of the one-pass list
         self._deferred = None       # int32 [1] device flag: searches check overflow later (captured steps)
 
@@ -413,7 +415,7 @@ class DeltaSPHSolver:
         dt = float(np.float32(self.dt))
         half = float(np.float32(dt) * np.float32(0.5))
         x0, u0, r0 = self.pos, self.vel, self.rho
-        xs, _, rs = self._stage
+        xs, rs = self._stage
         x, u, r = x0, u0, r0
         dxdt = [None] * 4
         for s, c in enumerate([half, half, dt, None]):
@@ -465,7 +467,7 @@ class DeltaSPHSolver:
         dt_dev, time_dev = self._device_clock()
         self._sort()
         x0, u0, r0 = self.pos, self.vel, self.rho
-        xs, _, rs = self._stage
+        xs, rs = self._stage
         x, u, r = x0, u0, r0
         dxdt = [None] * 4
         for k, half in enumerate((1, 1, 0, None)):
