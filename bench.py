@@ -520,8 +520,10 @@ def _solver_roofline(s, reps, vjp=False):
       k_dsph_rhs:           pos 8 + vel 8 + rho 4 + mass 4 + grad 8 + offset 4 + dudt 8 + drho/dt 4
                             = 48 B/particle + 4 B/entry
       with walls, each pass + 4 B/particle (wall-list offset) + 4 B per wall entry;
-      adjoint (dsph_deltasph_rhs_vjp: k_vjp_lg 32, k_vjp_lsm 52, k_vjp_main 108 B/particle, 4 B/entry each)
-                            = 192 B/particle + 12 B/entry."""
+      adjoint (dsph_deltasph_rhs_vjp, 4 B/entry each pass):
+      k_vjp_grad: pos 8 + mass 4 + rho 4 + cotangent 4 + grad 8 + offset 4 + write 16 = 48 B/particle
+      k_vjp_main: pos 8 + vel 8 + grad 8 + rho 4 + mass 4 + cotangents 8 + 4 + 8 + (lambda_s, g) 16 + offset 4
+                  + writes 8 + 8 + 4 = 92 B/particle; together 140 B/particle + 8 B/entry."""
     import torch
     from diffsph_amd import _lib
     from diffsph_amd.neighborhood import WORKSPACE
@@ -553,10 +555,10 @@ def _solver_roofline(s, reps, vjp=False):
                torch.randn(n, generator=g).to(s.pos.device)]
         ws = WORKSPACE.get(L.dsph_deltasph_vjp_workspace(n), s.pos.device)
         gx, gu, gr = torch.empty_like(s.pos), torch.empty_like(s.vel), torch.empty_like(s.rho)
-        passes["k_vjp_lg+k_vjp_lsm+k_vjp_main"] = (lambda: _lib.check(L.dsph_deltasph_rhs_vjp(
+        passes["k_vjp_grad+k_vjp_main"] = (lambda: _lib.check(L.dsph_deltasph_rhs_vjp(
             C.byref(pr), C.byref(s.prm), _lib.ptr(s.vel), _lib.ptr(s.mass), _lib.ptr(s.rho), _lib.ptr(s._grad),
             _lib.ptr(cot[0]), _lib.ptr(cot[1]), _lib.ptr(cot[2]), _lib.ptr(gx), _lib.ptr(gu), _lib.ptr(gr),
-            _lib.ptr(ws), ws.numel(), sh)), 192 * n + 12 * P)
+            _lib.ptr(ws), ws.numel(), sh)), 140 * n + 8 * P)
     out = {}
     for name, (fn, byt) in passes.items():
         t = _time_pass(fn, reps, stream)
@@ -567,8 +569,7 @@ def _solver_roofline(s, reps, vjp=False):
     return {"bound": "hbm", "achieved": r["gbs"], "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": round(r["gbs"] / HBM_PEAK_GBS, 4), "traffic": None, "kernel": dom, "kernel_us": r["us"],
             "algorithmic_bytes": r["bytes"], "entries": P, "wall_entries": wall_entries, "passes": out,
-            "limiter": "VALU-heavy pair kernels with two waves per SIMD at this size: gather latency "
-                       "(profiles/dambreak_131k_kernels.md)"}
+            "limiter": "VALU issue of the pair kernels (profiles/perf_cases_kernels.md)"}
 
 
 def _oracle_deltasph_rate(states, cfg, steps):

@@ -6,8 +6,8 @@
 // Inputs are the arrays of a reference neighborDict: row-sorted pair list
 // (CSR offsets over the rows, int64 j), precomputed kernel values W_ij,
 // gradients gradW_ij [P,2], normalised distances r_ij/h_ij, unit vectors
-// x_ij [P,2] and supports h_ij.  One thread per row sums its segment in
-// list order.  A quantity is either per particle (the reference's (q_i, q_j)
+// x_ij [P,2] and supports h_ij.  1 to 16 threads sum a row's segment in list
+// order.  A quantity is either per particle (the reference's (q_i, q_j)
 // tuple: qa indexed by i, qb by j) or per pair (a single tensor).
 #include "common.h"
 #include "near_math.h"

@@ -1,6 +1,7 @@
 // SPH pair operators as gather kernels over a CSR neighbor list; kernel
 // values are evaluated on the fly from positions (no per-pair arrays).
-// One thread per query particle, neighbors in CSR order, no atomics.
+// One thread per query particle unless said otherwise, neighbors in list order,
+// no atomics.
 #include "common.h"
 #include "near_math.h"
 
