@@ -166,9 +166,13 @@ __global__ void __launch_bounds__(kBlock) k_bscatter(int n, const int32_t* __res
   order[cell_start[keys[i]] + slot[i]] = i;
 }
 
-// The final order, by particle index within each cell (cell_rank, cells of any
-// size: a batch has no report of an overfull one); with `dst`, dst[slot] =
-// src[particle] in the same pass.
+// Largest cell ranked by index: the work of a diverged batch (NaN positions all
+// fall into one cell) stays bounded.  A larger cell always has rows beyond any
+// list width, which the batch's status reports.
+constexpr int kBatchCellMax = 1 << 16;
+
+// The final order, by particle index within each cell (cell_rank); with `dst`,
+// dst[slot] = src[particle] in the same pass.
 __global__ void __launch_bounds__(kBlock) k_bcellrank(int n, const int32_t* __restrict__ keys,
                                                       const int32_t* __restrict__ slot,
                                                       const int32_t* __restrict__ cell_start,
@@ -176,7 +180,7 @@ __global__ void __launch_bounds__(kBlock) k_bcellrank(int n, const int32_t* __re
                                                       const float2* __restrict__ src, float2* __restrict__ dst) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  const int p = cell_rank(i, keys[i], slot, cell_start, order, INT32_MAX);
+  const int p = cell_rank(i, keys[i], slot, cell_start, order, kBatchCellMax);
   si[p] = i;
   if (dst) dst[p] = src[i];
 }
