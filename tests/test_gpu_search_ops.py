@@ -436,7 +436,10 @@ def test_search_rows_by_cell_match_oracle(orc, nside, hscale, per, vary):
     (1000, 0.4, (True, True), False, False), (1001, 3.0, (False, True), True, False),
     (40001, 0.5, (True, True), False, False), (40001, 3.0, (True, False), False, True),
     (40001, 8.0, (True, True), False, False), (30001, 8.0, (False, False), True, True),
-    (300001, 3.0, (True, True), True, True)])
+    (300001, 3.0, (True, True), True, True),
+    # three cells a periodic axis: every cell row wraps
+    (1, 0.09, (True, True), False, False), (20, 1.8, (True, True), False, False),
+    (57, 5.13, (True, False), True, False), (60, 5.4, (True, True), True, False)])
 def test_search_of_sparse_cells_matches_oracle(orc, n, per_cell, per, vary, corner):
     print(f"case {n} {per_cell} {per} {vary} {corner}", flush=True)
     rng = np.random.default_rng(n)
